@@ -1,0 +1,440 @@
+// gemv_any.hip -- the Q4_K, Q6_K and Q8_0 GEMV y = W x for any K (the shapes
+// that have no kernel of their own in q4k_kernels.hip and kquant.hip).
+//
+// Work split ("column resident", as in q4k_gemv.hpp, with the row length a
+// run-time value): a row has S slots (Q4_K / Q6_K: four per super-block,
+// Q8_0: one per 32-element block).  Thread t of a workgroup owns slot t % S of
+// rows t / S + it * rpi (it < ITERS, rpi = T / S): consecutive threads read
+// consecutive pieces of a row, all ITERS rows' weights are in flight before
+// any arithmetic, and the activations are staged once per workgroup.
+//
+// Arithmetic: each 64-element activation chunk is scaled to integers
+// X = rint(x * s), s = top / 2^e with the chunk's max |x| < 2^e, written as
+// three balanced bytes X = 65536*x2 + 256*x1 + x0; Q6_K and Q8_0 keep
+// x3 = rint(254 (x*s - X)) as a fourth.  The weight codes multiply the digits
+// in exact integer dot products (v_dot4_i32_i8), so the roundings are the
+// last digit and the f32 combine per slot.  Against float64 on N(0,1) rows:
+// Q4_K 2.9e-7 to 3.2e-7 rel-L2, where f32 products and sums give 5.4e-7 to
+// 8.4e-7 (the codes' and the min's parts cancel); Q6_K 0.9e-7 to 1.1e-7
+// (f32 1.4e-7 to 2.8e-7), Q8_0 0.7e-7 to 1.0e-7 (f32 1.0e-7 to 2.3e-7; three
+// digits, 1.9e-7, would not do).  3 or 4 dot operations per 4 weights, where
+// f32 takes 4 conversions and 4 FMAs.
+// A chunk that holds an infinity or a NaN has no such digits: its delta is
+// NaN, which makes a Q4_K slot NaN as its f32 form is (scale*inf - min*inf),
+// and sends a Q6_K or Q8_0 slot through f32 products, element by element.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "../../include/rt_hip.h"
+#include "kquant_layout.hpp"
+#include "q4k_gemv.hpp"
+#include "rt_device.hpp"
+#include "rt_kernels.hpp"
+
+namespace rt {
+namespace {
+
+// Stage of one chunk, in dwords: the digit planes of 16 (dword i = elements
+// 4i .. 4i+3), then delta, for Q4_K the sums of X over the chunk's two halves
+// (the min term), padding, and for Q6_K per 16-element sub-block the integer sums of
+// x0 + 256*x1 and, packed in one dword, of x2 (low half) and x3.  The pitches
+// put the 16 lanes that a 16-byte LDS read serves together on distinct banks.
+template <int FMT>
+constexpr int kAnyDigits = FMT == RT_LINEAR_Q4K ? 3 : 4;
+template <int FMT>
+constexpr int kAnyPitch = 16 * kAnyDigits<FMT> + (FMT == RT_LINEAR_Q6K ? 12 : 4);
+constexpr float kAnyTop3 = 8355711.0f;  // 127 * (65536 + 256 + 1)
+constexpr float kAnyTop4 = 4194304.0f;  // 2^22: the scaling is exact
+constexpr float kAnyUnit3 = 1.0f / 8388608.0f, kAnyUnit4 = 1.0f / 4194304.0f;
+
+// Elements 4f .. 4f+3 of the vector (zeros past K); the 16 lanes of a chunk
+// are consecutive lanes of a wave and all call this; `store` masks the lanes
+// past the last chunk.
+template <int FMT>
+RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
+  uint32_t mb = max(max(f32_bits(v.x) & 0x7FFFFFFFu, f32_bits(v.y) & 0x7FFFFFFFu),
+                    max(f32_bits(v.z) & 0x7FFFFFFFu, f32_bits(v.w) & 0x7FFFFFFFu));
+  mb = max(mb, dpp_u32<0xB1>(mb));
+  mb = max(mb, dpp_u32<0x4E>(mb));
+  mb = max(mb, dpp_u32<0x141>(mb));
+  mb = max(mb, dpp_u32<0x140>(mb));
+  constexpr int ND = kAnyDigits<FMT>;
+  constexpr float kTop = ND == 3 ? kAnyTop3 : kAnyTop4;
+  // max < 2^e; below 2^-103 the scale stays at the largest normal one
+  const int e = max((int)(mb >> 23) - 126, -103);
+  const float s = bits_f32(f32_bits(kTop) - ((uint32_t)e << 23));
+  float delta = bits_f32(f32_bits(1.0f / (kTop * (ND == 3 ? kAnyUnit3 : kAnyUnit4))) + ((uint32_t)e << 23));
+  if (mb >= 0x7F800000u) delta = bits_f32(0x7FC00000u);
+  const float xs[4] = {v.x, v.y, v.z, v.w};
+  uint32_t b[4], r[4];  // bytes 0..2: X + 0x808080; the fourth digit + 128
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float t = __builtin_amdgcn_fmed3f(xs[i] * s, -kTop, kTop), X = __builtin_rintf(t);
+    b[i] = (uint32_t)(int)X + 0x808080u;
+    if constexpr (ND == 4) r[i] = (uint32_t)((int)__builtin_rintf((t - X) * 254.0f) + 128);
+  }
+  const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);  // b0.0 b1.0 b0.1 b1.1
+  const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
+  const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0602u);  // b0.2 b1.2 0 0
+  const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0602u);
+  uint32_t d[4];
+  d[0] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
+  d[1] = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
+  d[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u;
+  if constexpr (ND == 4) {
+    const uint32_t r01 = __builtin_amdgcn_perm(r[1], r[0], 0x0C0C0400u), r23 = __builtin_amdgcn_perm(r[3], r[2], 0x0C0C0400u);
+    d[3] = __builtin_amdgcn_perm(r23, r01, 0x05040100u) ^ 0x80808080u;
+  }
+  // Q4_K: sum of X over the 8 lanes of a half, exact (so the codes' and the
+  // min's parts see the same rounded activations)
+  int half = 0;
+  if constexpr (FMT == RT_LINEAR_Q4K) {
+    half = (int)(b[0] + b[1] + b[2] + b[3]) - 4 * 0x808080;
+    half += (int)dpp_u32<0xB1>((uint32_t)half);
+    half += (int)dpp_u32<0x4E>((uint32_t)half);
+    half += (int)dpp_u32<0x141>((uint32_t)half);
+  }
+  int s01 = 0, s23 = 0;
+  if constexpr (FMT == RT_LINEAR_Q6K) {
+    auto sum4 = [](uint32_t q) { return __builtin_amdgcn_sdot4((int)q, 0x01010101, 0, false); };
+    s01 = sum4(d[0]) + 256 * sum4(d[1]);
+    s23 = sum4(d[2]) + 65536 * sum4(d[3]);
+    s01 += (int)dpp_u32<0xB1>((uint32_t)s01);
+    s23 += (int)dpp_u32<0xB1>((uint32_t)s23);
+    s01 += (int)dpp_u32<0x4E>((uint32_t)s01);  // 4 lanes = 16 elements
+    s23 += (int)dpp_u32<0x4E>((uint32_t)s23);
+  }
+  if (!store) return;
+  const int sub = f & 15;
+  uint32_t *base = dl + (f >> 4) * kAnyPitch<FMT>, *st = base + 16 * ND;
+#pragma unroll
+  for (int i = 0; i < ND; ++i) base[16 * i + sub] = d[i];
+  if (sub == 0) st[0] = f32_bits(delta);
+  if constexpr (FMT == RT_LINEAR_Q4K) {
+    if ((sub & 7) == 0) st[1 + (sub >> 3)] = f32_bits((float)half * kAnyUnit3);
+  }
+  if constexpr (FMT == RT_LINEAR_Q6K) {
+    if ((sub & 3) == 0) st[4 + 2 * (sub >> 2)] = (uint32_t)s01, st[5 + 2 * (sub >> 2)] = (uint32_t)s23;
+  }
+}
+
+// sum_k c_k x_k / delta from a group's digit sums: the middle digits combine
+// exactly (|s0 + 256 s1| < 2^28), then one rounding per step.  The power of
+// two of `top` is taken out here, so delta (about 2^e) neither underflows
+// for small activations nor makes a product overflow before the last one.
+RT_DEV float any_dot(const int (&s)[3]) {
+  return fmaf((float)s[2], 65536.0f * kAnyUnit3, (float)(s[0] + 256 * s[1]) * kAnyUnit3);
+}
+RT_DEV float any_dot(const int (&s)[4]) {
+  return fmaf((float)s[2], 65536.0f * kAnyUnit4, fmaf((float)s[3], 1.0f / 254.0f, (float)(s[0] + 256 * s[1])) * kAnyUnit4);
+}
+
+// Weights of a thread's slot in ITERS rows, and their dot products with the
+// staged chunk(s): p[it] is the slot's part of row it.
+template <int FMT, int ITERS>
+struct AnyTile;
+
+template <int ITERS>
+struct AnyTile<RT_LINEAR_Q4K, ITERS> {
+  uint4 hd[ITERS], qa[ITERS], qb[ITERS];
+  RT_DEV void load(int it, const uint8_t *W, int, int K, int row, int slot) {
+    const uint8_t *bp = W + ((size_t)row * (K / 256) + (slot >> 2)) * kQ4KBlockBytes;
+    const int c = slot & 3;
+    hd[it] = *reinterpret_cast<const uint4 *>(bp);
+    qa[it] = *reinterpret_cast<const uint4 *>(bp + 16 + 32 * c);
+    qb[it] = *reinterpret_cast<const uint4 *>(bp + 32 + 32 * c);
+  }
+  RT_DEV void compute(const uint32_t *dl, int slot, float (&p)[ITERS]) const {
+    const uint32_t m4 = opaque_u32(0x0F0F0F0Fu);
+    const uint32_t *base = dl + slot * kAnyPitch<RT_LINEAR_Q4K>;
+    int l[ITERS][3], h[ITERS][3];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) l[it][d] = h[it][d] = 0;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      uint4 a[3], b[3];  // digits of low-half words 4g .. 4g+3 and of the high half's
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        a[d] = *reinterpret_cast<const uint4 *>(base + 16 * d + 4 * g);
+        b[d] = *reinterpret_cast<const uint4 *>(base + 16 * d + 8 + 4 * g);
+      }
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const uint4 q = g ? qb[it] : qa[it];
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int lo = (int)(w[j] & m4), hi = (int)((w[j] >> 4) & m4);
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            const uint32_t A[4] = {a[d].x, a[d].y, a[d].z, a[d].w}, B[4] = {b[d].x, b[d].y, b[d].z, b[d].w};
+            l[it][d] = __builtin_amdgcn_sdot4(lo, (int)A[j], l[it][d], false);
+            h[it][d] = __builtin_amdgcn_sdot4(hi, (int)B[j], h[it][d], false);
+          }
+        }
+      }
+    }
+    const float4 st = *reinterpret_cast<const float4 *>(base + 48);  // delta, sum_lo, sum_hi
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+      const float d = half_bits_to_f32(hd[it].x & 0xFFFFu), dm = half_bits_to_f32(hd[it].x >> 16);
+      uint32_t svp, mvp;
+      q4k_scale_min_pair(hd[it].y, hd[it].z, hd[it].w, slot & 3, svp, mvp);
+      const float qsum = fmaf((float)(svp >> 8), any_dot(h[it]),
+                              (float)(svp & 0xFFu) * any_dot(l[it]));
+      const float msum = fmaf((float)(mvp >> 8), st.z, (float)(mvp & 0xFFu) * st.y);
+      p[it] = fmaf(d * st.x, qsum, -(dm * st.x * msum));
+    }
+  }
+};
+
+template <int ITERS>
+struct AnyTile<RT_LINEAR_Q6K, ITERS> {  // slot: see Q6KTile (kquant_tile.hpp)
+  uint4 qa[ITERS], qb[ITERS], qh[ITERS];
+  uint2 sc[ITERS];
+  uint32_t dd[ITERS];
+  RT_DEV void load(int it, const uint8_t *W, int N, int K, int row, int slot) {
+    const Q6KPlanes P = q6k_planes(W, (size_t)N * (K / 256));
+    const size_t blk = (size_t)row * (K / 256) + (slot >> 2);
+    const int j = (slot >> 1) & 1, a = slot & 1;
+    qa[it] = *reinterpret_cast<const uint4 *>(P.ql + blk * 128 + 64 * j + 16 * a);
+    qb[it] = *reinterpret_cast<const uint4 *>(P.ql + blk * 128 + 64 * j + 32 + 16 * a);
+    qh[it] = *reinterpret_cast<const uint4 *>(P.qh + blk * 64 + 32 * j + 16 * a);
+    sc[it] = *reinterpret_cast<const uint2 *>(P.sc + blk * 16 + 8 * j);
+    dd[it] = P.d[blk];
+  }
+  RT_DEV void compute(const uint32_t *dl, int slot, float (&p)[ITERS]) const {
+    const int a = slot & 1;
+    const uint32_t m4 = opaque_u32(0x0F0F0F0Fu), m2 = opaque_u32(0x30303030u);
+    const uint32_t *base = dl + 2 * (slot >> 1) * kAnyPitch<RT_LINEAR_Q6K>;  // the half block's first chunk
+    float acc[ITERS][2];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) acc[it][0] = acc[it][1] = 0.f;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const uint32_t *cb = base + (m >> 1) * kAnyPitch<RT_LINEAR_Q6K>;
+      const int w0 = 8 * (m & 1) + 4 * a;
+      uint4 x[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) x[d] = *reinterpret_cast<const uint4 *>(cb + 16 * d + w0);
+      const uint2 xs = *reinterpret_cast<const uint2 *>(cb + 68 + 2 * (w0 >> 2));
+      const int xs01 = 32 * (int)xs.x, xs2 = 32 * (int)(int16_t)(xs.y & 0xFFFFu);
+      const int xs3 = 32 * (((int)xs.y - (int)(int16_t)(xs.y & 0xFFFFu)) >> 16);
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const uint4 ql = (m & 1) ? qb[it] : qa[it];
+        const uint32_t lw[4] = {ql.x, ql.y, ql.z, ql.w}, hb[4] = {qh[it].x, qh[it].y, qh[it].z, qh[it].w};
+        int s[4] = {-xs01, 0, -xs2, -xs3};  // sum X (q - 32), digit by digit
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t nib = (m < 2 ? lw[k] : lw[k] >> 4) & m4;
+          const int sh = 2 * m;
+          const int q = (int)(nib | ((sh <= 4 ? hb[k] << (4 - sh) : hb[k] >> (sh - 4)) & m2));
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            const uint32_t X[4] = {x[d].x, x[d].y, x[d].z, x[d].w};
+            s[d] = __builtin_amdgcn_sdot4(q, (int)X[k], s[d], false);
+          }
+        }
+        const float t = any_dot(s);
+        const uint32_t scw = m < 2 ? sc[it].x : sc[it].y;  // scales 2m + a of the half block: byte 2*(m&1) + a
+        acc[it][m >> 1] = fmaf((float)(int)__builtin_amdgcn_sbfe(scw, 16 * (m & 1) + 8 * a, 8), t, acc[it][m >> 1]);
+      }
+    }
+    const float d0 = bits_f32(base[64]), d1 = bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]);
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+      const float d = half_bits_to_f32(dd[it]);
+      p[it] = fmaf(acc[it][1], d * d1, acc[it][0] * (d * d0));
+    }
+  }
+  RT_DEV static bool plain(const uint32_t *dl, int slot) {
+    const uint32_t *base = dl + 2 * (slot >> 1) * kAnyPitch<RT_LINEAR_Q6K>;
+    return !__builtin_isnan(bits_f32(base[64])) && !__builtin_isnan(bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]));
+  }
+  // The slot's part of a row in f32: 16 elements of each quarter of its half block.
+  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot) {
+    const Q6KPlanes P = q6k_planes(W, (size_t)N * (K / 256));
+    float acc = 0.f;
+#pragma unroll 1
+    for (int i = 0; i < 64; ++i) {
+      const int e = 128 * ((slot >> 1) & 1) + 32 * (i >> 4) + 16 * (slot & 1) + (i & 15);
+      acc = fmaf(q6k_value(P, (size_t)row * (K / 256) + (slot >> 2), e), x[256 * (slot >> 2) + e], acc);
+    }
+    return acc;
+  }
+};
+
+template <int ITERS>
+struct AnyTile<RT_LINEAR_Q8_0, ITERS> {
+  uint4 qa[ITERS], qb[ITERS];
+  uint32_t dd[ITERS];
+  RT_DEV void load(int it, const uint8_t *W, int N, int K, int row, int slot) {
+    const uint8_t *q = W + (size_t)row * K + 32 * slot;
+    const uint16_t *D = reinterpret_cast<const uint16_t *>(W + (size_t)N * K) + (size_t)row * (K / 32);
+    qa[it] = *reinterpret_cast<const uint4 *>(q);
+    qb[it] = *reinterpret_cast<const uint4 *>(q + 16);
+    dd[it] = D[slot];
+  }
+  RT_DEV void compute(const uint32_t *dl, int slot, float (&p)[ITERS]) const {
+    const uint32_t *base = dl + (slot >> 1) * kAnyPitch<RT_LINEAR_Q8_0>;
+    int s[ITERS][4];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) s[it][d] = 0;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      uint4 x[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) x[d] = *reinterpret_cast<const uint4 *>(base + 16 * d + 8 * (slot & 1) + 4 * g);
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const uint4 q = g ? qb[it] : qa[it];
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            const uint32_t X[4] = {x[d].x, x[d].y, x[d].z, x[d].w};
+            s[it][d] = __builtin_amdgcn_sdot4((int)w[j], (int)X[j], s[it][d], false);
+          }
+      }
+    }
+    const float delta = bits_f32(base[64]);
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) p[it] = half_bits_to_f32(dd[it]) * delta * any_dot(s[it]);
+  }
+  RT_DEV static bool plain(const uint32_t *dl, int slot) {
+    return !__builtin_isnan(bits_f32(dl[(slot >> 1) * kAnyPitch<RT_LINEAR_Q8_0> + 64]));
+  }
+  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot) {
+    float acc = 0.f;
+#pragma unroll 1
+    for (int i = 32 * slot; i < 32 * slot + 32; ++i)
+      acc = fmaf(q8_0_value(W, (size_t)N * K, (size_t)row * K + i), x[i], acc);
+    return acc;
+  }
+};
+
+// Dynamic LDS: the staged chunks, then ITERS * T slot sums.  T = blockDim.x as
+// an argument: reading blockDim makes the runtime fill the launch's hidden
+// arguments, 0.6 us of host time.
+template <int FMT, int ITERS>
+__global__ __launch_bounds__(1024) void k_gemv_any(const uint8_t *__restrict__ W, const float *__restrict__ x,
+                                                   float *__restrict__ y, int N, int K, int S, int rpi, int T) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t any_lds[];
+  const int tid = (int)threadIdx.x;
+  const int nchunk = (K + 63) / 64, nf = K / 4;
+  uint32_t *dl = any_lds;
+  float *red = reinterpret_cast<float *>(any_lds + nchunk * kAnyPitch<FMT>);
+  // activation loads first (the host makes 16 T >= K), so their wait leaves
+  // the weight loads in flight
+  float4 xv[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xv[i] = reinterpret_cast<const float4 *>(x)[min(tid + i * T, nf - 1)];
+  const int slot = tid % S, rsub = tid / S;
+  const int row0 = (int)blockIdx.x * rpi * ITERS;
+  AnyTile<FMT, ITERS> tile;
+  // rows past N, and the threads past rpi * S, re-read a valid row
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) tile.load(it, W, N, K, min(row0 + it * rpi + rsub, N - 1), slot);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int f = tid + i * T;
+    if (i > 0 && i * T >= 16 * nchunk) break;  // uniform
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+    any_stage<FMT>(dl, f, f < nf ? xv[i] : z, f < 16 * nchunk);
+  }
+  __syncthreads();
+  float p[ITERS];
+  tile.compute(dl, slot, p);
+  if constexpr (FMT != RT_LINEAR_Q4K) {
+    if (!AnyTile<FMT, ITERS>::plain(dl, slot)) {
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it)
+        p[it] = AnyTile<FMT, ITERS>::exact(W, x, N, K, min(row0 + it * rpi + rsub, N - 1), slot);
+    }
+  }
+  if (rsub < rpi) {
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) red[it * rpi * S + tid] = p[it];
+  }
+  __syncthreads();
+  // 16 lanes per row: strided slot sums, then across the lanes
+  const int rows = min(rpi * ITERS, N - row0);
+  for (int r = tid >> 4; r < ((rows + 3) & ~3); r += T >> 4) {  // whole waves
+    float s = 0.f;
+    for (int c = tid & 15; c < S; c += 16) s += red[min(r, rows - 1) * S + c];
+    s = row16_sum(s);
+    if ((tid & 15) == 0 && r < rows) y[row0 + r] = s;
+  }
+}
+
+}  // namespace
+
+// Workgroup shape, from a sweep of 256..1024 threads and 1, 2 or 4 rows per
+// thread over 19 shapes (distinct matrices in a graph, us):
+//   T: the smallest multiple of 64 from 512 (768 for K >= 8192, whose staging
+//   is longer; 320 or, below K = 2048, 192 where 512
+//   would leave CUs without a workgroup) whose
+//   whole rows fill at least 0.9 of the threads.  Q4_K 15360x3840: 512 threads
+//   10.0, 960 (no idle thread) 10.9; 3840x15360: 1024 threads 12.0, 960 12.2.
+//   ITERS: the most that keeps about two workgroups per CU (one for K >= 8192:
+//   3072x12288 in 192 workgroups 9.4, 384 10.0, 768 10.3; 12288x3072 in 512
+//   to 768 workgroups 7.4-7.7).  Q6_K stops at two: four spill registers.
+// Before, one wave per row in f32 (kept for longer K): Q4_K 15360x3840 30.3 us
+// (1.1 TB/s; now 10.0, 3.3 TB/s, of a 6.7 us streaming floor), 3072x12288
+// 24.4 -> 9.4; Q6_K 12288x3072 57.5 -> 9.7, 1152x6912 39.2 -> 5.6; Q8_0
+// 12288x3072 47.0 -> 9.7, 6912x1152 8.1 -> 3.7.
+constexpr int kAnyMaxK = 16384;  // four float4 of x per thread at T = 1024
+
+template <int FMT, int ITERS>
+static hipError_t launch_any(const void *W, const float *x, float *y, int N, int K, int S, int T, hipStream_t s) {
+  const int rpi = T / S, rows = rpi * ITERS;
+  const size_t lds = (size_t)((K + 63) / 64) * kAnyPitch<FMT> * 4 + (size_t)rows * S * 4;
+  if (lds > 65536) {  // up to 92 KB of the CU's 160 KB
+    const hipError_t e = hipFuncSetAttribute((const void *)k_gemv_any<FMT, ITERS>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((k_gemv_any<FMT, ITERS>), dim3((unsigned)((N + rows - 1) / rows)), dim3(T), lds, s,
+                     static_cast<const uint8_t *>(W), x, y, N, K, S, rpi, T);
+  return hipGetLastError();
+}
+
+bool gemv_any_ok(int K) { return K <= kAnyMaxK; }
+
+template <int FMT>
+static hipError_t launch_fmt(const void *W, const float *x, float *y, int N, int K, hipStream_t s) {
+  const int S = FMT == RT_LINEAR_Q8_0 ? K / 32 : K / 64;
+  const bool longk = K >= 8192;
+  int t0 = longk ? 768 : 512;
+  if (!longk && N < 200 * (512 / S)) t0 = K < 2048 ? 192 : 320;
+  t0 = std::max(t0, std::max((S + 63) / 64 * 64, (K / 16 + 63) / 64 * 64));
+  int T = t0;
+  for (int t = t0; t <= 1024; t += 64) {
+    const int used = t / S * S, best = T / S * S;
+    if ((long)used * T > (long)best * t) T = t;  // a larger share of busy threads
+    if (10 * (T / S * S) >= 9 * T) break;
+  }
+  const int rpi = T / S, want = longk ? 192 : 448;
+  auto wgs = [&](int it) { return (N + rpi * it - 1) / (rpi * it); };
+  if (FMT != RT_LINEAR_Q6K && wgs(4) >= want) return launch_any<FMT, FMT == RT_LINEAR_Q6K ? 2 : 4>(W, x, y, N, K, S, T, s);
+  if (wgs(2) >= want) return launch_any<FMT, 2>(W, x, y, N, K, S, T, s);
+  return launch_any<FMT, 1>(W, x, y, N, K, S, T, s);
+}
+
+hipError_t launch_gemv_any(int fmt, const void *W, const float *x, float *y, int N, int K, hipStream_t s) {
+  switch (fmt) {
+    case RT_LINEAR_Q4K: return launch_fmt<RT_LINEAR_Q4K>(W, x, y, N, K, s);
+    case RT_LINEAR_Q6K: return launch_fmt<RT_LINEAR_Q6K>(W, x, y, N, K, s);
+    case RT_LINEAR_Q8_0: return launch_fmt<RT_LINEAR_Q8_0>(W, x, y, N, K, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace rt

@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "../../include/rt_hip.h"
 #include "q4k_gemv.hpp"
 #include "rt_device.hpp"
 #include "kquant_layout.hpp"
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(T) void k_q8_0_gemv(const uint8_t *__restrict__ W, 
 }
 
 // ---------------------------------------------------------------------------
-// Generic fallbacks (any K that is a whole number of blocks): one wave per
+// Fallbacks for K beyond gemv_any.hip's staging (whole blocks): one wave per
 // row, f32 arithmetic on activations read from global memory.
 __global__ __launch_bounds__(256) void k_q6k_gemv_generic(const uint8_t *__restrict__ W,
                                                           const float *__restrict__ x, float *__restrict__ y, int n,
@@ -211,6 +212,7 @@ hipError_t launch_q6k_gemv(const void *W, const float *x, float *y, int N, int K
     // against 8.4-10.7 us for 4 to 18 rows (34 distinct matrices in a graph)
     case 10240: return launch_q6k<40, 960, 2>(W, x, y, N, s);
     default:
+      if (gemv_any_ok(K)) return launch_gemv_any(RT_LINEAR_Q6K, W, x, y, N, K, s);
       hipLaunchKernelGGL(k_q6k_gemv_generic, dim3((N + 3) / 4), dim3(256), 0, s, static_cast<const uint8_t *>(W),
                          x, y, N, K / 256);
       return hipGetLastError();
@@ -225,6 +227,7 @@ hipError_t launch_q8_0_gemv(const void *W, const float *x, float *y, int N, int 
     // 8.8-11.1 us for 2 to 9 rows (34 distinct matrices in a graph)
     case 10240: return launch_q8<320, 960, 2>(W, x, y, N, s);
     default:
+      if (gemv_any_ok(K)) return launch_gemv_any(RT_LINEAR_Q8_0, W, x, y, N, K, s);
       hipLaunchKernelGGL(k_q8_0_gemv_generic, dim3((N + 3) / 4), dim3(256), 0, s, static_cast<const uint8_t *>(W),
                          x, y, N, K);
       return hipGetLastError();

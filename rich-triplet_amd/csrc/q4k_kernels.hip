@@ -6,6 +6,7 @@
 //   [0,2) f16 d   [2,4) f16 dmin   [4,16) 6-bit scale/min pairs   [16,144) nibbles
 // Chunk c (0..3) owns nibble bytes [32c, 32c+32): low nibbles are elements
 // 64c+0..31 (sub-block 2c), high nibbles are 64c+32..63 (sub-block 2c+1).
+#include "../../include/rt_hip.h"
 #include "rt_device.hpp"
 #include "q4k_gemv.hpp"
 #include "rt_kernels.hpp"
@@ -172,7 +173,8 @@ __global__ __launch_bounds__(T) void k_q4k_gemv_dig_multi(GemvMats m, const floa
   gemv_dig_tile<NB, T, ITERS>(w, x, y, n, (b - t0) * Q4KTile<NB, T, ITERS>::ROWS);
 }
 
-// Any K (multiple of 256): one wave per row, lanes stride over the row's chunks.
+// K beyond gemv_any.hip's staging (multiple of 256): one wave per row, lanes
+// stride over the row's chunks.
 __global__ __launch_bounds__(256) void k_q4k_gemv_generic(const uint8_t *__restrict__ W, const float *__restrict__ x,
                                                           float *__restrict__ y, int N, int K) {
   const int lane = threadIdx.x & 63;
@@ -258,8 +260,9 @@ static hipError_t launch_dig(const void *W, const float *x, float *y, int N, hip
 // digit-staged activations with workgroup sizes that trade activation staging
 // (once per workgroup) against parallelism: K=2560 with 8 rows per workgroup
 // up to 8k rows, 48 rows (960 threads, two row-iterations) up to 12k, 32 rows
-// beyond; K=2048 with 16 rows; K=10240 with 6 rows (960 threads).  Other K's
-// use the f32-staged tile.
+// beyond; K=2048 with 16 rows; K=10240 with 12 rows (960 threads).  K of 1, 2,
+// 4 or 16 super-blocks use the f32-staged tile (1024x4096 3.2 us against 3.7
+// for gemv_any.hip, and half its error); any other K up to 16384 gemv_any.hip.
 template <int NB, int T, int ITERS>
 static hipError_t launch_dig_multi(const void *const *w, float *const *y, const int *n, int count, const float *x,
                                    hipStream_t s) {
@@ -312,6 +315,7 @@ hipError_t launch_q4k_gemv(const void *W, const float *x, float *y, int N, int K
     case 40: return launch_dig<40, 960, 2>(W, x, y, N, s);
     default: break;
   }
+  if (gemv_any_ok(K)) return launch_gemv_any(RT_LINEAR_Q4K, W, x, y, N, K, s);
   return launch_q4k_gemv_generic(W, x, y, N, K, s);
 }
 

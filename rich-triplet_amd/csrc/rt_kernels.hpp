@@ -16,6 +16,10 @@ hipError_t launch_q4k_gemv_multi(const void *const *w, float *const *y, const in
                                  int K, hipStream_t s);
 hipError_t launch_q4k_gemv_generic(const void *W, const float *x, float *y, int N, int K, hipStream_t s);
 int q4k_gemv_rows_per_wg(int N, int K);
+// y = W x for RT_LINEAR_Q4K, _Q6K or _Q8_0 weights at any K that gemv_any_ok
+// takes (whole blocks; up to 16384).
+bool gemv_any_ok(int K);
+hipError_t launch_gemv_any(int fmt, const void *W, const float *x, float *y, int N, int K, hipStream_t s);
 hipError_t launch_bf16_gemv(const uint16_t *W, const float *x, float *y, int N, int K, hipStream_t s);
 // Q6_K / Q8_0 in the planar device layout of kquant.hip.
 void q6k_repack_host(const uint8_t *src, size_t n_blocks, uint8_t *dst);

@@ -1,0 +1,82 @@
+"""The any-K Q4_K / Q6_K / Q8_0 GEMV (gemv_any.hip) against float64 products
+of the oracle's dequantisers: row lengths and row counts at the edges of its
+workgroup shapes, and non-finite activations."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import rel_l2, to_dev
+from test_kquant import synth_q6k, synth_q8_0
+
+pytestmark = pytest.mark.gpu
+
+Q4K, Q6K, Q8_0 = 1, 4, 5
+
+
+def weight(rt, orc, fmt, n, k, seed):
+    """(device bytes, float64 values [n, k])."""
+    rng = np.random.default_rng(seed)
+    if fmt == Q4K:
+        w = orc.synth_q4k(seed, n, k)
+        return w, orc.q4k_dequant(w, n, k).reshape(n, k).astype(np.float64)
+    if fmt == Q6K:
+        w = synth_q6k(rng, n * k // 256)
+        return rt.q6k_repack(w), orc.q6k_dequant(w, n * k).reshape(n, k).astype(np.float64)
+    w = synth_q8_0(rng, n * k // 32)
+    return rt.q8_0_repack(w), orc.q8_0_dequant(w, n * k).reshape(n, k).astype(np.float64)
+
+
+def gemv(rt, dev, fmt, w, x, n, k):
+    import torch
+    y = torch.full((n + 64,), -7.0, dtype=torch.float32, device=dev)  # 64 words past the end must stay
+    call = {Q4K: rt.q4k_gemv, Q6K: rt.q6k_gemv, Q8_0: rt.q8_0_gemv}[fmt]
+    call(to_dev(w, dev), to_dev(x, dev), y, n, k)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.all(got[n:] == -7.0)
+    return got[:n]
+
+
+# The smallest and longest rows the kernel takes and the first one past it
+# (the wave-per-row kernel), rows of odd slot counts, one row, row counts one
+# off a workgroup's, and counts that take 1, 2 and 4 rows per thread.
+@pytest.mark.parametrize("fmt,n,k", [
+    (Q4K, 1, 768), (Q4K, 229, 3328), (Q4K, 3841, 3840), (Q4K, 10753, 1280), (Q4K, 193, 15360), (Q4K, 65, 16384),
+    (Q4K, 33, 16640),
+    (Q6K, 1, 256), (Q6K, 1151, 6912), (Q6K, 9001, 768), (Q6K, 385, 12288), (Q6K, 50, 16384), (Q6K, 9, 16640),
+    (Q8_0, 3, 32), (Q8_0, 515, 96), (Q8_0, 6913, 1152), (Q8_0, 1000, 9024), (Q8_0, 40, 16384), (Q8_0, 21, 16416),
+])
+def test_gemv_any_matches_float64(rt, orc, dev, fmt, n, k):
+    w, w64 = weight(rt, orc, fmt, n, k, seed=n + k)
+    x = (np.random.default_rng(k).normal(size=k) * np.exp(0.5 * np.random.default_rng(n).normal(size=k))).astype(np.float32)
+    x[k // 2] = 0.0
+    ref = w64 @ x.astype(np.float64)
+    got = gemv(rt, dev, fmt, w, x, n, k)
+    # Error of a row: the products' magnitudes times a few f32 roundings (the
+    # last digit is 2^-23 of a chunk's bound, at most 2^3 the typical |x|);
+    # Q4_K's scaled codes and mins cancel, so both parts count.
+    mag = np.sqrt(((np.abs(w64) + (np.abs(w64).max() if fmt == Q4K else 0)) ** 2) @ (x.astype(np.float64) ** 2)) + 1e-30
+    assert np.max(np.abs(got - ref) / mag) < 4e-6
+    assert rel_l2(got, ref) < 2e-6
+
+
+@pytest.mark.parametrize("fmt,k", [(Q4K, 1280), (Q6K, 1280), (Q8_0, 1152)])
+def test_gemv_any_keeps_non_finite_values(rt, orc, dev, fmt, k):
+    """A NaN makes every row NaN; an infinity makes a row non-finite, its
+    sign the weight's, and not a number where the weight is zero."""
+    n = 70
+    w, w64 = weight(rt, orc, fmt, n, k, seed=5)
+    x = np.random.default_rng(1).normal(size=k).astype(np.float32)
+    x[77] = np.nan
+    assert np.all(np.isnan(gemv(rt, dev, fmt, w, x, n, k)))
+    x[77] = -np.inf
+    got = gemv(rt, dev, fmt, w, x, n, k)
+    assert not np.any(np.isfinite(got))
+    if fmt != Q4K:  # Q4_K: scale * inf - min * inf, not a number in f32 either
+        live = w64[:, 77] != 0
+        assert np.array_equal(np.sign(got[live]), -np.sign(w64[live, 77])) and np.all(np.isnan(got[~live]))
+    for big in (1e33, 1e-28):  # near both ends of the exponent range
+        x[77] = 0.5
+        xs = (x * np.float32(big)).astype(np.float32)
+        assert rel_l2(gemv(rt, dev, fmt, w, xs, n, k), w64 @ xs.astype(np.float64)) < 2e-6
