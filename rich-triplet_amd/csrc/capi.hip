@@ -162,8 +162,8 @@ rt_status rt_q8_0_gemv(const void *w, const float *x, float *y, int64_t n, int64
 namespace {
 rt_status gemm_workspace(size_t bytes, hipStream_t stream, void **out);
 
-rt_status q4k_gemm_entry(const char *who, const void *a, bool a_bf16, const void *w, float *c, int64_t m, int64_t n,
-                         int64_t k, void *stream) {
+rt_status q4k_gemm_entry(const char *who, const void *a, bool a_bf16, const void *w, const float *bias, float *c,
+                         int64_t m, int64_t n, int64_t k, void *stream) {
   if (m <= 0 || n <= 0 || k <= 0)
     return set_error(RT_EINVAL, "%s: m=%lld n=%lld k=%lld must be positive", who, (long long)m, (long long)n,
                      (long long)k);
@@ -172,10 +172,18 @@ rt_status q4k_gemm_entry(const char *who, const void *a, bool a_bf16, const void
   if (!a || !w || !c) return set_error(RT_EINVAL, "%s: null pointer", who);
   if (!aligned16(a) || !aligned16(w)) return set_error(RT_EINVAL, "%s: a and w must be 16-byte aligned", who);
   if ((reinterpret_cast<uintptr_t>(c) & 3u) != 0) return set_error(RT_EINVAL, "%s: c must be 4-byte aligned", who);
+  const bool rows = rows_gemm_ok(RT_LINEAR_Q4K, (int)m, (int)n, (int)k);
   void *ws = nullptr;
-  rt_status st = gemm_workspace(q4k_gemm_workspace_bytes((int)m, (int)n, (int)k), (hipStream_t)stream, &ws);
+  rt_status st = gemm_workspace(rows ? rows_gemm_workspace_bytes(RT_LINEAR_Q4K, (int)m, (int)n, (int)k)
+                                     : q4k_gemm_workspace_bytes((int)m, (int)n, (int)k),
+                                (hipStream_t)stream, &ws);
   if (st != RT_OK) return st;
-  return hip_error(launch_q4k_gemm(a, a_bf16, w, c, (int)m, (int)n, (int)k, ws, (hipStream_t)stream), who);
+  if (rows)
+    return hip_error(launch_rows_gemm(RT_LINEAR_Q4K, a, a_bf16, w, bias, c, (int)m, (int)n, (int)k, ws,
+                                      (hipStream_t)stream), who);
+  hipError_t e = launch_q4k_gemm(a, a_bf16, w, c, (int)m, (int)n, (int)k, ws, (hipStream_t)stream);
+  if (e == hipSuccess && bias) e = launch_add_bias_rows(c, bias, (int)m, (int)n, (hipStream_t)stream);
+  return hip_error(e, who);
 }
 }  // namespace
 
@@ -183,11 +191,11 @@ extern "C" {
 
 rt_status rt_q4k_gemm_bf16(const uint16_t *a, const void *w, float *c, int64_t m, int64_t n, int64_t k,
                            void *stream) {
-  return q4k_gemm_entry("rt_q4k_gemm_bf16", a, true, w, c, m, n, k, stream);
+  return q4k_gemm_entry("rt_q4k_gemm_bf16", a, true, w, nullptr, c, m, n, k, stream);
 }
 
 rt_status rt_q4k_gemm_f32(const float *a, const void *w, float *c, int64_t m, int64_t n, int64_t k, void *stream) {
-  return q4k_gemm_entry("rt_q4k_gemm_f32", a, false, w, c, m, n, k, stream);
+  return q4k_gemm_entry("rt_q4k_gemm_f32", a, false, w, nullptr, c, m, n, k, stream);
 }
 
 // The matmul of QLinear::forward (qlinear.rs:82-111) for a weight of any
@@ -218,11 +226,7 @@ static rt_status linear_forward(const char *who, int32_t fmt, const void *w, con
   if ((reinterpret_cast<uintptr_t>(c) & 3u) != 0) return set_error(RT_EINVAL, "%s: c must be 4-byte aligned", who);
   if (bias && (reinterpret_cast<uintptr_t>(bias) & 3u) != 0)
     return set_error(RT_EINVAL, "%s: bias must be 4-byte aligned", who);
-  if (fmt == RT_LINEAR_Q4K) {
-    rt_status st = q4k_gemm_entry(who, a, false, w, c, m, n, k, stream);
-    if (st != RT_OK || !bias) return st;
-    return hip_error(launch_add_bias_rows(c, bias, (int)m, (int)n, s), who);
-  }
+  if (fmt == RT_LINEAR_Q4K) return q4k_gemm_entry(who, a, false, w, bias, c, m, n, k, stream);
   // f32 / bf16 weights with a few rows, or a K the 64-wide GEMM stages do not
   // divide: the weights stream once per 8 rows, the bias add fused
   if (fmt == RT_LINEAR_F32 && (few || k % 64 != 0))
@@ -230,9 +234,13 @@ static rt_status linear_forward(const char *who, int32_t fmt, const void *w, con
   if (fmt == RT_LINEAR_BF16 && (few || k % 64 != 0))
     return hip_error(launch_bf16_gemv_rows(static_cast<const uint16_t *>(w), a, bias, c, (int)m, (int)n, (int)k, s),
                      who);
+  const bool rows = rows_gemm_ok(fmt, (int)m, (int)n, (int)k);
   void *ws = nullptr;
-  rt_status st = gemm_workspace(proj_gemm_workspace_bytes((int)m, (int)n, (int)k), s, &ws);
+  rt_status st = gemm_workspace(rows ? rows_gemm_workspace_bytes(fmt, (int)m, (int)n, (int)k)
+                                     : proj_gemm_workspace_bytes((int)m, (int)n, (int)k), s, &ws);
   if (st != RT_OK) return st;
+  if (rows)
+    return hip_error(launch_rows_gemm(fmt, a, false, w, bias, c, (int)m, (int)n, (int)k, ws, s), who);
   hipError_t e = launch_proj_gemm(a, fmt, w, c, (int)m, (int)n, (int)k, ws, s);
   if (e == hipSuccess && bias) e = launch_add_bias_rows(c, bias, (int)m, (int)n, s);
   return hip_error(e, who);
@@ -509,21 +517,19 @@ rt_status rt_matmul_q4k_t(const float *a, size_t m, size_t k, const uint8_t *blo
     return set_error(RT_EINVAL, "rt_matmul_q4k_t: m=%zu k=%zu rows=%zu (k must be a positive multiple of 256)", m, k,
                      rows);
   if (m == 1) return rt_gemv_q4k_t(a, k, blocks, rows, out);
-  void *wdev = nullptr, *buf = nullptr, *ws = nullptr;
+  void *wdev = nullptr, *buf = nullptr;
   const size_t wbytes = rows * (k / 256) * 144;
   rt_status st = cached_upload(blocks, wbytes, &wdev);
   if (st != RT_OK) return st;
   const size_t abytes = (m * k * sizeof(float) + 255) & ~size_t(255);
   st = stage(abytes + m * rows * sizeof(float), &buf);
   if (st != RT_OK) return st;
-  st = gemm_workspace(q4k_gemm_workspace_bytes((int)m, (int)rows, (int)k), nullptr, &ws);
-  if (st != RT_OK) return st;
   float *ad = static_cast<float *>(buf);
   float *cd = reinterpret_cast<float *>(static_cast<char *>(buf) + abytes);
   hipError_t e = hipMemcpy(ad, a, m * k * sizeof(float), hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_error(e, "rt_matmul_q4k_t");
-  e = launch_q4k_gemm(ad, false, wdev, cd, (int)m, (int)rows, (int)k, ws, nullptr);
-  if (e != hipSuccess) return hip_error(e, "rt_matmul_q4k_t");
+  st = q4k_gemm_entry("rt_matmul_q4k_t", ad, false, wdev, nullptr, cd, (int64_t)m, (int64_t)rows, (int64_t)k, nullptr);
+  if (st != RT_OK) return st;
   e = hipMemcpy(out, cd, m * rows * sizeof(float), hipMemcpyDeviceToHost);
   return hip_error(e, "rt_matmul_q4k_t");
 }

@@ -32,6 +32,13 @@ hipError_t launch_q8_0_gemv(const void *W, const float *x, float *y, int N, int 
 hipError_t launch_gemm_splitk_sum(const float *part, float *c, size_t mn, int ksplit, hipStream_t s);
 // A (f32 [M][K]) -> f16 with a per-row power-of-two exponent (the GEMMs' A prep).
 hipError_t launch_gemm_prep_a(const float *a, int M, int K, _Float16 *a16, int *ea, hipStream_t s);
+// c[m][n] = a[m][k] . W[n][k] (+ bias[n]) of a few rows on packed RT_LINEAR_Q4K,
+// _Q6K or _Q8_0 weights (rows_gemm.hip), a f32 or bf16 bits; ws holds
+// rows_gemm_workspace_bytes.  rows_gemm_ok: where it is the fastest path.
+bool rows_gemm_ok(int fmt, int M, int N, int K);
+size_t rows_gemm_workspace_bytes(int fmt, int M, int N, int K);
+hipError_t launch_rows_gemm(int fmt, const void *a, bool a_bf16, const void *w, const float *bias, float *c, int M,
+                            int N, int K, void *ws, hipStream_t s);
 // C[M,N] = A[M,K] . W[N,K]^T for a projection stored as RT_LINEAR_Q6K, _Q8_0
 // or _BF16 (planar layouts of kquant.hip): its rows are widened to f16 with a
 // per-row power-of-two scale and multiplied on the matrix cores in f32.
