@@ -67,12 +67,22 @@ struct DecodeArgs {
 // test widths) ...
 bool decode_shape_supported(const DecodeShape &s, const char **why);
 bool decode_rows_divisible(const DecodeShape &s, const char **why);
-// ... and the wider set the rows kernels serve (every projection Q4_K).
+// ... and the wider set that the any-width step (gemv_any.hip) and the rows
+// kernels serve.
 bool decode_shape_generic(const DecodeShape &s, const char **why);
 constexpr int kLmHeadMaxHidden = 4096;
 // Allows the batched lm_head's LDS for `hidden` (once per process and width).
 hipError_t prepare_lm_head_batch(int hidden);
 hipError_t enqueue_decode_step(const DecodeShape &s, const DecodeArgs &a, const LayerArgs *layers, hipStream_t stream);
+// The same step on the kernels of gemv_any.hip: any shape that
+// decode_shape_generic takes, projections of any mix of formats.
+hipError_t enqueue_decode_step_any(const DecodeShape &s, const DecodeArgs &a, const LayerArgs *layers,
+                                   hipStream_t stream);
+// One layer's decode attention and the merge of its key chunks (a.q, a.k, a.v
+// to a.attn and the cache row).
+hipError_t enqueue_decode_attention(const DecodeShape &s, const DecodeArgs &a, const LayerArgs &L, hipStream_t stream);
+// h = gelu_tanh(h) * u, n floats.
+hipError_t launch_gelu_mul_vec(float *h, const float *u, int n, hipStream_t s);
 // Final residual, final norm and lm_head of the token whose last-layer x2
 // and down-projection output sit in a.x2 / a.dn; logits into a.logits.
 hipError_t enqueue_lm_head(const DecodeShape &s, const DecodeArgs &a, const LayerArgs &last, hipStream_t stream);

@@ -58,7 +58,7 @@ struct rt_decode {
   PrefillBuffers pf;                     // rt_decode_prefill scratch (grown on demand)
   PrefillBuffers vb;                     // decode_step_batch rows (kMaxBatch), allocated at create
   bool rows_mb = true;                   // every layer's formats served by the batched GEMVs (verify, short chunks)
-  bool fused = true;                     // the fused single-token kernels serve this shape (else the rows path)
+  bool fused = true;                     // the fused single-token kernels serve this shape (else enqueue_decode_step_any)
   int pf_chunk = 4096;                   // rows per prefill chunk (~180 KB of scratch per row at Gemma-3-4B)
   std::vector<void *> pf_owned;
   int *pf_tokens_host = nullptr;         // pinned staging: [pf.cap] tokens
@@ -126,7 +126,7 @@ rt_status rt_decode_create(const rt_gemma3_config *cfg, rt_decode **out) {
   if (c.hidden <= 0 || c.ffn <= 0 || c.n_q_heads <= 0 || c.n_kv_heads <= 0 || c.head_dim <= 0)
     return set_error(RT_EINVAL, "rt_decode_create: hidden, ffn, heads and head_dim must be positive");
   // The fused single-token kernels where their templates cover the shape,
-  // else every step through the rows kernels (projections in Q4_K only).
+  // else the any-width step, with verify and prefill on the rows kernels.
   const bool fused = decode_shape_supported(s, &why) && decode_rows_divisible(s, &why);
   if (!fused && !decode_shape_generic(s, &why_generic))
     return set_error(RT_EINVAL, "rt_decode_create: unsupported shape: %s (fused kernels), %s (rows kernels)", why,
@@ -646,12 +646,9 @@ rt_status rt_decode_step_async(rt_decode *d, int32_t token, int32_t position) {
   if (st != RT_OK) return st;
   fill_slot(d, 0, token, position);
   if ((st = params_send(d, 1)) != RT_OK) return st;
-  if (!d->fused)  // one row through the rows kernels: batched GEMVs, row attention, lm_head
-    return run_graph(d, d->exec, [&] {
-      RowsPlan plan = rows_plan_params(d, 1);
-      plan.logits = RowsPlan::kLastRow;
-      return enqueue_rows(d->shape, d->args, d->layers.data(), d->vb, plan, d->stream);
-    }, "rt_decode_step");
+  if (!d->fused)
+    return run_graph(d, d->exec, [&] { return enqueue_decode_step_any(d->shape, d->args, d->layers.data(), d->stream); },
+                     "rt_decode_step");
   return run_graph(d, d->exec, [&] { return enqueue_decode_step(d->shape, d->args, d->layers.data(), d->stream); },
                    "rt_decode_step");
 }

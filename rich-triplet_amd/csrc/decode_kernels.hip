@@ -1050,6 +1050,19 @@ static void launch_attn_d(Launch &l, const DecodeArgs &a, const LayerArgs &L, in
   l.check();
 }
 
+hipError_t enqueue_decode_attention(const DecodeShape &s, const DecodeArgs &a, const LayerArgs &L, hipStream_t stream) {
+  Launch l{stream};
+  const int nchunk = L.window > 0 ? s.nchunk_local : s.nchunk_global, group = s.n_q_heads / s.n_kv_heads;
+  if (s.head_dim == 256) launch_attn_d<256>(l, a, L, nchunk, group);
+  else launch_attn_d<128>(l, a, L, nchunk, group);
+  return l.err;
+}
+
+hipError_t launch_gelu_mul_vec(float *h, const float *u, int n, hipStream_t s) {
+  hipLaunchKernelGGL(k_gelu_mul_vec, dim3((n + 255) / 256), dim3(256), 0, s, h, u, n);
+  return hipGetLastError();
+}
+
 // A projection that is not Q4_K: the plain GEMV of its format.
 static void launch_proj(Launch &l, int fmt, const uint8_t *W, const float *x, float *y, int n, int k) {
   if (l.err != hipSuccess) return;
@@ -1076,7 +1089,6 @@ static void launch_prologue(Launch &l, const DecodeShape &s, const DecodeArgs &a
 static hipError_t enqueue_layers(const DecodeShape &s, const DecodeArgs &a, const LayerArgs *layers, hipStream_t stream) {
   Launch l{stream};
   const int qd = s.n_q_heads * s.head_dim, kvd = s.n_kv_heads * s.head_dim;
-  const int group = s.n_q_heads / s.n_kv_heads;
   const bool big = s.hidden == 2560;
   for (int li = 0; li < s.n_layers && l.err == hipSuccess; ++li) {
     const LayerArgs &L = layers[li];
@@ -1105,11 +1117,7 @@ static hipError_t enqueue_layers(const DecodeShape &s, const DecodeArgs &a, cons
       launch_proj(l, L.fmt[kProjK], L.wk, a.xn, a.k, kvd, s.hidden);
       launch_proj(l, L.fmt[kProjV], L.wv, a.xn, a.v, kvd, s.hidden);
     }
-    const int nchunk = L.window > 0 ? s.nchunk_local : s.nchunk_global;
-    if (s.head_dim == 256)
-      launch_attn_d<256>(l, a, L, nchunk, group);
-    else
-      launch_attn_d<128>(l, a, L, nchunk, group);
+    if (l.err == hipSuccess) l.err = enqueue_decode_attention(s, a, L, stream);
     if (!q4(kProjO)) launch_proj(l, L.fmt[kProjO], L.wo, a.attn, a.o, s.hidden, qd);
     else if (qd == 2048) launch_gemv<8, 512, 1>(l, L.wo, a.attn, a.o, s.hidden);
     else launch_gemv<2, 256, 1>(l, L.wo, a.attn, a.o, s.hidden);
@@ -1128,10 +1136,7 @@ static hipError_t enqueue_layers(const DecodeShape &s, const DecodeArgs &a, cons
       launch_prologue<Pro::Resid>(l, s, a, a.hid, a.o, L.g_post_attn, L.g_pre_ffn, a.x2);
       launch_proj(l, L.fmt[kProjGate], L.wgate, a.xn, a.h, s.ffn, s.hidden);
       launch_proj(l, L.fmt[kProjUp], L.wup, a.xn, a.u, s.ffn, s.hidden);
-      if (l.err == hipSuccess) {
-        hipLaunchKernelGGL(k_gelu_mul_vec, dim3((s.ffn + 255) / 256), dim3(256), 0, l.s, a.h, a.u, s.ffn);
-        l.check();
-      }
+      if (l.err == hipSuccess) l.err = launch_gelu_mul_vec(a.h, a.u, s.ffn, l.s);
     }
     if (!q4(kProjDown)) launch_proj(l, L.fmt[kProjDown], L.wdown, a.h, a.dn, s.hidden, s.ffn);
     else if (s.ffn == 10240) launch_gemv<40, 960, 2>(l, L.wdown, a.h, a.dn, s.hidden);
@@ -1221,8 +1226,8 @@ hipError_t enqueue_lm_head_batch(const DecodeShape &s, const DecodeArgs &a, cons
   return l.err;
 }
 
-// Shapes the rows kernels serve: the decode step then runs as a one-row
-// pass of enqueue_rows.  Their projections take any format the batched
+// Shapes the rows kernels serve; their decode step is enqueue_decode_step_any.
+// Their projections take any format the batched
 // GEMVs take; a width that is not whole super-blocks (Gemma-3-1B's hidden
 // 1152) leaves the projections that read it to Q8_0 and BF16.
 bool decode_shape_generic(const DecodeShape &s, const char **why) {

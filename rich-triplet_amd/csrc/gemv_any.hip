@@ -27,6 +27,8 @@
 #include <algorithm>
 
 #include "../../include/rt_hip.h"
+#include "decode.hpp"
+#include "gemma3_math.hpp"
 #include "kquant_layout.hpp"
 #include "q4k_gemv.hpp"
 #include "rt_device.hpp"
@@ -374,6 +376,173 @@ __global__ __launch_bounds__(1024) void k_gemv_any(const uint8_t *__restrict__ W
   }
 }
 
+// ---------------------------------------------------------------------------
+// The decode step's q|k|v and gate|up launches for any hidden width: the
+// prologue of k_qkv / k_gateup (decode_kernels.hip) in front of the same tiles.
+// ---------------------------------------------------------------------------
+// Sum over the T threads (T/64 waves) of a workgroup; `red` holds 16 floats
+// that no earlier call reads.
+RT_DEV float any_block_sum(float v, float *red, int T) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float s = 0.f;
+  for (int i = 0; i < T / 64; ++i) s += red[i];
+  return s;
+}
+
+// x = EMBED: the token's embedding row * embed_scale, else base + rms(add)
+// (1 + g_add); xn = rms(x) (1 + g_out).  Two float4 per thread (8 T >= K).
+// load() issues every global load, finish() returns xn and lets workgroup 0
+// store x and xn.
+template <bool EMBED>
+struct AnyPrologue {
+  float4 add[2], base[2], ga[2], go[2];
+  RT_DEV void load(const DecodeArgs &a, const float *b, const float *ad, const float *g_add, const float *g_out, int K,
+                   int T) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int f = min((int)threadIdx.x + i * T, K / 4 - 1);
+      if constexpr (EMBED) {
+        const uint2 w = reinterpret_cast<const uint2 *>(a.embed + (size_t)a.params[0] * K)[f];
+        add[i] = make_float4(mul_nc(bf16_lo(w.x), a.embed_scale), mul_nc(bf16_hi(w.x), a.embed_scale),
+                             mul_nc(bf16_lo(w.y), a.embed_scale), mul_nc(bf16_hi(w.y), a.embed_scale));
+      } else {
+        add[i] = reinterpret_cast<const float4 *>(ad)[f];
+        base[i] = reinterpret_cast<const float4 *>(b)[f];
+        ga[i] = reinterpret_cast<const float4 *>(g_add)[f];
+      }
+      go[i] = reinterpret_cast<const float4 *>(g_out)[f];
+    }
+  }
+  RT_DEV void finish(const DecodeArgs &a, float *x_out, float *xn_out, float *red, int K, int T, float4 (&xn)[2]) {
+    const float inv_k = 1.0f / (float)K;
+    const int f0 = (int)threadIdx.x, nf = K / 4;
+    if constexpr (!EMBED) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) ss += f0 + i * T < nf ? sumsq4(add[i]) : 0.f;
+      const float r = rms_inv_from_sumsq(any_block_sum(ss, red, T), inv_k, a.eps);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) add[i] = add4(base[i], norm4(add[i], r, ga[i]));
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ss += f0 + i * T < nf ? sumsq4(add[i]) : 0.f;
+    const float r = rms_inv_from_sumsq(any_block_sum(ss, red + 16, T), inv_k, a.eps);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int f = f0 + i * T;
+      xn[i] = norm4(add[i], r, go[i]);
+      if (blockIdx.x == 0 && f < nf) {
+        if (x_out) reinterpret_cast<float4 *>(x_out)[f] = add[i];
+        if (xn_out) reinterpret_cast<float4 *>(xn_out)[f] = xn[i];
+      }
+    }
+  }
+};
+
+template <int FMT>
+RT_DEV void any_stage_pro(uint32_t *dl, const float4 (&xn)[2], int K, int T) {
+  const int nf = K / 4, nst = 16 * ((K + 63) / 64);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int f = (int)threadIdx.x + i * T;
+    if (i > 0 && T >= nst) break;  // uniform
+    any_stage<FMT>(dl, f, f < nf ? xn[i] : make_float4(0.f, 0.f, 0.f, 0.f), f < nst);
+  }
+}
+
+// Rows of q, then k, then (nv > 0) v, all of format FMT; a thread picks its
+// rows' matrix, so a workgroup may hold rows of two.  x goes to a.hid, xn to
+// a.xn (for a v of another format).
+template <int FMT, bool EMBED>
+__global__ __launch_bounds__(1024) void k_any_qkv(DecodeArgs a, LayerArgs L, LayerArgs prev, int K, int S, int rpi,
+                                                  int T, int nv) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t any_lds[];
+  __shared__ float bred[32];
+  const int tid = (int)threadIdx.x;
+  uint32_t *dl = any_lds;
+  float *red = reinterpret_cast<float *>(any_lds + (K + 63) / 64 * kAnyPitch<FMT>);
+  AnyPrologue<EMBED> pro;
+  pro.load(a, a.x2, a.dn, prev.g_post_ffn, L.g_in, K, T);
+  const int qd = a.n_q_heads * a.head_dim, kvd = a.n_kv_heads * a.head_dim, N = qd + kvd + nv;
+  const int slot = tid % S, rsub = tid / S, row0 = (int)blockIdx.x * rpi;
+  const int row = min(row0 + rsub, N - 1);
+  const bool in_q = row < qd, in_k = !in_q && row < qd + kvd;
+  __syncthreads();  // the prologue's loads leave before any weight load of the workgroup
+  AnyTile<FMT, 1> tile;
+  tile.load(0, in_q ? L.wq : (in_k ? L.wk : L.wv), in_q ? qd : kvd, K, row - (in_q ? 0 : (in_k ? qd : qd + kvd)), slot);
+  float4 xn[2];
+  pro.finish(a, a.hid, a.xn, bred, K, T, xn);
+  any_stage_pro<FMT>(dl, xn, K, T);
+  __syncthreads();
+  float p[1];
+  tile.compute(dl, slot, p);
+  if (rsub < rpi) red[tid] = p[0];
+  __syncthreads();
+  const int rows = min(rpi, N - row0);
+  for (int r = tid >> 4; r < ((rows + 3) & ~3); r += T >> 4) {  // whole waves
+    float s = 0.f;
+    for (int c = tid & 15; c < S; c += 16) s += red[min(r, rows - 1) * S + c];
+    s = row16_sum(s);
+    const int n = row0 + r;
+    if ((tid & 15) == 0 && r < rows)
+      (n < qd ? a.q + n : (n < qd + kvd ? a.k + (n - qd) : a.v + (n - qd - kvd)))[0] = s;
+  }
+}
+
+// PAIRS * rpi gate rows and the same up rows; h = gelu_tanh(g) * u.
+template <int FMT, int PAIRS>
+__global__ __launch_bounds__(1024) void k_any_gateup(DecodeArgs a, LayerArgs L, int ffn, int K, int S, int rpi, int T) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t any_lds[];
+  __shared__ float bred[32];
+  const int tid = (int)threadIdx.x;
+  uint32_t *dl = any_lds;
+  float *red = reinterpret_cast<float *>(any_lds + (K + 63) / 64 * kAnyPitch<FMT>);
+  AnyPrologue<false> pro;
+  pro.load(a, a.hid, a.o, L.g_post_attn, L.g_pre_ffn, K, T);
+  const int slot = tid % S, rsub = tid / S, row0 = (int)blockIdx.x * rpi * PAIRS;
+  __syncthreads();
+  AnyTile<FMT, 2 * PAIRS> tile;
+#pragma unroll
+  for (int it = 0; it < 2 * PAIRS; ++it)
+    tile.load(it, it & 1 ? L.wup : L.wgate, ffn, K, min(row0 + (it >> 1) * rpi + rsub, ffn - 1), slot);
+  float4 xn[2];
+  pro.finish(a, a.x2, a.xn, bred, K, T, xn);
+  any_stage_pro<FMT>(dl, xn, K, T);
+  __syncthreads();
+  float p[2 * PAIRS];
+  tile.compute(dl, slot, p);
+  if (rsub < rpi) {
+#pragma unroll
+    for (int it = 0; it < 2 * PAIRS; ++it) red[(PAIRS * (it & 1) + (it >> 1)) * rpi * S + tid] = p[it];
+  }
+  __syncthreads();
+  const int rows = min(rpi * PAIRS, ffn - row0);
+  const float *up = red + PAIRS * rpi * S;
+  for (int r = tid >> 4; r < ((rows + 3) & ~3); r += T >> 4) {
+    const int rr = min(r, rows - 1) * S;
+    float g = 0.f, u = 0.f;
+    for (int c = tid & 15; c < S; c += 16) g += red[rr + c], u += up[rr + c];
+    g = row16_sum(g);
+    u = row16_sum(u);
+    if ((tid & 15) == 0 && r < rows) a.h[row0 + r] = mul_nc(gelu_tanh(g), u);
+  }
+}
+
+// The prologue alone, one workgroup: x to x_out (if any), xn to xn_out.
+template <bool EMBED>
+__global__ __launch_bounds__(512) void k_any_prologue(DecodeArgs a, const float *base, const float *add,
+                                                      const float *g_add, const float *g_out, int K, float *x_out,
+                                                      float *xn_out) {
+  __shared__ float bred[32];
+  AnyPrologue<EMBED> pro;
+  pro.load(a, base, add, g_add, g_out, K, 512);
+  float4 xn[2];
+  pro.finish(a, x_out, xn_out, bred, K, 512, xn);
+}
+
 }  // namespace
 
 // Workgroup shape, from a sweep of 256..1024 threads and 1, 2 or 4 rows per
@@ -408,19 +577,26 @@ static hipError_t launch_any(const void *W, const float *x, float *y, int N, int
 
 bool gemv_any_ok(int K) { return K <= kAnyMaxK; }
 
+// The smallest multiple of 64 threads from t0 (and of at least `per` elements
+// of x each) whose whole rows of S slots fill 0.9 of them, else the fullest.
+static int any_threads(int S, int K, int per, int t0) {
+  t0 = std::max((t0 + 63) / 64 * 64, std::max((S + 63) / 64 * 64, (K / per + 63) / 64 * 64));
+  int T = t0 = std::min(t0, 1024);
+  for (int t = t0; t <= 1024; t += 64) {
+    const int used = t / S * S, best = T / S * S;
+    if ((long)used * T > (long)best * t) T = t;
+    if (10 * (T / S * S) >= 9 * T) break;
+  }
+  return T;
+}
+
 template <int FMT>
 static hipError_t launch_fmt(const void *W, const float *x, float *y, int N, int K, hipStream_t s) {
   const int S = FMT == RT_LINEAR_Q8_0 ? K / 32 : K / 64;
   const bool longk = K >= 8192;
   int t0 = longk ? 768 : 512;
   if (!longk && N < 200 * (512 / S)) t0 = K < 2048 ? 192 : 320;
-  t0 = std::max(t0, std::max((S + 63) / 64 * 64, (K / 16 + 63) / 64 * 64));
-  int T = t0;
-  for (int t = t0; t <= 1024; t += 64) {
-    const int used = t / S * S, best = T / S * S;
-    if ((long)used * T > (long)best * t) T = t;  // a larger share of busy threads
-    if (10 * (T / S * S) >= 9 * T) break;
-  }
+  const int T = any_threads(S, K, 16, t0);
   const int rpi = T / S, want = longk ? 192 : 448;
   auto wgs = [&](int it) { return (N + rpi * it - 1) / (rpi * it); };
   if (FMT != RT_LINEAR_Q6K && wgs(4) >= want) return launch_any<FMT, FMT == RT_LINEAR_Q6K ? 2 : 4>(W, x, y, N, K, S, T, s);
@@ -436,5 +612,122 @@ hipError_t launch_gemv_any(int fmt, const void *W, const float *x, float *y, int
     default: return hipErrorInvalidValue;
   }
 }
+
+// ---------------------------------------------------------------------------
+// The single-token step of a shape without fused templates: six launches per
+// layer (q|k|v, attention, its merge, o, gate|up, down) where the formats of a
+// set agree, each projection of another mix its own GEMV behind k_any_prologue.
+// As a one-row pass of the verify's kernels (eleven launches per layer, split-K
+// partial sums between them) the step at Gemma-3-1B widths (26 layers, hidden
+// 1152, Q8_0, 700 keys, logits to the host) took 1,685 us; so 1,000 us, of which
+// per layer q|k|v 5.0, attention 6.7, merge 4.6, o 4.1, gate|up 7.2 and down
+// 6.1 us, and the BF16 head 104 us (5.8 TB/s).  Error against float64 2.6e-4
+// before (16-bit digits), 1.7e-5 so.
+// ---------------------------------------------------------------------------
+static bool any_set_fmt(int fmt) { return fmt == RT_LINEAR_Q4K || fmt == RT_LINEAR_Q6K || fmt == RT_LINEAR_Q8_0; }
+
+template <int FMT>
+static void any_qkv(const DecodeArgs &a, const LayerArgs &L, const LayerArgs &P, bool first, int K, int rows, int nv,
+                    hipStream_t s) {
+  // about one workgroup per CU: 1,536 rows of 1152 in 220 workgroups of 256
+  const int S = FMT == RT_LINEAR_Q8_0 ? K / 32 : K / 64;
+  const int T = any_threads(S, K, 8, std::max(256, S * ((rows + 255) / 256)));
+  const int rpi = T / S;
+  const dim3 grid((unsigned)((rows + rpi - 1) / rpi));
+  const size_t lds = (size_t)((K + 63) / 64) * kAnyPitch<FMT> * 4 + (size_t)rpi * S * 4;
+  if (first)
+    hipLaunchKernelGGL((k_any_qkv<FMT, true>), grid, dim3(T), lds, s, a, L, P, K, S, rpi, T, nv);
+  else
+    hipLaunchKernelGGL((k_any_qkv<FMT, false>), grid, dim3(T), lds, s, a, L, P, K, S, rpi, T, nv);
+}
+
+template <int FMT, int PAIRS>
+static void any_gateup_p(const DecodeArgs &a, const LayerArgs &L, int ffn, int K, int S, int T, hipStream_t s) {
+  const int rpi = T / S;
+  const size_t lds = (size_t)((K + 63) / 64) * kAnyPitch<FMT> * 4 + (size_t)2 * PAIRS * rpi * S * 4;
+  hipLaunchKernelGGL((k_any_gateup<FMT, PAIRS>), dim3((unsigned)((ffn + rpi * PAIRS - 1) / (rpi * PAIRS))), dim3(T),
+                     lds, s, a, L, ffn, K, S, rpi, T);
+}
+
+template <int FMT>
+static void any_gateup(const DecodeArgs &a, const LayerArgs &L, int ffn, int K, hipStream_t s) {
+  const int S = FMT == RT_LINEAR_Q8_0 ? K / 32 : K / 64;
+  const int T = any_threads(S, K, 8, 512), rpi = T / S;
+  // two gate and two up rows per thread (one each for Q6_K, whose four rows
+  // spill) while that leaves most CUs a workgroup: 6,912 rows in 247
+  if (FMT != RT_LINEAR_Q6K && ffn >= 2 * rpi * 200) any_gateup_p<FMT, FMT == RT_LINEAR_Q6K ? 1 : 2>(a, L, ffn, K, S, T, s);
+  else any_gateup_p<FMT, 1>(a, L, ffn, K, S, T, s);
+}
+
+#define RT_ANY_FMT(fmt, call)                                     \
+  switch (fmt) {                                                  \
+    case RT_LINEAR_Q4K: call(RT_LINEAR_Q4K); break;               \
+    case RT_LINEAR_Q6K: call(RT_LINEAR_Q6K); break;               \
+    default: call(RT_LINEAR_Q8_0); break;                         \
+  }
+
+static hipError_t any_proj(int fmt, const uint8_t *W, const float *x, float *y, int n, int k, hipStream_t s) {
+  switch (fmt) {
+    case RT_LINEAR_Q6K: return launch_q6k_gemv(W, x, y, n, k, s);
+    case RT_LINEAR_Q8_0: return launch_q8_0_gemv(W, x, y, n, k, s);
+    case RT_LINEAR_BF16: return launch_bf16_gemv(reinterpret_cast<const uint16_t *>(W), x, y, n, k, s);
+    default: return launch_q4k_gemv(W, x, y, n, k, s);
+  }
+}
+
+hipError_t enqueue_decode_step_any(const DecodeShape &sh, const DecodeArgs &a, const LayerArgs *layers, hipStream_t s) {
+  const int H = sh.hidden, qd = sh.n_q_heads * sh.head_dim, kvd = sh.n_kv_heads * sh.head_dim;
+  hipError_t e = hipSuccess;
+  auto ok = [&](hipError_t r) { return (e = e == hipSuccess ? r : e) == hipSuccess; };
+  for (int i = 0; i < sh.n_layers; ++i) {
+    const LayerArgs &L = layers[i], &P = layers[i > 0 ? i - 1 : 0];
+    const int fq = L.fmt[kProjQ], fv = L.fmt[kProjV];
+    if (any_set_fmt(fq) && L.fmt[kProjK] == fq) {
+      const int nv = fv == fq ? kvd : 0;
+#define RT_QKV(F) any_qkv<F>(a, L, P, i == 0, H, qd + kvd + nv, nv, s)
+      RT_ANY_FMT(fq, RT_QKV)
+#undef RT_QKV
+      ok(hipGetLastError());
+      if (nv == 0) ok(any_proj(fv, L.wv, a.xn, a.v, kvd, H, s));
+    } else {
+      if (i == 0)
+        hipLaunchKernelGGL(k_any_prologue<true>, dim3(1), dim3(512), 0, s, a, nullptr, nullptr, nullptr, L.g_in, H, a.hid,
+                           a.xn);
+      else
+        hipLaunchKernelGGL(k_any_prologue<false>, dim3(1), dim3(512), 0, s, a, a.x2, a.dn, P.g_post_ffn, L.g_in, H,
+                           a.hid, a.xn);
+      ok(hipGetLastError());
+      ok(any_proj(fq, L.wq, a.xn, a.q, qd, H, s));
+      ok(any_proj(L.fmt[kProjK], L.wk, a.xn, a.k, kvd, H, s));
+      ok(any_proj(fv, L.wv, a.xn, a.v, kvd, H, s));
+    }
+    ok(enqueue_decode_attention(sh, a, L, s));
+    ok(any_proj(L.fmt[kProjO], L.wo, a.attn, a.o, H, qd, s));
+    const int fg = L.fmt[kProjGate];
+    if (any_set_fmt(fg) && L.fmt[kProjUp] == fg) {
+#define RT_GU(F) any_gateup<F>(a, L, sh.ffn, H, s)
+      RT_ANY_FMT(fg, RT_GU)
+#undef RT_GU
+      ok(hipGetLastError());
+    } else {
+      hipLaunchKernelGGL(k_any_prologue<false>, dim3(1), dim3(512), 0, s, a, a.hid, a.o, L.g_post_attn, L.g_pre_ffn, H,
+                         a.x2, a.xn);
+      ok(hipGetLastError());
+      ok(any_proj(fg, L.wgate, a.xn, a.h, sh.ffn, H, s));
+      ok(any_proj(L.fmt[kProjUp], L.wup, a.xn, a.u, sh.ffn, H, s));
+      ok(launch_gelu_mul_vec(a.h, a.u, sh.ffn, s));
+    }
+    ok(any_proj(L.fmt[kProjDown], L.wdown, a.h, a.dn, H, sh.ffn, s));
+    if (e != hipSuccess) return e;
+  }
+  // final residual and norm (transformer4.rs:2370-2380), then the head
+  hipLaunchKernelGGL(k_any_prologue<false>, dim3(1), dim3(512), 0, s, a, a.x2, a.dn, layers[sh.n_layers - 1].g_post_ffn,
+                     a.g_final, H, nullptr, a.xn);
+  ok(hipGetLastError());
+  if (a.lm_q4k) ok(launch_q4k_gemv(a.lm_q4k, a.xn, a.logits, sh.vocab, H, s));
+  else ok(launch_bf16_gemv(a.lm_bf16, a.xn, a.logits, sh.vocab, H, s));
+  return e;
+}
+#undef RT_ANY_FMT
 
 }  // namespace rt

@@ -520,12 +520,13 @@ RowsPlanG rows_plan(int fmt, int M, int N, int K) {
     // 100 rows: 32.8 us against 40.3 with two); Q8_0 the same within 5%
     p.mt = p.tiles == 1 ? 1 : (fmt == RT_LINEAR_Q6K && p.tiles > 2 ? 4 : 2);
   }
-  // K over workgroups: about one workgroup per CU, at least two super-blocks
-  // (four 64-wide chunks) per wave.  2560x10240 of 40 rows: ks 3 to 6 20.2-21.0
-  // us, 1 29.
+  // K over workgroups: about one workgroup per CU (two of the Q4_K form, once
+  // the rows alone give 80), at least two super-blocks (four 64-wide chunks)
+  // per wave.  2560x10240 of 40 rows: ks 3 to 6 20.2-21.0 us, 1 29; of 200
+  // rows (160 workgroups): ks 3 37.8, 1 44.
   const int wgs = (N + 32 * p.nt - 1) / (32 * p.nt) * ((p.tiles + p.mt - 1) / p.mt);
   const int most = q4k ? K / 256 / (2 * kRowsQ4kWaves) : K / 64 / (4 * kRowsWaves);
-  p.ks = std::max(1, std::min(240 / wgs, most));
+  p.ks = std::max(1, std::min((q4k && wgs >= 80 ? 480 : 240) / wgs, most));
   return p;
 }
 
@@ -535,9 +536,12 @@ size_t r256(size_t b) { return (b + 255) & ~size_t(255); }
 
 bool rows_gemm_ok(int fmt, int M, int N, int K) {
   if (fmt != RT_LINEAR_Q4K && fmt != RT_LINEAR_Q6K && fmt != RT_LINEAR_Q8_0) return false;
-  (void)N;
-  (void)K;
-  return M <= 384;
+  // Up to 384 rows at any width (this path against the tiled ones, us: Q4_K
+  // 10240x2560 300 rows 41 / 45, 512 rows 53 / 55; 2560x10240 384 rows 47 / 51,
+  // 450 rows 66 / 57; Q8_0 10000x6016 384 rows 154 / 186).  Longer, where the
+  // output has too few tiles to fill the chip: 2560x2560 1000 rows 38 / 41,
+  // 1024x2560 1000 rows 25 / 38, 6000x2560 640 rows 48 / 47.
+  return M <= 384 || (M <= 1024 && K <= 4096 && (long)M * N <= 2600000);
 }
 
 size_t rows_gemm_workspace_bytes(int fmt, int M, int N, int K) {
