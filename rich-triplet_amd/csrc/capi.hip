@@ -241,9 +241,7 @@ static rt_status linear_forward(const char *who, int32_t fmt, const void *w, con
   if (st != RT_OK) return st;
   if (rows)
     return hip_error(launch_rows_gemm(fmt, a, false, w, bias, c, (int)m, (int)n, (int)k, ws, s), who);
-  hipError_t e = launch_proj_gemm(a, fmt, w, c, (int)m, (int)n, (int)k, ws, s);
-  if (e == hipSuccess && bias) e = launch_add_bias_rows(c, bias, (int)m, (int)n, s);
-  return hip_error(e, who);
+  return hip_error(launch_proj_gemm(a, fmt, w, bias, c, (int)m, (int)n, (int)k, ws, s), who);
 }
 
 rt_status rt_linear_gemm_f32(int32_t fmt, const void *w, const float *a, float *c, int64_t m, int64_t n, int64_t k,

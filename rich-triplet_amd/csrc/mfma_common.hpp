@@ -53,17 +53,26 @@ RT_DEV void lds_wait(u32x4 &a, u32x4 &b, u32x4 &c, u32x4 &d) {
 }
 
 
+// v + bias[col .. col+3], columns past N left alone.
+RT_DEV float4 add_bias4(float4 v, const float *__restrict__ bias, int col, int N) {
+  if (col < N) v.x += bias[col];
+  if (col + 1 < N) v.y += bias[col + 1];
+  if (col + 2 < N) v.z += bias[col + 2];
+  if (col + 3 < N) v.w += bias[col + 3];
+  return v;
+}
+
 // Stores a wave's C tile from v_mfma_f32_32x32x16 accumulators: four row
 // tiles of 32 rows by NT column tiles of 32 columns, register r of tile (i, j)
 // being C[row0 + 32i + 8(r/4) + 4(lane/32) + r%4][col0 + 32j + lane%32],
-// scaled by 2^(ea[row] + ecol[j]).  One 32-row slice at a time goes through
+// scaled by 2^(ea[row] + ecol[j]), plus bias[col] if any.  One 32-row slice at a time goes through
 // `stage` (32 x (32NT + 8) floats of LDS that only this wave uses; the pitch
 // puts the two row groups of a 4-byte write on disjoint banks) and leaves as
 // whole rows in 16-byte lanes, so no store waits on a load and every store
 // instruction writes full row pieces.
 template <int NT>
 RT_DEV void store_c_tile(const floatx16 (&acc)[4][NT], float *stage, float *c, int M, int N, int row0, int col0,
-                         const int *ea, const int (&ecol)[NT]) {
+                         const int *ea, const int (&ecol)[NT], const float *bias = nullptr) {
   constexpr int P = 32 * NT + 8, F4 = 8 * NT, RPI = 64 / F4;
   const int lane = (int)(threadIdx.x & 63), g = lane >> 5, l32 = lane & 31;
   const bool vec = (N & 3) == 0;
@@ -85,7 +94,8 @@ RT_DEV void store_c_tile(const floatx16 (&acc)[4][NT], float *stage, float *c, i
     for (int q = 0; q < 32 / RPI; ++q) {
       const int rl = q * RPI + lane / F4, f = lane % F4;
       const int row = row0 + 32 * i + rl, col = col0 + 4 * f;
-      const float4 v = *reinterpret_cast<const float4 *>(stage + rl * P + 4 * f);
+      float4 v = *reinterpret_cast<const float4 *>(stage + rl * P + 4 * f);
+      if (bias) v = add_bias4(v, bias, col, N);
       if (row < M) {
         float *dst = c + (size_t)row * N + col;
         if (vec && col + 4 <= N) {

@@ -23,186 +23,375 @@
 namespace rt {
 namespace {
 
-// Element e of row n of a projection in format FMT (decode_*_to_f32 values).
+// Elements 8p .. 8p+7 of row n of a weight in format FMT (decode_*_to_f32 values).
 template <int FMT>
-RT_DEV float proj_value(const uint8_t *__restrict__ W, int N, int K, int n, int e) {
+RT_DEV void proj_load8(const uint8_t *__restrict__ W, int N, int K, int n, int p, float (&v)[8]) {
 #pragma clang fp contract(off)
   if constexpr (FMT == RT_LINEAR_BF16) {
-    return bf16_lo((uint32_t) reinterpret_cast<const uint16_t *>(W)[(size_t)n * K + e]);
+    const uint4 q = reinterpret_cast<const uint4 *>(W)[(size_t)n * (K / 8) + p];
+    const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[2 * i] = bf16_lo(u[i]), v[2 * i + 1] = bf16_hi(u[i]);
   } else if constexpr (FMT == RT_LINEAR_F32) {
-    return reinterpret_cast<const float *>(W)[(size_t)n * K + e];
+    const float4 *r = reinterpret_cast<const float4 *>(W) + (size_t)n * (K / 4) + 2 * p;
+    const float4 a = r[0], b = r[1];
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
   } else if constexpr (FMT == RT_LINEAR_Q8_0) {
-    return q8_0_value(W, (size_t)N * K, (size_t)n * K + e);
-  } else {  // RT_LINEAR_Q6K, planar
-    return q6k_value(q6k_planes(W, (size_t)N * (K / 256)), (size_t)n * (K / 256) + e / 256, e & 255);
+    const uint2 q = reinterpret_cast<const uint2 *>(W)[(size_t)n * (K / 8) + p];
+    const float d = half_bits_to_f32(reinterpret_cast<const uint16_t *>(W + (size_t)N * K)[(size_t)n * (K / 32) + (p >> 2)]);
+    const uint32_t u[2] = {q.x, q.y};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = d * (float)(int8_t)(u[i >> 2] >> (8 * (i & 3)));
+  } else {  // RT_LINEAR_Q6K, planar: piece p is l = 8 (p & 3) .. of quarter m of half j (see q6k_value)
+    const Q6KPlanes P = q6k_planes(W, (size_t)N * (K / 256));
+    const size_t blk = (size_t)n * (K / 256) + (p >> 5);
+    const int j = (p >> 4) & 1, m = (p >> 2) & 3, l = 8 * (p & 3);
+    const uint2 ql = *reinterpret_cast<const uint2 *>(P.ql + blk * 128 + 64 * j + 32 * (m & 1) + l);
+    const uint2 qh = *reinterpret_cast<const uint2 *>(P.qh + blk * 64 + 32 * j + l);
+    const float s = half_bits_to_f32(P.d[blk]) * (float)(int8_t)P.sc[blk * 16 + 8 * j + (l >> 4) + 2 * m];
+    const uint32_t lo[2] = {(ql.x >> (m < 2 ? 0 : 4)) & 0x0F0F0F0Fu, (ql.y >> (m < 2 ? 0 : 4)) & 0x0F0F0F0Fu};
+    const uint32_t hi[2] = {(qh.x >> (2 * m)) & 0x03030303u, (qh.y >> (2 * m)) & 0x03030303u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t c = ((lo[i >> 2] | (hi[i >> 2] << 4)) >> (8 * (i & 3))) & 0x3Fu;
+      v[i] = s * (float)((int)c - 32);
+    }
   }
 }
 
-// One row per workgroup: bound, exponent, then the scaled f16 row.
+// One row per wave: its bound and exponent, then its f16 pieces; the first
+// 64 * 8 * kKeep values stay in registers between the two, the rest is read
+// again.
 template <int FMT>
-__global__ __launch_bounds__(256) void k_rows_to_f16(const uint8_t *__restrict__ W, int N, int K,
-                                                     _Float16 *__restrict__ w16, int *__restrict__ ew) {
-  __shared__ float red[4];
-  const int n = (int)blockIdx.x;
-  float amax = 0.f;
-  for (int e = threadIdx.x; e < K; e += 256) amax = fmaxf(amax, fabsf(proj_value<FMT>(W, N, K, n, e)));
-  amax = wave_max(amax);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
-  __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const int ex = f16_exponent_for(amax);
-  if (threadIdx.x == 0) ew[n] = ex;
-  for (int e = threadIdx.x; e < K; e += 256)
-    w16[(size_t)n * K + e] = (_Float16)__builtin_amdgcn_ldexpf(proj_value<FMT>(W, N, K, n, e), -ex);
+RT_DEV void row_to_f16(const uint8_t *__restrict__ W, int N, int K, int n, _Float16 *__restrict__ w16,
+                       int *__restrict__ ew) {
+  constexpr int kKeep = 6;
+  const int lane = (int)(threadIdx.x & 63), np = K / 8;
+  float v[kKeep][8], amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < kKeep; ++i) {
+    if (64 * i >= np) break;  // wave-uniform
+    proj_load8<FMT>(W, N, K, n, min(lane + 64 * i, np - 1), v[i]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[i][k]));
+  }
+  for (int p = lane + 64 * kKeep; p < np; p += 64) {
+    float t[8];
+    proj_load8<FMT>(W, N, K, n, p, t);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(t[k]));
+  }
+  const int ex = f16_exponent_for(wave_max(amax));
+  if (lane == 0) ew[n] = ex;
+  auto store = [&](int p, const float (&x)[8]) {
+    const uint2 lo = f16x4_scaled(make_float4(x[0], x[1], x[2], x[3]), ex);
+    const uint2 hi = f16x4_scaled(make_float4(x[4], x[5], x[6], x[7]), ex);
+    reinterpret_cast<uint4 *>(w16)[(size_t)n * np + p] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+  };
+#pragma unroll
+  for (int i = 0; i < kKeep; ++i)
+    if (lane + 64 * i < np) store(lane + 64 * i, v[i]);
+  for (int p = lane + 64 * kKeep; p < np; p += 64) {
+    float t[8];
+    proj_load8<FMT>(W, N, K, n, p, t);
+    store(p, t);
+  }
 }
 
-// C[M][N] = 2^(ea[m]+ew[n]) * sum_k a16[m][k] w16[n][k] on
-// v_mfma_f32_32x32x16_f16.  C tile 256 x 256 per workgroup of four waves
-// (2 x 2), each wave 128 x 128 = 4 x 4 MFMA tiles with its 256 accumulator
-// registers in AGPRs (one wave per SIMD issues MFMAs back to back).
-//   Operands: K moves in stages of 64 through two LDS slots per operand,
-//   filled by global_load_lds_dwordx4 (no VGPRs), each copy instruction
-//   moving whole 128-B row pieces.  A slot row is 128 B (8 segments of 8
-//   halves) and holds logical segment s at physical segment
-//   s ^ ((row >> 1) & 7), so the 16 lanes served together by a ds_read_b128
-//   (16 consecutive rows) hit 16 distinct bank groups.  Lane l of an MFMA
-//   reads row l%32 of its 32-row tile; k-step t of a stage is logical
-//   segment 2t + l/32.
-//   Schedule per stage: each k-step's MFMAs run while the next k-step's
-//   fragments are read; before the last k-step's MFMAs, the barrier that
-//   publishes the next stage (and frees this slot), the refill of this slot
-//   two stages ahead, and the next stage's first fragment reads.
-//   Epilogue: store_c_tile (32-row slices staged in LDS, 16-byte stores).
-//   Measured on the config-4 shapes (4608 x 9216 x 3072): loads and LDS reads
-//   alone take about 60% of the kernel's time; the two-slot ring keeps one
-//   stage in flight, which is what bounds the overlap with the MFMAs.
-constexpr int kFTile = 256, kFK = 64;
-constexpr int kFSlot = kFTile * kFK * 2;  // 32 KB per operand per stage
+// Rows [0, M) are A's (f32), the rest W's.  Bound by memory: 16-byte pieces,
+// four rows per workgroup.  Element by element with one row per workgroup and
+// a second read of every value the same widening took (W alone) 14.3 us for
+// BF16 3072x3072 and 15.3 us for Q8_0 6912x1152.
+template <int FMT>
+__global__ __launch_bounds__(256) void k_rows_to_f16(const float *__restrict__ a, int M, _Float16 *__restrict__ a16,
+                                                     int *__restrict__ ea, const uint8_t *__restrict__ W, int N, int K,
+                                                     _Float16 *__restrict__ w16, int *__restrict__ ew) {
+  const int r = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (r < M)
+    row_to_f16<RT_LINEAR_F32>(reinterpret_cast<const uint8_t *>(a), M, K, r, a16, ea);
+  else if (r - M < N)
+    row_to_f16<FMT>(W, N, K, r - M, w16, ew);
+}
 
-__global__ __launch_bounds__(256) void k_gemm_f16_t256(const _Float16 *__restrict__ a16, const int *__restrict__ ea,
+// The tile of workgroup `bid`: XCD b % 8 gets a contiguous run of tiles, walked
+// in groups of eight tile rows so neighbours share A and W in L2.
+RT_DEV void pick_tile(int bid, int tiles_m, int tiles_n, int &tm, int &tn) {
+  const int ntiles = tiles_m * tiles_n, x = bid & 7, r = ntiles & 7, q = ntiles >> 3;
+  const int tile = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (bid >> 3);
+  const int group = tile / (8 * tiles_n), in_group = tile % (8 * tiles_n), gm = min(8, tiles_m - group * 8);
+  tm = group * 8 + in_group % gm;
+  tn = in_group / gm;
+}
+
+// ---------------------------------------------------------------------------
+// C[M][N] = 2^(ea[m]+ew[n]) * sum_k a16[m][k] w16[n][k] (+ bias[n]), C tile
+// 128 x 128, for outputs of few tiles.  Eight waves, two per SIMD: four own 64
+// x 64 of C each and the other four the same, the two groups taking
+// half of every K stage (64 wide), so a stage's fragments are read
+// once per group (64 KB of LDS reads per stage where 64 x 32 wave tiles read
+// 96) and one wave's waits run under the other's MFMAs.  The groups' sums meet
+// in LDS at the end.
+//   Stages arrive by global_load_lds_dwordx4 two ahead in a ring of three
+//   32 KB slots (four and five slots: the same within 2%); one barrier per
+//   stage.  A slot row is 128 B (8 segments of 8 halves), logical segment s at
+//   s ^ ((row >> 1) & 7), so the 16 lanes served together by a ds_read_b128
+//   hit 16 distinct bank groups.
+//   1000 x 3072 x 3072 (192 tiles): 33 us (570 TFLOP/s) against 48 us for the
+//   256 x 256 tiles split five ways with their sum; 512 x 2560 x 10240 split
+//   three ways 41 us.
+// ---------------------------------------------------------------------------
+constexpr int kT128Slots = 3;
+
+__global__ __launch_bounds__(512) void k_gemm_f16_t128(const _Float16 *__restrict__ a16, const int *__restrict__ ea,
                                                        const _Float16 *__restrict__ w16, const int *__restrict__ ew,
-                                                       float *__restrict__ c, int M, int N, int K, int tiles_m,
-                                                       int tiles_n, int ksplit) {
-  // [A slot 0 | A slot 1 | B slot 0 | B slot 1]; the epilogue reuses the start
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * kFSlot];
-  auto slot_a = [&](int i) __attribute__((always_inline)) { return lds + i * kFSlot; };
-  auto slot_b = [&](int i) __attribute__((always_inline)) { return lds + (2 + i) * kFSlot; };
+                                                       const float *__restrict__ bias, float *__restrict__ c, int M,
+                                                       int N, int K, int tiles_m, int tiles_n, int ksplit) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kT128Slots][2][128 * 128];
   const int tid = (int)threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  // Workgroup b runs on XCD b % 8: give each XCD a contiguous run of tiles,
-  // walked in groups of eight tile rows so neighbours share A and W in L2.
-  const int ntiles = tiles_m * tiles_n, per_xcd = (ntiles + 7) / 8;
-  const int bid = (int)blockIdx.x;
-  const int tile = ntiles % 8 == 0 ? (bid & 7) * per_xcd + (bid >> 3) : bid;
-  const int group = tile / (8 * tiles_n), in_group = tile % (8 * tiles_n);
-  const int gm = min(8, tiles_m - group * 8);
-  const int m0 = (group * 8 + in_group % gm) * kFTile, n0 = (in_group / gm) * kFTile;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+  int tm, tn;
+  pick_tile((int)blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * 128, n0 = tn * 128;
   // Split-K: blockIdx.y = s takes stages [s*nk/ksplit, (s+1)*nk/ksplit) and,
   // with ksplit > 1, writes its scaled partial tile to c + s*M*N.
-  const int nk_all = K / kFK, split = (int)blockIdx.y;
-  const int kb = split * nk_all / ksplit, nk = (split + 1) * nk_all / ksplit - kb;  // nk >= 1 (host)
+  const int nk = K / 64, split = (int)blockIdx.y, kb = split * nk / ksplit, n = (split + 1) * nk / ksplit - kb;  // n >= 1
   if (ksplit > 1) c += (size_t)split * M * N;
-
-  // Copies: wave w moves rows [64w, 64w+64) of both operands, eight 1 KB
-  // instructions each; lane -> row 8*(8w+i) + lane/8, physical segment lane%8.
-  const _Float16 *a_src[8], *b_src[8];
+  const uint8_t *ab = reinterpret_cast<const uint8_t *>(a16 + (size_t)m0 * K) + (size_t)kb * 128;
+  const uint8_t *wb = reinterpret_cast<const uint8_t *>(w16 + (size_t)n0 * K) + (size_t)kb * 128;
+  uint32_t ao[2], bo[2];  // copy i: rows 8 (2 wave + i) + [0, 8), eight lanes per row
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 64 * wave + 8 * i + (lane >> 3);
-    const int seg = (lane & 7) ^ ((r >> 1) & 7);
-    a_src[i] = a16 + (size_t)min(m0 + r, M - 1) * K + 8 * seg;
-    b_src[i] = w16 + (size_t)min(n0 + r, N - 1) * K + 8 * seg;
+  for (int i = 0; i < 2; ++i) {
+    const int r = 8 * (2 * wave + i) + (lane >> 3), seg = 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    ao[i] = (uint32_t)(min(m0 + r, M - 1) - m0) * (uint32_t)K * 2u + seg;
+    bo[i] = (uint32_t)(min(n0 + r, N - 1) - n0) * (uint32_t)K * 2u + seg;
   }
-  auto issue = [&](int kt, int slot) __attribute__((always_inline)) {  // kt: stage of this split
-    uint8_t *da = slot_a(slot), *db = slot_b(slot);
-    kt += kb;
+  auto issue = [&](int j, int slot) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      __builtin_amdgcn_global_load_lds((gvoid *)(a_src[i] + (size_t)kt * kFK), (lvoid *)(da + (8 * wave + i) * 1024),
-                                       16, 0, 0);
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds((gvoid *)(ab + (size_t)j * 128 + ao[i]),
+                                       (lvoid *)(lds[slot][0] + (2 * wave + i) * 1024), 16, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      __builtin_amdgcn_global_load_lds((gvoid *)(b_src[i] + (size_t)kt * kFK), (lvoid *)(db + (8 * wave + i) * 1024),
-                                       16, 0, 0);
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds((gvoid *)(wb + (size_t)j * 128 + bo[i]),
+                                       (lvoid *)(lds[slot][1] + (2 * wave + i) * 1024), 16, 0, 0);
   };
-  int ra[4], rb[4];  // this lane's fragment rows
+  uint32_t fa[2], fb[2];  // this group's k-steps 2 kg + t: segment 2 (2 kg + t) + g of the lane's row
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    ra[i] = 128 * wm + 32 * i + l32;
-    rb[i] = 128 * wn + 32 * i + l32;
+  for (int t = 0; t < 2; ++t) {
+    const uint32_t seg = 16 * ((2 * (2 * kg + t) + g) ^ ((l32 >> 1) & 7));
+    fa[t] = (64 * wm + l32) * 128 + seg;
+    fb[t] = (64 * wn + l32) * 128 + seg;
   }
-  auto frag_off = [&](int r, int s) __attribute__((always_inline)) { return r * 128 + 16 * (s ^ ((r >> 1) & 7)); };
-  auto read = [&](int slot, int s, u32x4 (&af)[4], u32x4 (&bf)[4]) __attribute__((always_inline)) {
-    const uint8_t *pa = slot_a(slot), *pb = slot_b(slot);
+  floatx16 acc[2][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      af[i] = lds_read16(pa + frag_off(ra[i], s));
-      bf[i] = lds_read16(pb + frag_off(rb[i], s));
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
+#pragma unroll
+  for (int i = 0; i < kT128Slots - 1; ++i) issue(min(i, n - 1), i);
+  // Past the last stage the copies repeat it, so every stage issues four.
+  auto stage = [&](int j, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<4 * (kT128Slots - 2)>();  // stage j's copies; the next stage's may be in flight
+    wg_barrier();                        // everyone's; the slot refilled below is read out
+    issue(min(j + kT128Slots - 1, n - 1), slot == 0 ? kT128Slots - 1 : slot - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 af[2][2], bf[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        af[t][i] = lds_read16(lds[slot][0] + fa[t] + 4096 * i);
+        bf[t][i] = lds_read16(lds[slot][1] + fb[t] + 4096 * i);
+      }
+    auto mfma4 = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          acc[i][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, af[t][i]),
+                                                              __builtin_bit_cast(half8, bf[t][q]), acc[i][q], 0, 0, 0);
+    };
+    asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(af[0][0]), "+v"(af[0][1]), "+v"(bf[0][0]), "+v"(bf[0][1]));
+    mfma4(0);
+    lds_wait(af[1][0], af[1][1], bf[1][0], bf[1][1]);
+    mfma4(1);
+  };
+  static_assert(kT128Slots == 3, "the loop below is unrolled by the ring");
+  int j = 0;
+  for (; j + 3 <= n; j += 3) {
+    stage(j, 0);
+    stage(j + 1, 1);
+    stage(j + 2, 2);
+  }
+  if (j < n) stage(j, 0);
+  if (j + 1 < n) stage(j + 1, 1);
+  wait_vmcnt<0>();
+  wg_barrier();
+  // group 1's sums to LDS, group 0 adds its own and scales, both store
+  constexpr int P = 72;
+  static_assert(4 * 64 * P * 4 <= kT128Slots * 2 * 128 * 128, "the staged tile fits in the ring");
+  float *st = reinterpret_cast<float *>(&lds[0][0][0]) + (wave & 3) * 64 * P;
+  if (kg) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[(32 * i + 8 * (r >> 2) + 4 * g + (r & 3)) * P + 32 * q + l32] = acc[i][q][r];
+  }
+  __syncthreads();
+  if (!kg) {
+    int ec[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) ec[q] = ew[min(n0 + 64 * wn + 32 * q + l32, N - 1)];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int R = 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), er = ea[min(m0 + 64 * wm + R, M - 1)];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float *p = st + R * P + 32 * q + l32;
+          *p = __builtin_amdgcn_ldexpf(acc[i][q][r] + *p, er + ec[q]);
+        }
+      }
+  }
+  __syncthreads();
+  const bool vec = (N & 3) == 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int R = 32 * kg + 4 * q + (lane >> 4), f = lane & 15, row = m0 + 64 * wm + R, col = n0 + 64 * wn + 4 * f;
+    float4 v = *reinterpret_cast<const float4 *>(st + R * P + 4 * f);
+    if (bias) v = add_bias4(v, bias, col, N);
+    if (row >= M) continue;
+    float *dst = c + (size_t)row * N + col;
+    if (vec) {
+      if (col < N) *reinterpret_cast<float4 *>(dst) = v;
+    } else {
+      const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (col + k < N) dst[k] = x[k];
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same product on 256 x 256 tiles, one workgroup per CU: eight waves of
+// 128 x 64, two per SIMD.  The two groups of four waves run half a stage apart
+// between workgroup barriers: while one multiplies (16 MFMAs), the other reads
+// its next fragments and issues its copies, so each SIMD's matrix core always
+// has one wave's MFMAs.
+//   K moves in stages of 32 through four slots of 16 KB per operand, copied
+//   three stages ahead.  A slot row is 64 B (4 segments of 8 halves), logical
+//   segment s at s ^ ((row >> 2) & 3): the 16 lanes of a ds_read_b128 hit 16
+//   distinct bank groups.
+//   4608 x 12288 x 3072 333 us (1.04 PFLOP/s; the four-wave form with 64-wide
+//   stages and 128 x 128 wave tiles 400), 4096 x 4096 x 2560 82 us, 2000 x 12000
+//   x 3072 159 us.  With zero operands 250 us: the rest is the card's power
+//   limit.  Storing C takes 45 us of the 333.
+// ---------------------------------------------------------------------------
+constexpr int kT256Slot = 256 * 64;  // one operand, one stage
+
+__global__ __launch_bounds__(512, 2) void k_gemm_f16_t256(const _Float16 *__restrict__ a16, const int *__restrict__ ea,
+                                                          const _Float16 *__restrict__ w16, const int *__restrict__ ew,
+                                                          const float *__restrict__ bias, float *__restrict__ c, int M,
+                                                          int N, int K, int tiles_m, int tiles_n) {
+  __shared__ __attribute__((aligned(1024))) uint8_t sa[4][kT256Slot], sb[4][kT256Slot];
+  const int tid = (int)threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3;
+  int tm, tn;
+  pick_tile((int)blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * 256, n0 = tn * 256, n = K / 32;
+  const uint8_t *ab = reinterpret_cast<const uint8_t *>(a16 + (size_t)m0 * K);
+  const uint8_t *wb = reinterpret_cast<const uint8_t *>(w16 + (size_t)n0 * K);
+  uint32_t ao[2], bo[2];  // copy i: rows 16 (2 wave + i) + [0, 16), four lanes per row
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 16 * (2 * wave + i) + (lane >> 2), seg = 16 * ((lane & 3) ^ ((r >> 2) & 3));
+    ao[i] = (uint32_t)(min(m0 + r, M - 1) - m0) * (uint32_t)K * 2u + seg;
+    bo[i] = (uint32_t)(min(n0 + r, N - 1) - n0) * (uint32_t)K * 2u + seg;
+  }
+  auto issue = [&](int j, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds((gvoid *)(ab + (size_t)j * 64 + ao[i]), (lvoid *)(sa[slot] + (2 * wave + i) * 1024),
+                                       16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds((gvoid *)(wb + (size_t)j * 64 + bo[i]), (lvoid *)(sb[slot] + (2 * wave + i) * 1024),
+                                       16, 0, 0);
   };
-  auto await = [&](u32x4 (&af)[4], u32x4 (&bf)[4]) __attribute__((always_inline)) {
-    lds_wait(af[0], af[1], af[2], af[3]);
-    lds_wait(bf[0], bf[1], bf[2], bf[3]);
-  };
-  floatx16 acc[4][4];
+  uint32_t fa[2], fb[2];  // k-step t: segment 2t + g; 32 rows further is 2048 bytes (whole swizzle periods)
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const uint32_t seg = 16 * ((2 * t + g) ^ ((l32 >> 2) & 3));
+    fa[t] = (128 * wm + l32) * 64 + seg;
+    fb[t] = (64 * wn + l32) * 64 + seg;
+  }
+  floatx16 acc[4][2];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = floatx16{};
-  auto mfma16 = [&](const u32x4 (&af)[4], const u32x4 (&bf)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, af[i]),
-                                                            __builtin_bit_cast(half8, bf[j]), acc[i][j], 0, 0, 0);
-  };
-
+    for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
+  // Past the last stage the copies repeat it, so every stage issues four.
   issue(0, 0);
-  if (nk > 1) issue(1, 1);
-  u32x4 a0[4], b0[4], a1[4], b1[4];
-  if (nk > 1) wait_vmcnt<16>();  // stage 0 landed, stage 1 may be in flight
-  else wait_vmcnt<0>();
+  issue(min(1, n - 1), 1);
+  issue(min(2, n - 1), 2);
+  wait_vmcnt<8>();
   wg_barrier();
-  read(0, g, a0, b0);
-  await(a0, b0);
-  auto step = [&](int kt, int slot) __attribute__((always_inline)) {
-    read(slot, 2 + g, a1, b1);
-    mfma16(a0, b0);
-    await(a1, b1);
-    read(slot, 4 + g, a0, b0);
-    mfma16(a1, b1);
-    await(a0, b0);
-    read(slot, 6 + g, a1, b1);
-    mfma16(a0, b0);
-    await(a1, b1);
-    if (kt + 1 < nk) {
-      wait_vmcnt<0>();  // stage kt+1, the only one in flight, has landed
-      wg_barrier();     // everywhere, and this slot is read out everywhere
-      __builtin_amdgcn_sched_barrier(0);
-      if (kt + 2 < nk) issue(kt + 2, slot);
-      __builtin_amdgcn_sched_barrier(0);
-      read(slot ^ 1, g, a0, b0);
-    }
-    mfma16(a1, b1);
-    if (kt + 1 < nk) await(a0, b0);
-  };
-  int kt = 0;
-  for (; kt + 2 <= nk; kt += 2) {
-    step(kt, 0);
-    step(kt + 1, 1);
-  }
-  if (kt < nk) step(kt, 0);
-
-  // Epilogue: the wave's 128 x 128 tile through LDS in 32-row slices (17 KB
-  // per wave at the start of the free slots), 16-byte stores.
-  int ec[4];
+  if (wm) wg_barrier();  // group 1 runs half a stage behind
+  auto stage = [&](int j, int slot) __attribute__((always_inline)) {
+    u32x4 af[2][4], bf[2][2];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) ec[j] = ew[min(n0 + rb[j], N - 1)];
-  wg_barrier();  // the slots are free: every wave's last fragments are read
-  store_c_tile<4>(acc, reinterpret_cast<float *>(lds) + wave * 32 * (32 * 4 + 8), c, M, N, m0 + 128 * wm,
-                  n0 + 128 * wn, ea, ec);
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) bf[t][i] = lds_read16(sb[slot] + fb[t] + 2048 * i);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) af[t][i] = lds_read16(sa[slot] + fa[t] + 2048 * i);
+    }
+    // the slot of stage j-1: both groups have read it (group 1 in the half
+    // stage that the last barrier closed)
+    issue(min(j + 3, n - 1), (slot + 3) & 3);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<8>();  // this wave's part of stage j+1, published by the barrier
+    lds_wait(af[0][0], af[0][1], af[0][2], af[0][3]);
+    lds_wait(af[1][0], af[1][1], af[1][2], af[1][3]);
+    lds_wait(bf[0][0], bf[0][1], bf[1][0], bf[1][1]);
+    wg_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          acc[i][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, af[t][i]),
+                                                              __builtin_bit_cast(half8, bf[t][q]), acc[i][q], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    wg_barrier();
+  };
+  int j = 0;
+  for (; j + 4 <= n; j += 4) {
+    stage(j, 0);
+    stage(j + 1, 1);
+    stage(j + 2, 2);
+    stage(j + 3, 3);
+  }
+  if (j < n) stage(j, 0);
+  if (j + 1 < n) stage(j + 1, 1);
+  if (j + 2 < n) stage(j + 2, 2);
+  if (!wm) wg_barrier();  // as many barriers as group 1
+  wait_vmcnt<0>();
+  wg_barrier();
+  int ec[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) ec[q] = ew[min(n0 + 64 * wn + 32 * q + l32, N - 1)];
+  static_assert(32 * 72 * 4 <= kT256Slot, "a staging slice fits in a slot");
+  store_c_tile<2>(acc, reinterpret_cast<float *>(wave < 4 ? sa[wave] : sb[wave - 4]), c, M, N, m0 + 128 * wm,
+                  n0 + 64 * wn, ea, ec, bias);
 }
 
 // ---------------------------------------------------------------------------
@@ -350,72 +539,96 @@ hipError_t launch_add_bias_rows(float *c, const float *bias, int M, int N, hipSt
   return hipGetLastError();
 }
 
-// Split-K count: enough workgroups to cover the 256 CUs when the output has
-// few 256 x 256 tiles (M = 512, N = 2560: 20 tiles), at least 8 stages
-// (K = 512) per split.
-static int proj_ksplit(int M, int N, int K) {
-  const int ntiles = ((M + kFTile - 1) / kFTile) * ((N + kFTile - 1) / kFTile);
-  return std::max(1, std::min(256 / ntiles, (K / kFK) / 8));
+// Kernel and K split of an M x N x K product, by a time model fitted to
+// measurements (us): 256 x 256 tiles, one per CU and round, 0.0267 per unit of K;
+// 128 x 128 tiles 0.0100 per unit of K and round, plus 4 per launch; a split
+// adds the sum kernel and (2 ks + 1) M N words at 5 TB/s.  1000x3072x3072: 192
+// small tiles in one round 33 against 65; 2000x12000x3072: 376 large tiles 159
+// against 196; 512x2560x10240: 80 small tiles split three ways 41, whole 79.
+struct ProjPlan {
+  bool big;
+  int ks;
+};
+static ProjPlan proj_plan(int M, int N, int K) {
+  const long tb = (long)((M + 255) / 256) * ((N + 255) / 256), ts = (long)((M + 127) / 128) * ((N + 127) / 128);
+  ProjPlan best{true, 1};
+  double t = (double)((tb + 255) / 256) * K * 0.0267;
+  for (int ks = 1; ks <= 4 && K / 64 / ks >= 8; ++ks) {
+    const double part = ks > 1 ? 4.0 + (2.0 * ks + 1.0) * M * N * 4.0 / 5e6 : 0.0;
+    const double x = 4.0 + (double)((ts * ks + 255) / 256) * K / ks * 0.0100 + part;
+    if (x < t) best = {false, ks}, t = x;
+  }
+  if (K < 512 && 4.0 + (double)((ts + 255) / 256) * K * 0.0100 < t) best = {false, 1};
+  return best;
+}
+
+static size_t proj_r256(size_t b) { return (b + 255) & ~size_t(255); }
+
+size_t proj_gemm_prepped_ws_bytes(int M, int N, int K) {
+  const int ks = proj_plan(M, N, K).ks;
+  return proj_r256((size_t)N * K * 2) + proj_r256((size_t)N * 4) + (ks > 1 ? (size_t)ks * M * N * 4 : 0);
 }
 
 size_t proj_gemm_workspace_bytes(int M, int N, int K) {
-  auto r256 = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const int ks = proj_ksplit(M, N, K);
-  return r256((size_t)M * K * 2) + r256((size_t)M * 4) + r256((size_t)N * K * 2) + r256((size_t)N * 4) +
-         (ks > 1 ? (size_t)ks * M * N * 4 : 0);
+  return proj_r256((size_t)M * K * 2) + proj_r256((size_t)M * 4) + proj_gemm_prepped_ws_bytes(M, N, K);
 }
 
-size_t proj_gemm_prepped_ws_bytes(int M, int N, int K) {
-  auto r256 = [](size_t b) { return (b + 255) & ~size_t(255); };
-  return proj_gemm_workspace_bytes(M, N, K) - r256((size_t)M * K * 2) - r256((size_t)M * 4);
-}
-
-hipError_t launch_proj_gemm_prepped(const _Float16 *a16, const int *ea, int fmt, const void *w, float *c, int M,
-                                    int N, int K, void *ws, hipStream_t s) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % kFK != 0) return hipErrorInvalidValue;  // K moves in stages of 64
-  auto r256 = [](size_t b) { return (b + 255) & ~size_t(255); };
+// Widens W (and the am rows of a, if any) into ws, then multiplies.
+static hipError_t proj_gemm(const float *a, int am, _Float16 *a16, int *ea, int fmt, const void *w, const float *bias,
+                            float *c, int M, int N, int K, void *ws, hipStream_t s) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return hipErrorInvalidValue;  // K moves in stages of 64
   char *p = static_cast<char *>(ws);
   _Float16 *w16 = reinterpret_cast<_Float16 *>(p);
-  p += r256((size_t)N * K * 2);
+  p += proj_r256((size_t)N * K * 2);
   int *ew = reinterpret_cast<int *>(p);
-  p += r256((size_t)N * 4);
+  p += proj_r256((size_t)N * 4);
   const uint8_t *wb = static_cast<const uint8_t *>(w);
+  const dim3 grid((unsigned)((am + N + 3) / 4)), block(256);
   switch (fmt) {
     case RT_LINEAR_Q6K:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_Q6K>, dim3(N), dim3(256), 0, s, wb, N, K, w16, ew);
+      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_Q6K>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
       break;
     case RT_LINEAR_Q8_0:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_Q8_0>, dim3(N), dim3(256), 0, s, wb, N, K, w16, ew);
+      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_Q8_0>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
       break;
     case RT_LINEAR_BF16:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_BF16>, dim3(N), dim3(256), 0, s, wb, N, K, w16, ew);
+      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_BF16>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
       break;
     case RT_LINEAR_F32:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_F32>, dim3(N), dim3(256), 0, s, wb, N, K, w16, ew);
+      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_F32>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
       break;
     default: return hipErrorInvalidValue;
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int tiles_m = (M + kFTile - 1) / kFTile, tiles_n = (N + kFTile - 1) / kFTile;
-  const int ks = proj_ksplit(M, N, K);
-  float *out = ks > 1 ? reinterpret_cast<float *>(p) : c;
-  hipLaunchKernelGGL(k_gemm_f16_t256, dim3(tiles_m * tiles_n, ks), dim3(256), 0, s, a16, ea, w16, ew, out, M, N, K,
-                     tiles_m, tiles_n, ks);
+  const ProjPlan plan = proj_plan(M, N, K);
+  float *out = plan.ks > 1 ? reinterpret_cast<float *>(p) : c;
+  const float *b = plan.ks > 1 ? nullptr : bias;
+  if (plan.big) {
+    const int tm = (M + 255) / 256, tn = (N + 255) / 256;
+    hipLaunchKernelGGL(k_gemm_f16_t256, dim3(tm * tn), dim3(512), 0, s, a16, ea, w16, ew, b, out, M, N, K, tm, tn);
+  } else {
+    const int tm = (M + 127) / 128, tn = (N + 127) / 128;
+    hipLaunchKernelGGL(k_gemm_f16_t128, dim3(tm * tn, plan.ks), dim3(512), 0, s, a16, ea, w16, ew, b, out, M, N, K, tm,
+                       tn, plan.ks);
+  }
   e = hipGetLastError();
-  if (e == hipSuccess && ks > 1) e = launch_gemm_splitk_sum(out, c, (size_t)M * N, ks, s);
-  return e;
+  if (e != hipSuccess || plan.ks == 1) return e;
+  e = launch_gemm_splitk_sum(out, c, (size_t)M * N, plan.ks, s);
+  return e == hipSuccess && bias ? launch_add_bias_rows(c, bias, M, N, s) : e;
 }
 
-hipError_t launch_proj_gemm(const float *a, int fmt, const void *w, float *c, int M, int N, int K, void *ws,
-                            hipStream_t s) {
-  auto r256 = [](size_t b) { return (b + 255) & ~size_t(255); };
+hipError_t launch_proj_gemm_prepped(const _Float16 *a16, const int *ea, int fmt, const void *w, float *c, int M,
+                                    int N, int K, void *ws, hipStream_t s) {
+  return proj_gemm(nullptr, 0, const_cast<_Float16 *>(a16), const_cast<int *>(ea), fmt, w, nullptr, c, M, N, K, ws, s);
+}
+
+hipError_t launch_proj_gemm(const float *a, int fmt, const void *w, const float *bias, float *c, int M, int N, int K,
+                            void *ws, hipStream_t s) {
   char *p = static_cast<char *>(ws);
   _Float16 *a16 = reinterpret_cast<_Float16 *>(p);
-  int *ea = reinterpret_cast<int *>(p + r256((size_t)M * K * 2));
-  hipError_t e = launch_gemm_prep_a(a, M, K, a16, ea, s);
-  if (e != hipSuccess) return e;
-  return launch_proj_gemm_prepped(a16, ea, fmt, w, c, M, N, K, p + r256((size_t)M * K * 2) + r256((size_t)M * 4), s);
+  int *ea = reinterpret_cast<int *>(p + proj_r256((size_t)M * K * 2));
+  return proj_gemm(a, M, a16, ea, fmt, w, bias, c, M, N, K, p + proj_r256((size_t)M * K * 2) + proj_r256((size_t)M * 4), s);
 }
 
 }  // namespace rt

@@ -54,8 +54,8 @@ hipError_t launch_bf16_gemv_rows(const uint16_t *w, const float *a, const float 
 hipError_t launch_gelu_tanh(const float *x, float *y, size_t n, hipStream_t s);
 // c[m][n] += bias[n]
 hipError_t launch_add_bias_rows(float *c, const float *bias, int M, int N, hipStream_t s);
-hipError_t launch_proj_gemm(const float *a, int fmt, const void *w, float *c, int M, int N, int K, void *ws,
-                            hipStream_t s);
+hipError_t launch_proj_gemm(const float *a, int fmt, const void *w, const float *bias, float *c, int M, int N, int K,
+                            void *ws, hipStream_t s);
 // The same two GEMMs on an A prepared once (launch_gemm_prep_a) for several
 // matrices; ws needs the respective workspace bytes minus the A part
 // (M*K*2 and M*4 bytes, each rounded up to 256).
