@@ -173,11 +173,16 @@ rt_status q4k_gemm_entry(const char *who, const void *a, bool a_bf16, const void
   if (!aligned16(a) || !aligned16(w)) return set_error(RT_EINVAL, "%s: a and w must be 16-byte aligned", who);
   if ((reinterpret_cast<uintptr_t>(c) & 3u) != 0) return set_error(RT_EINVAL, "%s: c must be 4-byte aligned", who);
   const bool rows = rows_gemm_ok(RT_LINEAR_Q4K, (int)m, (int)n, (int)k);
+  const bool widen = !rows && q4k_gemm_widen((int)m, (int)n, (int)k);
   void *ws = nullptr;
-  rt_status st = gemm_workspace(rows ? rows_gemm_workspace_bytes(RT_LINEAR_Q4K, (int)m, (int)n, (int)k)
-                                     : q4k_gemm_workspace_bytes((int)m, (int)n, (int)k),
+  rt_status st = gemm_workspace(rows    ? rows_gemm_workspace_bytes(RT_LINEAR_Q4K, (int)m, (int)n, (int)k)
+                                : widen ? proj_gemm_workspace_bytes((int)m, (int)n, (int)k)
+                                        : q4k_gemm_workspace_bytes((int)m, (int)n, (int)k),
                                 (hipStream_t)stream, &ws);
   if (st != RT_OK) return st;
+  if (widen)
+    return hip_error(launch_proj_gemm(a, a_bf16, RT_LINEAR_Q4K, w, bias, c, (int)m, (int)n, (int)k, ws,
+                                      (hipStream_t)stream), who);
   if (rows)
     return hip_error(launch_rows_gemm(RT_LINEAR_Q4K, a, a_bf16, w, bias, c, (int)m, (int)n, (int)k, ws,
                                       (hipStream_t)stream), who);
@@ -241,7 +246,7 @@ static rt_status linear_forward(const char *who, int32_t fmt, const void *w, con
   if (st != RT_OK) return st;
   if (rows)
     return hip_error(launch_rows_gemm(fmt, a, false, w, bias, c, (int)m, (int)n, (int)k, ws, s), who);
-  return hip_error(launch_proj_gemm(a, fmt, w, bias, c, (int)m, (int)n, (int)k, ws, s), who);
+  return hip_error(launch_proj_gemm(a, false, fmt, w, bias, c, (int)m, (int)n, (int)k, ws, s), who);
 }
 
 rt_status rt_linear_gemm_f32(int32_t fmt, const void *w, const float *a, float *c, int64_t m, int64_t n, int64_t k,

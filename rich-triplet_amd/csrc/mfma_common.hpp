@@ -99,7 +99,8 @@ RT_DEV void store_c_tile(const floatx16 (&acc)[4][NT], float *stage, float *c, i
       if (row < M) {
         float *dst = c + (size_t)row * N + col;
         if (vec && col + 4 <= N) {
-          *reinterpret_cast<float4 *>(dst) = v;
+          typedef float v4f __attribute__((ext_vector_type(4)));
+          __builtin_nontemporal_store((v4f){v.x, v.y, v.z, v.w}, reinterpret_cast<v4f *>(dst));
         } else {
           if (col < N) dst[0] = v.x;
           if (col + 1 < N) dst[1] = v.y;

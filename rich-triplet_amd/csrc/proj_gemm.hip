@@ -42,6 +42,17 @@ RT_DEV void proj_load8(const uint8_t *__restrict__ W, int N, int K, int n, int p
     const uint32_t u[2] = {q.x, q.y};
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = d * (float)(int8_t)(u[i >> 2] >> (8 * (i & 3)));
+  } else if constexpr (FMT == RT_LINEAR_Q4K) {
+    const uint8_t *blk = W + ((size_t)n * (K / 256) + (p >> 5)) * kQ4KBlockBytes;
+    const int c = (p >> 3) & 3, h = (p >> 2) & 1;  // chunk, its low or high nibbles
+    const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
+    const uint2 q = *reinterpret_cast<const uint2 *>(blk + 16 + 32 * c + 8 * (p & 3));
+    uint32_t sv, mv;
+    q4k_scale_min(hd.y, hd.z, hd.w, 2 * c + h, sv, mv);
+    const float s = half_bits_to_f32(hd.x & 0xFFFFu) * (float)sv, m = half_bits_to_f32(hd.x >> 16) * (float)mv;
+    const uint32_t u[2] = {(q.x >> (4 * h)) & 0x0F0F0F0Fu, (q.y >> (4 * h)) & 0x0F0F0F0Fu};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = s * (float)((u[i >> 2] >> (8 * (i & 3))) & 0xFu) - m;
   } else {  // RT_LINEAR_Q6K, planar: piece p is l = 8 (p & 3) .. of quarter m of half j (see q6k_value)
     const Q6KPlanes P = q6k_planes(W, (size_t)N * (K / 256));
     const size_t blk = (size_t)n * (K / 256) + (p >> 5);
@@ -98,17 +109,17 @@ RT_DEV void row_to_f16(const uint8_t *__restrict__ W, int N, int K, int n, _Floa
   }
 }
 
-// Rows [0, M) are A's (f32), the rest W's.  Bound by memory: 16-byte pieces,
+// Rows [0, M) are A's (AFMT: f32 or bf16), the rest W's.  Bound by memory: 16-byte pieces,
 // four rows per workgroup.  Element by element with one row per workgroup and
 // a second read of every value the same widening took (W alone) 14.3 us for
 // BF16 3072x3072 and 15.3 us for Q8_0 6912x1152.
-template <int FMT>
-__global__ __launch_bounds__(256) void k_rows_to_f16(const float *__restrict__ a, int M, _Float16 *__restrict__ a16,
+template <int FMT, int AFMT>
+__global__ __launch_bounds__(256) void k_rows_to_f16(const void *__restrict__ a, int M, _Float16 *__restrict__ a16,
                                                      int *__restrict__ ea, const uint8_t *__restrict__ W, int N, int K,
                                                      _Float16 *__restrict__ w16, int *__restrict__ ew) {
   const int r = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (r < M)
-    row_to_f16<RT_LINEAR_F32>(reinterpret_cast<const uint8_t *>(a), M, K, r, a16, ea);
+    row_to_f16<AFMT>(static_cast<const uint8_t *>(a), M, K, r, a16, ea);
   else if (r - M < N)
     row_to_f16<FMT>(W, N, K, r - M, w16, ew);
 }
@@ -545,22 +556,24 @@ hipError_t launch_add_bias_rows(float *c, const float *bias, int M, int N, hipSt
 // adds the sum kernel and (2 ks + 1) M N words at 5 TB/s.  1000x3072x3072: 192
 // small tiles in one round 33 against 65; 2000x12000x3072: 376 large tiles 159
 // against 196; 512x2560x10240: 80 small tiles split three ways 41, whole 79.
+// The plan is the same for every M of a 128-row step.
 struct ProjPlan {
   bool big;
   int ks;
+  double est_us;
 };
 static ProjPlan proj_plan(int M, int N, int K) {
   const long tb = (long)((M + 255) / 256) * ((N + 255) / 256), ts = (long)((M + 127) / 128) * ((N + 127) / 128);
-  ProjPlan best{true, 1};
-  double t = (double)((tb + 255) / 256) * K * 0.0267;
-  for (int ks = 1; ks <= 4 && K / 64 / ks >= 8; ++ks) {
-    const double part = ks > 1 ? 4.0 + (2.0 * ks + 1.0) * M * N * 4.0 / 5e6 : 0.0;
+  ProjPlan best{true, 1, (double)((tb + 255) / 256) * K * 0.0267};
+  for (int ks = 1; ks <= 4 && (ks == 1 || K / 64 / ks >= 8); ++ks) {
+    const double part = ks > 1 ? 4.0 + (2.0 * ks + 1.0) * ((M + 127) / 128 * 128.0) * N * 4.0 / 5e6 : 0.0;
     const double x = 4.0 + (double)((ts * ks + 255) / 256) * K / ks * 0.0100 + part;
-    if (x < t) best = {false, ks}, t = x;
+    if (x < best.est_us) best = {false, ks, x};
   }
-  if (K < 512 && 4.0 + (double)((ts + 255) / 256) * K * 0.0100 < t) best = {false, 1};
   return best;
 }
+
+double proj_gemm_est_us(int M, int N, int K) { return proj_plan(M, N, K).est_us; }
 
 static size_t proj_r256(size_t b) { return (b + 255) & ~size_t(255); }
 
@@ -574,7 +587,7 @@ size_t proj_gemm_workspace_bytes(int M, int N, int K) {
 }
 
 // Widens W (and the am rows of a, if any) into ws, then multiplies.
-static hipError_t proj_gemm(const float *a, int am, _Float16 *a16, int *ea, int fmt, const void *w, const float *bias,
+static hipError_t proj_gemm(const void *a, bool a_bf16, int am, _Float16 *a16, int *ea, int fmt, const void *w, const float *bias,
                             float *c, int M, int N, int K, void *ws, hipStream_t s) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return hipErrorInvalidValue;  // K moves in stages of 64
   char *p = static_cast<char *>(ws);
@@ -584,21 +597,19 @@ static hipError_t proj_gemm(const float *a, int am, _Float16 *a16, int *ea, int 
   p += proj_r256((size_t)N * 4);
   const uint8_t *wb = static_cast<const uint8_t *>(w);
   const dim3 grid((unsigned)((am + N + 3) / 4)), block(256);
+#define RT_WIDEN(F, A) hipLaunchKernelGGL((k_rows_to_f16<F, A>), grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew)
   switch (fmt) {
-    case RT_LINEAR_Q6K:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_Q6K>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
+    case RT_LINEAR_Q4K:
+      if (a_bf16) RT_WIDEN(RT_LINEAR_Q4K, RT_LINEAR_BF16);
+      else RT_WIDEN(RT_LINEAR_Q4K, RT_LINEAR_F32);
       break;
-    case RT_LINEAR_Q8_0:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_Q8_0>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
-      break;
-    case RT_LINEAR_BF16:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_BF16>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
-      break;
-    case RT_LINEAR_F32:
-      hipLaunchKernelGGL(k_rows_to_f16<RT_LINEAR_F32>, grid, block, 0, s, a, am, a16, ea, wb, N, K, w16, ew);
-      break;
+    case RT_LINEAR_Q6K: RT_WIDEN(RT_LINEAR_Q6K, RT_LINEAR_F32); break;
+    case RT_LINEAR_Q8_0: RT_WIDEN(RT_LINEAR_Q8_0, RT_LINEAR_F32); break;
+    case RT_LINEAR_BF16: RT_WIDEN(RT_LINEAR_BF16, RT_LINEAR_F32); break;
+    case RT_LINEAR_F32: RT_WIDEN(RT_LINEAR_F32, RT_LINEAR_F32); break;
     default: return hipErrorInvalidValue;
   }
+#undef RT_WIDEN
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const ProjPlan plan = proj_plan(M, N, K);
@@ -620,15 +631,15 @@ static hipError_t proj_gemm(const float *a, int am, _Float16 *a16, int *ea, int 
 
 hipError_t launch_proj_gemm_prepped(const _Float16 *a16, const int *ea, int fmt, const void *w, float *c, int M,
                                     int N, int K, void *ws, hipStream_t s) {
-  return proj_gemm(nullptr, 0, const_cast<_Float16 *>(a16), const_cast<int *>(ea), fmt, w, nullptr, c, M, N, K, ws, s);
+  return proj_gemm(nullptr, false, 0, const_cast<_Float16 *>(a16), const_cast<int *>(ea), fmt, w, nullptr, c, M, N, K, ws, s);
 }
 
-hipError_t launch_proj_gemm(const float *a, int fmt, const void *w, const float *bias, float *c, int M, int N, int K,
+hipError_t launch_proj_gemm(const void *a, bool a_bf16, int fmt, const void *w, const float *bias, float *c, int M, int N, int K,
                             void *ws, hipStream_t s) {
   char *p = static_cast<char *>(ws);
   _Float16 *a16 = reinterpret_cast<_Float16 *>(p);
   int *ea = reinterpret_cast<int *>(p + proj_r256((size_t)M * K * 2));
-  return proj_gemm(a, M, a16, ea, fmt, w, bias, c, M, N, K, p + proj_r256((size_t)M * K * 2) + proj_r256((size_t)M * 4), s);
+  return proj_gemm(a, a_bf16, M, a16, ea, fmt, w, bias, c, M, N, K, p + proj_r256((size_t)M * K * 2) + proj_r256((size_t)M * 4), s);
 }
 
 }  // namespace rt

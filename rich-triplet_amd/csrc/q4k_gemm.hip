@@ -55,9 +55,6 @@ RT_DEV void load8<float>(const float *p, float v[8]) {
   v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
 }
 
-RT_DEV uint32_t half_bits(_Float16 h) { return (uint32_t)__builtin_bit_cast(uint16_t, h); }
-
-
 // Row exponent of W row n (one wave, one block header per lane: a strided
 // walk by a single thread is latency-bound at K = 12288).
 RT_DEV void prep_w_row(const uint8_t *__restrict__ w, int *__restrict__ ew, int n, int K, int lane) {
@@ -76,34 +73,46 @@ template <typename TA>
 __global__ __launch_bounds__(256) void k_gemm_prep(const TA *__restrict__ a, _Float16 *__restrict__ a16,
                                                    int *__restrict__ ea, const uint8_t *__restrict__ w,
                                                    int *__restrict__ ew, int M, int N, int K) {
+  constexpr int KEEP = 6;  // pieces of a row kept in registers between its maximum and its conversion
   __shared__ float red[4];
   const int b = (int)blockIdx.x;
   if (b < M) {
     const TA *row = a + (size_t)b * K;
-    float amax = 0.f;
-    for (int g = threadIdx.x; g < K / 8; g += 256) {
-      float v[8];
-      load8<TA>(row + g * 8, v);
+    const int np = K / 8, tid = (int)threadIdx.x;
+    float v[KEEP][8], amax = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    for (int i = 0; i < KEEP; ++i) {
+      if (256 * i >= np) break;  // uniform
+      load8<TA>(row + 8 * min(tid + 256 * i, np - 1), v[i]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[i][k]));
+    }
+    for (int g = tid + 256 * KEEP; g < np; g += 256) {
+      float t[8];
+      load8<TA>(row + g * 8, t);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(t[k]));
     }
     amax = wave_max(amax);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     // A NaN anywhere makes the row NaN in the product too; keep it visible.
     const int e = f16_exponent_for(amax);
-    if (threadIdx.x == 0) ea[b] = e;
-    _Float16 *out = a16 + (size_t)b * K;
-    for (int g = threadIdx.x; g < K / 8; g += 256) {
-      float v[8];
-      load8<TA>(row + g * 8, v);
-      uint32_t ow[4];
+    if (tid == 0) ea[b] = e;
+    uint4 *out = reinterpret_cast<uint4 *>(a16 + (size_t)b * K);
+    auto store = [&](int g, const float (&x)[8]) {
+      const uint2 lo = f16x4_scaled(make_float4(x[0], x[1], x[2], x[3]), e);
+      const uint2 hi = f16x4_scaled(make_float4(x[4], x[5], x[6], x[7]), e);
+      out[g] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    };
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        ow[i] = half_bits((_Float16)__builtin_amdgcn_ldexpf(v[2 * i], -e)) |
-                (half_bits((_Float16)__builtin_amdgcn_ldexpf(v[2 * i + 1], -e)) << 16);
-      *reinterpret_cast<uint4 *>(out + g * 8) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+    for (int i = 0; i < KEEP; ++i)
+      if (tid + 256 * i < np) store(tid + 256 * i, v[i]);
+    for (int g = tid + 256 * KEEP; g < np; g += 256) {
+      float t[8];
+      load8<TA>(row + g * 8, t);
+      store(g, t);
     }
   } else {
     // one wave per W row
@@ -332,61 +341,6 @@ __global__ __launch_bounds__(512) void k_q4k_gemm_w8b(const _Float16 *__restrict
 // ---------------------------------------------------------------------------
 constexpr int kHSlotA = 128 * 128;       // bytes
 
-// The GELU epilogue: each staged value is gelu_tanh(g) * u of the wave's gate
-// (acc[i][0]) and up (acc[i][1]) accumulators, each scaled by
-// 2^(ea[row] + ew of its matrix) as store_c_tile scales them, and h goes out
-// as the next GEMM's A operand: f16 scaled by 2^-eh[row] with eh[row] =
-// f16_exponent_for(2 * a_nrm2[row] * gu_bound).  By Cauchy-Schwarz
-// |g| <= |a| |w_gate|, |u| <= |a| |w_up| and |gelu_tanh(g)| <= |g|, so
-// |h| <= |a|^2 max_n |w_gate,n| |w_up,n|: a_nrm2 = |a|^2 of the row of A (f32,
-// before its f16 rounding) and gu_bound that maximum; the factor 2 covers
-// the f16 operands and the f32 sums.  No value overflows, and f16 rounding is
-// relative, so h rounds as with the exponent of its exact row maximum except
-// for elements below 2^-14 of the scale.
-RT_DEV void store_gelu_tile(const floatx16 (&acc)[4][2], float *stage, _Float16 *h16, int *eh, int M, int N,
-                            int row0, int col0, const int *ea, const int (&ecol)[2], const float *a_nrm2,
-                            float gu_bound) {
-  constexpr int P = 40, F4 = 8, RPI = 8;
-  const int lane = (int)(threadIdx.x & 63), g = lane >> 5, l32 = lane & 31;
-  const bool vec = (N & 3) == 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int er[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) er[r] = ea[min(row0 + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), M - 1)];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float gv = __builtin_amdgcn_ldexpf(acc[i][0][r], er[r] + ecol[0]);
-      const float uv = __builtin_amdgcn_ldexpf(acc[i][1][r], er[r] + ecol[1]);
-      stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + l32] = mul_nc(gelu_tanh(gv), uv);
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int q = 0; q < 32 / RPI; ++q) {
-      const int rl = q * RPI + lane / F4, f = lane % F4;
-      const int row = row0 + 32 * i + rl, col = col0 + 4 * f;
-      const float4 v = *reinterpret_cast<const float4 *>(stage + rl * P + 4 * f);
-      if (row < M) {
-        const int e = f16_exponent_for(2.0f * a_nrm2[row] * gu_bound);
-        if (col == 0) eh[row] = e;
-        _Float16 *dst = h16 + (size_t)row * N + col;
-        if (vec && col + 4 <= N) {
-          *reinterpret_cast<uint2 *>(dst) = f16x4_scaled(v, e);
-        } else {
-          const float x[4] = {v.x, v.y, v.z, v.w};
-          for (int k = 0; k < 4; ++k)
-            if (col + k < N) dst[k] = (_Float16)__builtin_amdgcn_ldexpf(x[k], -e);
-        }
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-}
-
 // |W row n|_2 of a Q4_K weight [N][K] over its dequantised values (one wave
 // per row, f32 sums): the GELU GEMM's bound on |h| is built from them.
 __global__ __launch_bounds__(256) void k_q4k_row_norms(const uint8_t *__restrict__ w, float *__restrict__ nrm, int N,
@@ -422,27 +376,6 @@ __global__ __launch_bounds__(256) void k_gemm_prep_w_multi(HMats mats, int K) {
   while (i + 1 < mats.count && r >= mats.n[i]) r -= mats.n[i++];  // wave-uniform
   if (r < mats.n[i]) prep_w_row(mats.w[i], const_cast<int *>(mats.ew[i]), r, K, threadIdx.x & 63);
 }
-
-// GELU mode's output: h16 [M][N] f16 and its row exponents eh [M]; a_nrm2 and
-// gu_bound as store_gelu_tile uses them.
-struct GeluOut {
-  _Float16 *h16;
-  int *eh;
-  const float *a_nrm2;
-  float gu_bound;
-};
-
-// QKV mode: the per-head RMSNorm (gamma g_q for matrix 0, g_k for matrix 1)
-// and NeoX RoPE of row m with cos | sin at cs + m*cs_stride (+ head_dim),
-// applied before the store; matrix 2 (v) is stored as computed.
-struct QkRope {
-  const float *cs;
-  int cs_stride;
-  const float *g_q, *g_k;
-  float eps;
-};
-
-enum HMode { kHPlain = 0, kHGelu = 1, kHQkv = 2 };
 
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void k_q4k_gemm_h(const _Float16 *__restrict__ a16, const int *__restrict__ ea,
@@ -633,89 +566,10 @@ __global__ __launch_bounds__(256, 2) void k_q4k_gemm_h(const _Float16 *__restric
     store_gelu_tile(acc, reinterpret_cast<float *>(sbase), go.h16, go.eh, M, N, m0, n0 + 32 * wave, ea, ecol,
                     go.a_nrm2, go.gu_bound);
   } else if constexpr (QKV) {
-    // The tile is one head (256 columns) of 128 rows; lane (g, l32) of wave w
-    // holds columns c = 32w + l32 (j = 0) and c + 128 (j = 1), the RoPE pair.
-    // One 32-row MFMA tile (i) at a time, so its accumulators are free once
-    // it is stored.
-    float *stage = reinterpret_cast<float *>(sbase);
     // each wave's sums of squares of the tile's rows: the last 2 KB of slot 3
     // (the staging slices use the first 9 KB of each slot)
-    float(*wsum)[128] = reinterpret_cast<float(*)[128]>(sa3 + kHSlotA - 2048);
-    const int colp[2] = {n0 + 32 * wave, n0 + 128 + 32 * wave};
-    const int cl = 32 * wave + l32;  // the pair's column within the head
-    const float *gam = mi == 0 ? qr.g_q : qr.g_k;
-    const float g0 = mi < 2 ? 1.0f + gam[cl] : 0.f, g1 = mi < 2 ? 1.0f + gam[cl + 128] : 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_barrier(0);
-      floatx16 v0, v1;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int er = ea[min(m0 + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), M - 1)];
-        v0[r] = __builtin_amdgcn_ldexpf(acc[i][0][r], er + ecol[0]);
-        v1[r] = __builtin_amdgcn_ldexpf(acc[i][1][r], er + ecol[1]);
-      }
-      if (mi < 2) {  // workgroup-uniform
-        // sums of squares of the 32 rows: this wave's 64 columns through its
-        // LDS slot ([row][l32], 16-byte groups swizzled by the row), two
-        // lanes per row, then the four waves' sums through wsum
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int R = 8 * (r >> 2) + 4 * g + (r & 3);
-          stage[R * 32 + ((((l32 >> 2) ^ R) & 7) << 2) + (l32 & 3)] = v0[r] * v0[r] + v1[r] * v1[r];
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        {
-          const int R = lane >> 1;
-          float t = 0.f;
-#pragma unroll
-          for (int m4 = 4 * (lane & 1); m4 < 4 * (lane & 1) + 4; ++m4) {
-            const float4 x = *reinterpret_cast<const float4 *>(stage + R * 32 + (((m4 ^ R) & 7) << 2));
-            t += (x.x + x.y) + (x.z + x.w);
-          }
-          t += __shfl_xor(t, 1);
-          if ((lane & 1) == 0) wsum[wave][32 * i + R] = t;
-        }
-        wg_barrier();
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-#pragma clang fp contract(off)
-          const int R = 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
-          const float ss = (wsum[0][R] + wsum[1][R]) + (wsum[2][R] + wsum[3][R]);
-          const float rinv = rms_inv_from_sumsq(ss, 1.0f / 256.0f, qr.eps);
-          const int co = min(m0 + R, M - 1) * qr.cs_stride + cl;  // 32-bit offset from the uniform base
-          const float cv = qr.cs[co], sv = qr.cs[co + 128];
-          const float a0 = (v0[r] * rinv) * g0, a1 = (v1[r] * rinv) * g1;
-          v0[r] = a0 * cv - a1 * sv;
-          v1[r] = a0 * sv + a1 * cv;
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
-      // stage and store the tile's 32 rows x (32 + 32) columns
-      constexpr int P = 72;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + l32] = v0[r];
-        stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + 32 + l32] = v1[r];
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int rl = q * 4 + lane / 16, f = lane % 16;
-        const int row = m0 + 32 * i + rl, cc = colp[f >> 3] + 4 * (f & 7);
-        const float4 x = *reinterpret_cast<const float4 *>(stage + rl * P + 4 * f);
-        if (row < M) *reinterpret_cast<float4 *>(c + (size_t)row * N + cc) = x;
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
+    store_qkv_tile(acc, reinterpret_cast<float *>(sbase), reinterpret_cast<float(*)[128]>(sa3 + kHSlotA - 2048), wave, c,
+                   M, N, m0, n0, mi, ea, ecol, qr);
   } else {
     store_c_tile<2>(acc, reinterpret_cast<float *>(sbase), c, M, N, m0, n0 + 64 * wave, ea, ecol);
   }
@@ -744,64 +598,74 @@ __global__ __launch_bounds__(256) void k_gemm_splitk_sum(const float *__restrict
 }
 
 // Which matrix-core kernel takes an M x N output, and how many ways K is
-// split (blockIdx.y; a split of ks writes ks partial products of M x N).
-// Tiles are 128 x 256 (th) for the eight-wave and half-block kernels and
-// 256 x 256 (tw) for the wide one.
-//   w8b:   up to 1024 rows and th < 512; the eight-wave kernel, one
-//          workgroup per CU, fills the chip better with few tiles
-//          (512x10240, 160 tiles: 54.9 us against 61.6 us for the
-//          half-block kernel).  K splits into enough workgroups to cover the
-//          256 CUs (a prefill's down projection, M=512 N=2560: 40 tiles),
-//          keeping at least 16 chunks (K=1024) per split.
-//   wide:  a single matrix of more than 1024 rows with 128 < tw <= 256: one
-//          round of one workgroup per CU, where the half-block kernel runs
-//          two on most CUs.  4608x3072x12288 (216 tiles): 349 us against
-//          377 us; 4096x2560x10240 split 3 ways: 230 against 235 us.
-//   half:  the rest (and every set of matrices sharing A); two workgroups per
-//          CU.  4608x12288x3072 (864 wide tiles, 3.4 rounds): 375 us against
-//          425 us for the wide kernel, whose last round runs 96 workgroups
-//          on 256 CUs; with tw <= 128 its 128-row tiles, one workgroup per
-//          CU, spread the work over twice as many CUs.
-// Above 1024 rows K takes the split that minimises a time model fitted to
-// MI355X measurements:
-//   rounds/ks of c us per K element, plus (2*ks+1)*M*N*4 bytes of partial
-//   tiles at 5 TB/s;
-//   wide:  rounds = ceil(tw*ks/256), c = 0.036;
-//   half:  rounds = ceil(th*ks/512), x0.75 when at most 256 workgroups run
-//          (one per CU), c = 0.032.
-// 4096x2560 outputs (160 wide tiles) split K=10240 three ways: 2 rounds of a
-// third instead of 1 round of the whole K on 160 of the 256 CUs.
-enum class GemmKind { w8b, half, wide };
+// split (blockIdx.y; a split of ks writes ks partial products of M x N), by a
+// time model fitted to measurements (us; k = K / ks, per round of workgroups):
+//   w8b:   128 x 256 tiles, one workgroup per CU, up to 1024 rows and 512 tiles:
+//          0.0185 k, plus 3 (512x10240x2560 50).  K splits into enough
+//          workgroups to cover the 256 CUs, at least 16 chunks (K = 1024) each.
+//   half:  128 x 256 tiles, two workgroups per CU: 4 + 0.032 k, three quarters of
+//          that 0.032 when at most 256 workgroups run.
+//   pp:    256 x 256 tiles, one per CU, so nothing runs beside its stores:
+//          17.4 + 0.0229 k with every CU busy, 10 + 0.0199 k with up to 160 (the
+//          card's power goes to fewer CUs), plus 2.  4608x12288x3072: 351 in
+//          four rounds against 385 for half, 1000x10240x2560 61 against 100,
+//          4096x2560x10240 214 whole against 256; but 4257x5324x768 72 against
+//          58 for half.
+// Splits add the sum kernel and (2 ks + 1) M N words at 5 TB/s.  The plan is the
+// same for every M of a 128-row step (prefill_gemm_workspace_bytes).  A set of
+// matrices sharing A (q|k|v, gate|up) runs on half or pp, whole.
+enum class GemmKind { w8b, half, pp };
 struct GemmPlan {
   GemmKind kind;
   int ks;
 };
-static GemmKind gemm_kind(int M, int tiles_n, bool single) {
-  const int th = ((M + 127) / 128) * tiles_n, tw = ((M + 255) / 256) * tiles_n;
-  if (single && M > 1024 && tw > 128 && tw <= 256) return GemmKind::wide;
-  return M > 1024 || th >= 512 ? GemmKind::half : GemmKind::w8b;
+static double gemm_est_us(GemmKind kind, int M, int tiles_n, int K, int ks) {
+  const int th = (M + 127) / 128 * tiles_n, tp = (M + 255) / 256 * tiles_n, wgs = (kind == GemmKind::pp ? tp : th) * ks;
+  const double k = (double)K / ks;
+  const double part = ks > 1 ? 4.0 + (2.0 * ks + 1.0) * ((M + 127) / 128 * 128.0) * (256.0 * tiles_n) * 4.0 / 5e6 : 0.0;
+  if (kind == GemmKind::w8b) return 3.0 + (wgs + 255) / 256 * k * 0.0185 + part;
+  if (kind == GemmKind::half) return (wgs + 511) / 512 * (4.0 + k * 0.032 * (wgs <= 256 ? 0.75 : 1.0)) + part;
+  const double busy = std::min(1.0, std::max(0.0, (wgs - 160) / 96.0));
+  return 2.0 + (wgs + 255) / 256 * (10.0 + 7.4 * busy + k * (0.0199 + 0.0030 * busy)) + part;
+}
+// Whether a set of tiles_n column tiles runs as one launch (half or pp): above
+// 1024 rows or 512 tiles.
+static bool gemm_set(int M, int tiles_n) { return M > 1024 || (M + 127) / 128 * tiles_n >= 512; }
+// half or pp for such a set.
+static GemmKind gemm_set_kind(int M, int tiles_n, int K) {
+  return gemm_est_us(GemmKind::pp, M, tiles_n, K, 1) <= gemm_est_us(GemmKind::half, M, tiles_n, K, 1) ? GemmKind::pp
+                                                                                                     : GemmKind::half;
 }
 
-static GemmPlan gemm_plan(int M, int N, int K) {
-  const int tiles_n = (N + 255) / 256;
-  const GemmKind kind = gemm_kind(M, tiles_n, true);
-  if (kind == GemmKind::w8b) {
-    const int by_cus = 256 / (((M + 127) / 128) * tiles_n), by_k = (K / kBK) / 16;
-    return {kind, max(1, min(by_cus, by_k))};
-  }
-  if (M <= 1024) return {kind, 1};
-  const bool wide = kind == GemmKind::wide;
-  const int ntiles = wide ? ((M + 255) / 256) * tiles_n : ((M + 127) / 128) * tiles_n;
-  auto est_us = [&](int ks) {
-    const int wgs = ntiles * ks;
-    const double rounds = wide ? (double)((wgs + 255) / 256) : (double)((wgs + 511) / 512) * (wgs <= 256 ? 0.75 : 1.0);
-    const double partial = ks > 1 ? (2.0 * ks + 1.0) * M * N * 4.0 / 5e6 : 0.0;
-    return rounds / ks * K * (wide ? 0.036 : 0.032) + partial;
+static GemmPlan gemm_plan(int M, int N, int K, double *est = nullptr) {
+  const int tiles_n = (N + 255) / 256, th = (M + 127) / 128 * tiles_n;
+  GemmPlan best{GemmKind::half, 1};
+  double t = gemm_est_us(best.kind, M, tiles_n, K, 1);
+  auto offer = [&](GemmKind kind, int ks) {
+    const double x = gemm_est_us(kind, M, tiles_n, K, ks);
+    if (x < t) best = {kind, ks}, t = x;
   };
-  int best = 1;
-  for (int ks = 2; ks <= 4 && ks <= K / 256; ++ks)
-    if (est_us(ks) < est_us(best)) best = ks;
-  return {kind, best};
+  if (!gemm_set(M, tiles_n)) {
+    const int ks = std::max(1, std::min(256 / th, (K / kBK) / 16));
+    best = {GemmKind::w8b, ks};
+    t = gemm_est_us(best.kind, M, tiles_n, K, ks);
+  }
+  for (int ks = 1; ks <= 4 && (ks == 1 || ks <= K / 512); ++ks) {
+    offer(GemmKind::pp, ks);
+    if (M > 1024) offer(GemmKind::half, ks);
+  }
+  if (est) *est = t;
+  return best;
+}
+
+// Narrow outputs of many rows have few tiles for these kernels: where the
+// weight widened to f16 once (N K words written and read, 4 TB/s) and the
+// smaller tiles of proj_gemm.hip come out a tenth ahead, they take the
+// product.  1400x259x3584: 28 us against 40.
+bool q4k_gemm_widen(int M, int N, int K) {
+  double t = 0.0;
+  (void)gemm_plan(M, N, K, &t);
+  return proj_gemm_est_us(M, N, K) + (double)N * K * 2.0 / 4e6 < 0.9 * t;
 }
 
 hipError_t launch_gemm_splitk_sum(const float *part, float *c, size_t mn, int ksplit, hipStream_t s) {
@@ -832,8 +696,9 @@ static hipError_t q4k_gemm_core(const _Float16 *a16, const int *ea, const uint8_
   const int ks = plan.ks;
   float *out = ks > 1 ? part : c;
   hipError_t e = hipSuccess;
-  if (kind == GemmKind::wide) {
-    e = launch_q4k_gemm_wide(a16, ea, HMats{{wb}, {ew}, {out}, {N}, {0}, 1}, M, K, tiles_n, ks, s);
+  if (kind == GemmKind::pp) {
+    e = launch_q4k_gemm_pp(kHPlain, a16, ea, HMats{{wb}, {ew}, {out}, {N}, {0}, 1}, M, K, tiles_n, ks, GeluOut{}, QkRope{},
+                           s);
   } else {
     if (kind == GemmKind::w8b)
       hipLaunchKernelGGL(k_q4k_gemm_w8b<1>, dim3(tiles_m * tiles_n, ks), dim3(512), 0, s, a16, ea, wb, ew, out, M,
@@ -904,7 +769,7 @@ bool q4k_gemm_multi_ok(int M, int count, const int *n) {
   if (count < 1 || count > 3) return false;
   int tiles_n = 0;
   for (int i = 0; i < count; ++i) tiles_n += (n[i] + 255) / 256;
-  return gemm_kind(M, tiles_n, false) == GemmKind::half;
+  return gemm_set(M, tiles_n);
 }
 
 bool q4k_gemm_gelu_ok(int M, int N) {
@@ -925,6 +790,8 @@ hipError_t launch_q4k_gemm_gelu_prepped(const _Float16 *a16, const int *ea, cons
   mats.n[0] = mats.n[1] = N;
   mats.count = 2;
   const int tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
+  if (gemm_set_kind(M, tiles_n, K) == GemmKind::pp)
+    return launch_q4k_gemm_pp(kHGelu, a16, ea, mats, M, K, tiles_n, 1, GeluOut{h16, eh, a_nrm2, gu_bound}, QkRope{}, s);
   hipLaunchKernelGGL(k_q4k_gemm_h<kHGelu>, dim3(tiles_m * tiles_n), dim3(256), 0, s, a16, ea, mats, M, K, tiles_m,
                      tiles_n, 1, GeluOut{h16, eh, a_nrm2, gu_bound});
   return hipGetLastError();
@@ -955,6 +822,8 @@ hipError_t launch_q4k_gemm_qkv_prepped(const _Float16 *a16, const int *ea, const
   }
   mats.count = 3;
   const int tiles_m = (M + 127) / 128;
+  if (gemm_set_kind(M, tiles_n, K) == GemmKind::pp)
+    return launch_q4k_gemm_pp(kHQkv, a16, ea, mats, M, K, tiles_n, 1, GeluOut{}, QkRope{cs, cs_stride, g_q, g_k, eps}, s);
   hipLaunchKernelGGL(k_q4k_gemm_h<kHQkv>, dim3(tiles_m * tiles_n), dim3(256), 0, s, a16, ea, mats, M, K, tiles_m,
                      tiles_n, 1, GeluOut{}, QkRope{cs, cs_stride, g_q, g_k, eps});
   return hipGetLastError();
@@ -992,6 +861,8 @@ hipError_t launch_q4k_gemm_multi_prepped(const _Float16 *a16, const int *ea, int
     if (e != hipSuccess) return e;
   }
   const int tiles_m = (M + 127) / 128;
+  if (gemm_set_kind(M, tiles_n, K) == GemmKind::pp)
+    return launch_q4k_gemm_pp(kHPlain, a16, ea, mats, M, K, tiles_n, 1, GeluOut{}, QkRope{}, s);
   hipLaunchKernelGGL(k_q4k_gemm_h<kHPlain>, dim3(tiles_m * tiles_n), dim3(256), 0, s, a16, ea, mats, M, K, tiles_m, tiles_n,
                      1);
   return hipGetLastError();

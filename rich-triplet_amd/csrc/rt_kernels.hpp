@@ -39,8 +39,8 @@ bool rows_gemm_ok(int fmt, int M, int N, int K);
 size_t rows_gemm_workspace_bytes(int fmt, int M, int N, int K);
 hipError_t launch_rows_gemm(int fmt, const void *a, bool a_bf16, const void *w, const float *bias, float *c, int M,
                             int N, int K, void *ws, hipStream_t s);
-// C[M,N] = A[M,K] . W[N,K]^T for a projection stored as RT_LINEAR_Q6K, _Q8_0
-// or _BF16 (planar layouts of kquant.hip): its rows are widened to f16 with a
+// C[M,N] = A[M,K] . W[N,K]^T (+ bias) for a weight in any RT_LINEAR_* format
+// (planar layouts of kquant.hip; a bf16 A with Q4_K only): its rows are widened to f16 with a
 // per-row power-of-two scale and multiplied on the matrix cores in f32.
 size_t proj_gemm_workspace_bytes(int M, int N, int K);
 // c[m][n] = a[m][k] . W[n][k] (+ bias[n]) on f32 weights, rows of A in groups
@@ -54,8 +54,8 @@ hipError_t launch_bf16_gemv_rows(const uint16_t *w, const float *a, const float 
 hipError_t launch_gelu_tanh(const float *x, float *y, size_t n, hipStream_t s);
 // c[m][n] += bias[n]
 hipError_t launch_add_bias_rows(float *c, const float *bias, int M, int N, hipStream_t s);
-hipError_t launch_proj_gemm(const float *a, int fmt, const void *w, const float *bias, float *c, int M, int N, int K,
-                            void *ws, hipStream_t s);
+hipError_t launch_proj_gemm(const void *a, bool a_bf16, int fmt, const void *w, const float *bias, float *c, int M,
+                            int N, int K, void *ws, hipStream_t s);
 // The same two GEMMs on an A prepared once (launch_gemm_prep_a) for several
 // matrices; ws needs the respective workspace bytes minus the A part
 // (M*K*2 and M*4 bytes, each rounded up to 256).
@@ -113,6 +113,10 @@ size_t proj_gemm_prepped_ws_bytes(int M, int N, int K);
 // Q4_K GEMM C[M,N] = A[M,K] . W[N,K]^T; A bf16 bits (a_bf16) or f32; ws holds
 // q4k_gemm_workspace_bytes(M, N, K) bytes of device scratch.
 size_t q4k_gemm_workspace_bytes(int M, int N, int K);
+// Whether a Q4_K product runs faster on launch_proj_gemm (RT_LINEAR_Q4K) than
+// on launch_q4k_gemm, from the two time models.
+bool q4k_gemm_widen(int M, int N, int K);
+double proj_gemm_est_us(int M, int N, int K);
 hipError_t launch_q4k_gemm(const void *a, bool a_bf16, const void *w, float *c, int M, int N, int K, void *ws,
                            hipStream_t s);
 
