@@ -756,15 +756,25 @@ size_t prefill_gemm_workspace_bytes(const DecodeShape &s, int cap) {
   const int kmax = std::max({H, QD, F});
   auto r256 = [](size_t v) { return (v + 255) & ~size_t(255); };
   // A chunk may hold fewer rows than cap, and a smaller M may split K more
-  // ways: take the largest requirement over every row count up to cap.
+  // ways: take the largest requirement over every row count up to cap (the
+  // few-row kernel's plan changes at multiples of 32 rows, up to 1024 of them,
+  // the tiled kernels' at multiples of 128).
   size_t m = 0;
-  for (int rows = 1; rows <= cap; ++rows)
+  for (int r0 = 0, step = 32; r0 < cap; r0 += step)
     for (auto &st : sets) {
+      step = r0 < 1024 ? 32 : 128;
+      const int rows = std::min(r0 + step, cap);
       const int K = st[0];
-      size_t b = r256((size_t)rows * kmax * 2) + r256((size_t)rows * 4);
-      for (int i = 1; i < 4 && st[i]; ++i)
-        b += std::max(q4k_gemm_prepped_ws_bytes(rows, st[i], K), proj_gemm_prepped_ws_bytes(rows, st[i], K));
-      m = std::max(m, b);
+      size_t b = r256((size_t)rows * kmax * 2) + r256((size_t)rows * 4), few = b + rows_pack_bytes(rows, K);
+      for (int i = 1; i < 4 && st[i]; ++i) {
+        const size_t tiled = std::max(q4k_gemm_prepped_ws_bytes(rows, st[i], K), proj_gemm_prepped_ws_bytes(rows, st[i], K));
+        b += tiled;
+        size_t r = tiled;  // a matrix of a set that the few-row kernel does not take
+        for (int f : {RT_LINEAR_Q4K, RT_LINEAR_Q6K, RT_LINEAR_Q8_0})
+          if (rows_gemm_ok(f, r0 + 1, st[i], K)) r = std::max(r, rows_part_bytes(f, rows, st[i], K));  // any row count of the step
+        few += r;
+      }
+      m = std::max({m, b, few});
     }
   return m;
 }
@@ -887,12 +897,26 @@ hipError_t enqueue_rows(const DecodeShape &s, const DecodeArgs &a, const LayerAr
       return launch_q4k_gemm_multi_prepped(a16, ea, i, w, c, nn, ew, n, K, st, ews.begin());
     }
     // each matrix in its own region; a split Q4_K GEMM leaves its partials
-    // there and the consumer adds them while reading (views)
+    // there and the consumer adds them while reading (views).  Few rows go
+    // through the kernel that streams the packed weight once (rows_gemm.hip),
+    // on the rows packed once for the set.
     int i = 0;
+    const void *frag = nullptr;
     for (const MbMat &m : mats) {
       const int fmt = fmts.begin()[i];
       RowsIn &v = *views.begin()[i++];
-      if (fmt == RT_LINEAR_Q4K) {
+      if (rows_gemm_ok(fmt, n, m.n, K)) {
+        if (!frag) {
+          frag = rest;
+          rest += rows_pack_bytes(n, K);
+          r = launch_rows_pack(a16, n, K, const_cast<void *>(frag), st);
+          if (r != hipSuccess) return r;
+        }
+        GemmLeft left{};
+        r = launch_rows_gemm_packed(fmt, frag, ea, m.w, m.y, n, m.n, K, reinterpret_cast<float *>(rest), st, &left);
+        v = left.ks > 1 ? RowsIn{left.part, left.ks, (size_t)n * m.n, m.n, 0} : rows_plain(m.y, m.n);
+        rest += rows_part_bytes(fmt, n, m.n, K);
+      } else if (fmt == RT_LINEAR_Q4K) {
         GemmLeft left{};
         r = launch_q4k_gemm_prepped(a16, ea, m.w, m.y, n, m.n, K, rest, st, &left, ews.begin()[i - 1]);
         v = left.ks > 1 ? RowsIn{left.part, left.ks, (size_t)n * m.n, m.n, 0} : rows_plain(m.y, m.n);

@@ -99,6 +99,16 @@ __global__ __launch_bounds__(kRowsPrepT) void k_rows_prep(const TA *__restrict__
   }
 }
 
+// The same order from rows already in f16 (row-major, prepared with their
+// exponents by the kernel that produced them).
+__global__ __launch_bounds__(256) void k_rows_pack(const uint4 *__restrict__ a16, uint4 *__restrict__ frag, int M, int K,
+                                                   int tiles) {
+  const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, np = K / 8;  // piece i % np of row i / np
+  if (i >= M * np) return;
+  const int m = i / np, s = i - m * np, c = s >> 3, q = s & 7, g = (q >> 1) & 1, t = (q & 1) + 2 * (q >> 2);
+  frag[(size_t)((c * tiles + (m >> 5)) * 4 + t) * 64 + 32 * g + (m & 31)] = a16[i];
+}
+
 // Eight f16 weights s*(1024 + u) + negc of eight code bytes u (two words), as
 // dq_step (q4k_gemm_dev.hpp) forms them, one rounding each.
 RT_DEV half8 rows_dq(uint32_t a, uint32_t b, float s, float negc) {
@@ -549,21 +559,10 @@ size_t rows_gemm_workspace_bytes(int fmt, int M, int N, int K) {
   return r256((size_t)(K / 64) * p.tiles * 4096) + r256((size_t)M * 4) + (p.ks > 1 ? (size_t)p.ks * M * N * 4 : 0);
 }
 
-hipError_t launch_rows_gemm(int fmt, const void *a, bool a_bf16, const void *w, const float *bias, float *c, int M,
-                            int N, int K, void *ws, hipStream_t s) {
-  const RowsPlanG p = rows_plan(fmt, M, N, K);
-  uint8_t *frag = static_cast<uint8_t *>(ws);
-  int *ea = reinterpret_cast<int *>(frag + r256((size_t)(K / 64) * p.tiles * 4096));
-  float *part = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(ea) + r256((size_t)M * 4));
+// The product of packed rows; partial products (ks > 1) go to part.
+static hipError_t rows_core(int fmt, const RowsPlanG &p, const uint8_t *frag, const int *ea, const void *w,
+                            const float *bias, float *c, float *part, int M, int N, int K, hipStream_t s) {
   const uint8_t *wb = static_cast<const uint8_t *>(w);
-  if (a_bf16)
-    hipLaunchKernelGGL(k_rows_prep<uint16_t>, dim3(M), dim3(kRowsPrepT), 0, s, static_cast<const uint16_t *>(a), frag,
-                       ea, K, p.tiles);
-  else
-    hipLaunchKernelGGL(k_rows_prep<float>, dim3(M), dim3(kRowsPrepT), 0, s, static_cast<const float *>(a), frag, ea, K,
-                       p.tiles);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   float *out = p.ks > 1 ? part : c;
   const float *b = p.ks > 1 ? nullptr : bias;
   const dim3 grid((unsigned)((N + 32 * p.nt - 1) / (32 * p.nt)), (unsigned)p.ks, (unsigned)((p.tiles + p.mt - 1) / p.mt));
@@ -584,10 +583,46 @@ hipError_t launch_rows_gemm(int fmt, const void *a, bool a_bf16, const void *w, 
     RT_ROWS(RT_LINEAR_Q6K, 4)
 #undef RT_ROWS
   }
-  e = hipGetLastError();
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_gemm(int fmt, const void *a, bool a_bf16, const void *w, const float *bias, float *c, int M,
+                            int N, int K, void *ws, hipStream_t s) {
+  const RowsPlanG p = rows_plan(fmt, M, N, K);
+  uint8_t *frag = static_cast<uint8_t *>(ws);
+  int *ea = reinterpret_cast<int *>(frag + r256((size_t)(K / 64) * p.tiles * 4096));
+  float *part = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(ea) + r256((size_t)M * 4));
+  if (a_bf16)
+    hipLaunchKernelGGL(k_rows_prep<uint16_t>, dim3(M), dim3(kRowsPrepT), 0, s, static_cast<const uint16_t *>(a), frag,
+                       ea, K, p.tiles);
+  else
+    hipLaunchKernelGGL(k_rows_prep<float>, dim3(M), dim3(kRowsPrepT), 0, s, static_cast<const float *>(a), frag, ea, K,
+                       p.tiles);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = rows_core(fmt, p, frag, ea, w, bias, c, part, M, N, K, s);
   if (e != hipSuccess || p.ks == 1) return e;
   e = launch_gemm_splitk_sum(part, c, (size_t)M * N, p.ks, s);
   return e == hipSuccess && bias ? launch_add_bias_rows(c, bias, M, N, s) : e;
+}
+
+size_t rows_pack_bytes(int M, int K) { return r256((size_t)(K / 64) * ((M + 31) / 32) * 4096); }
+
+size_t rows_part_bytes(int fmt, int M, int N, int K) {
+  const int ks = rows_plan(fmt, M, N, K).ks;
+  return ks > 1 ? r256((size_t)ks * M * N * 4) : 0;
+}
+
+hipError_t launch_rows_pack(const _Float16 *a16, int M, int K, void *frag, hipStream_t s) {
+  hipLaunchKernelGGL(k_rows_pack, dim3((unsigned)(((size_t)M * (K / 8) + 255) / 256)), dim3(256), 0, s,
+                     reinterpret_cast<const uint4 *>(a16), static_cast<uint4 *>(frag), M, K, (M + 31) / 32);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_gemm_packed(int fmt, const void *frag, const int *ea, const void *w, float *c, int M, int N,
+                                   int K, float *part, hipStream_t s, GemmLeft *left) {
+  const RowsPlanG p = rows_plan(fmt, M, N, K);
+  *left = GemmLeft{p.ks > 1 ? part : c, p.ks};
+  return rows_core(fmt, p, static_cast<const uint8_t *>(frag), ea, w, nullptr, c, part, M, N, K, s);
 }
 
 }  // namespace rt

@@ -68,6 +68,14 @@ struct GemmLeft {
   const float *part;
   int ks;
 };
+// The few-row GEMM on rows already prepared (a16, ea): launch_rows_pack once into
+// rows_pack_bytes, then each matrix of the set; a product that splits K
+// leaves its partials in part (rows_part_bytes) for the consumer.
+size_t rows_pack_bytes(int M, int K);
+size_t rows_part_bytes(int fmt, int M, int N, int K);
+hipError_t launch_rows_pack(const _Float16 *a16, int M, int K, void *frag, hipStream_t s);
+hipError_t launch_rows_gemm_packed(int fmt, const void *frag, const int *ea, const void *w, float *c, int M, int N,
+                                   int K, float *part, hipStream_t s, GemmLeft *left);
 // ew_pre: the weight's row exponents from launch_q4k_row_exponents, kept
 // with the weight (null: computed into ws by this call).
 hipError_t launch_q4k_gemm_prepped(const _Float16 *a16, const int *ea, const void *w, float *c, int M, int N, int K,
