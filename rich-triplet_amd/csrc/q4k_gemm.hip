@@ -603,14 +603,16 @@ __global__ __launch_bounds__(256) void k_gemm_splitk_sum(const float *__restrict
 //   w8b:   128 x 256 tiles, one workgroup per CU, up to 1024 rows and 512 tiles:
 //          0.0185 k, plus 3 (512x10240x2560 50).  K splits into enough
 //          workgroups to cover the 256 CUs, at least 16 chunks (K = 1024) each.
-//   half:  128 x 256 tiles, two workgroups per CU: 4 + 0.032 k, three quarters of
-//          that 0.032 when at most 256 workgroups run.
+//   half:  128 x 256 tiles, two workgroups per CU: 0.035 k per full round of 512,
+//          less in a round that fills less of the chip (the card's power goes
+//          to fewer CUs): 0.019 k + 0.016 k (w / 512) of w > 256 workgroups,
+//          0.0185 k of up to 256 (0.015 k as the tail of full rounds).
 //   pp:    256 x 256 tiles, one per CU, so nothing runs beside its stores:
-//          17.4 + 0.0229 k with every CU busy, 10 + 0.0199 k with up to 160 (the
-//          card's power goes to fewer CUs), plus 2.  4608x12288x3072: 351 in
-//          four rounds against 385 for half, 1000x10240x2560 61 against 100,
-//          4096x2560x10240 214 whole against 256; but 4257x5324x768 72 against
-//          58 for half.
+//          17.4 + 0.026 k with every CU busy, 10 + 0.019 k with up to 160, plus 2.
+//   pp / half: 4608x12288x3072 351 / 385, 1000x10240x2560 61 / 100, 2023x5080x4096
+//   104 / 134, 4096x2560x10240 214 / 256 (split); where 256 half workgroups
+//   cover C, 1148x5129x3072 82 / 69; 2119x8399x1024 100 / 84.  Over 90 random
+//   products of 1025 to 2600 rows the choice costs 0.3% against the better of the two.
 // Splits add the sum kernel and (2 ks + 1) M N words at 5 TB/s.  The plan is the
 // same for every M of a 128-row step (prefill_gemm_workspace_bytes).  A set of
 // matrices sharing A (q|k|v, gate|up) runs on half or pp, whole.
@@ -624,9 +626,18 @@ static double gemm_est_us(GemmKind kind, int M, int tiles_n, int K, int ks) {
   const double k = (double)K / ks;
   const double part = ks > 1 ? 4.0 + (2.0 * ks + 1.0) * ((M + 127) / 128 * 128.0) * (256.0 * tiles_n) * 4.0 / 5e6 : 0.0;
   if (kind == GemmKind::w8b) return 3.0 + (wgs + 255) / 256 * k * 0.0185 + part;
-  if (kind == GemmKind::half) return (wgs + 511) / 512 * (4.0 + k * 0.032 * (wgs <= 256 ? 0.75 : 1.0)) + part;
-  const double busy = std::min(1.0, std::max(0.0, (wgs - 160) / 96.0));
-  return 2.0 + (wgs + 255) / 256 * (10.0 + 7.4 * busy + k * (0.0199 + 0.0030 * busy)) + part;
+  double t = part;
+  if (kind == GemmKind::half) {
+    const int full = wgs / 512, rem = wgs % 512;
+    t += 4.0 + full * k * 0.035 + (full || rem > 256 ? 6.0 : 0.0);
+    return t + (rem > 256 ? k * (0.019 + 0.016 * rem / 512) : rem ? k * (full ? 0.015 : 0.0185) : 0.0);
+  }
+  t += 2.0;
+  for (int w = wgs; w > 0; w -= 256) {
+    const double busy = std::min(1.0, std::max(0.0, (std::min(w, 256) - 160) / 96.0));
+    t += 10.0 + 7.4 * busy + k * (0.019 + 0.007 * busy);
+  }
+  return t;
 }
 // Whether a set of tiles_n column tiles runs as one launch (half or pp): above
 // 1024 rows or 512 tiles.
@@ -661,11 +672,12 @@ static GemmPlan gemm_plan(int M, int N, int K, double *est = nullptr) {
 // Narrow outputs of many rows have few tiles for these kernels: where the
 // weight widened to f16 once (N K words written and read, 4 TB/s) and the
 // smaller tiles of proj_gemm.hip come out a tenth ahead, they take the
-// product.  1400x259x3584: 28 us against 40.
+// product (C costs that path 0.8 us more per million outputs).  1400x259x3584:
+// 28 us against 40, 2115x1160x2560 34 against 41, but 2367x5862x512 51 against 46.
 bool q4k_gemm_widen(int M, int N, int K) {
   double t = 0.0;
   (void)gemm_plan(M, N, K, &t);
-  return proj_gemm_est_us(M, N, K) + (double)N * K * 2.0 / 4e6 < 0.9 * t;
+  return proj_gemm_est_us(M, N, K) + (double)N * K * 2.0 / 4e6 + (double)M * N * 0.8e-6 < 0.9 * t;
 }
 
 hipError_t launch_gemm_splitk_sum(const float *part, float *c, size_t mn, int ksplit, hipStream_t s) {

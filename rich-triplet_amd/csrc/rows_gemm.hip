@@ -536,7 +536,12 @@ RowsPlanG rows_plan(int fmt, int M, int N, int K) {
   // rows (160 workgroups): ks 3 37.8, 1 44.
   const int wgs = (N + 32 * p.nt - 1) / (32 * p.nt) * ((p.tiles + p.mt - 1) / p.mt);
   const int most = q4k ? K / 256 / (2 * kRowsQ4kWaves) : K / 64 / (4 * kRowsWaves);
-  p.ks = std::max(1, std::min((q4k && wgs >= 80 ? 480 : 240) / wgs, most));
+  int ks = (q4k && wgs >= 80 ? 480 : 240) / wgs;
+  // Little more than one workgroup per CU leaves the second round nearly empty:
+  // halve it where K is long (9636x11776 of 75 rows, 302 workgroups: 71 -> 68;
+  // 4096x14336 of 300 rows, 320: 86 -> 81; from 400 workgroups on it loses)
+  if (q4k && K >= 8192 && wgs > 256 && wgs <= 400) ks = 2;
+  p.ks = std::max(1, std::min(ks, most));
   return p;
 }
 
@@ -551,6 +556,10 @@ bool rows_gemm_ok(int fmt, int M, int N, int K) {
   // 450 rows 66 / 57; Q8_0 10000x6016 384 rows 154 / 186).  Longer, where the
   // output has too few tiles to fill the chip: 2560x2560 1000 rows 38 / 41,
   // 1024x2560 1000 rows 25 / 38, 6000x2560 640 rows 48 / 47.
+  // Not on a large Q4_K weight whose rows fill 128-row tiles (an even number of
+  // 64-row pairs): 9636x11776 of 75 rows 68 / 62, of 200 rows 112 / 100, of
+  // 140 rows 80 / 97; 10240x10240 of 200 rows 97 / 90; 12000x8192 of 200 86 / 90.
+  if (fmt == RT_LINEAR_Q4K && K > 8192 && N > 4096 && ((M + 63) / 64) % 2 == 0) return false;
   return M <= 384 || (M <= 1024 && K <= 4096 && (long)M * N <= 2600000);
 }
 
