@@ -406,103 +406,83 @@ __global__ __launch_bounds__(512, 2) void k_gemm_f16_t256(const _Float16 *__rest
 }
 
 // ---------------------------------------------------------------------------
-// f32 weights with a few activation rows (QLinear's f32 branch, x.matmul_bt(W),
-// qlinear.rs:102-106, for M <= 8 per launch row group): each wave owns four
-// weight rows and streams them once for the MR activation rows of its group
-// (blockIdx.y), 16-byte loads along K; per output a lane-strided f32 sum, then
-// the wave's DPP sum.  With a bias, out = sum + bias[n], the one f32 add of
-// add_bias_rows (qlinear.rs:49-60).
+// f32 and bf16 weights with a few activation rows (QLinear's f32 branch,
+// x.matmul_bt(W), qlinear.rs:102-106, and MatBf16::matmul_by_t,
+// autograd2.rs:757-852), M <= 8 per launch row group (blockIdx.y): four weight
+// rows per group of kw = 2^lkw waves, streamed once for the MR activation rows, 16-byte
+// loads along K (bf16 widened exactly); per output a lane-strided f32 sum, the
+// wave's DPP sum, then the kw waves' sums through LDS.  With a bias, out = sum +
+// bias[n], the one f32 add of add_bias_rows (qlinear.rs:49-60).
+// Bound by the latency of a wave's loads where the rows alone give few waves.
 // ---------------------------------------------------------------------------
-template <int MR>
-__global__ __launch_bounds__(256) void k_f32_gemv_rows(const float *__restrict__ W, const float *__restrict__ a,
-                                                       const float *__restrict__ bias, float *__restrict__ c, int M,
-                                                       int N, int K) {
-  constexpr int RW = 4;
-  const int lane = (int)threadIdx.x & 63;
-  const int n0 = (int)((blockIdx.x * 256u + threadIdx.x) >> 6) * RW;
+constexpr int kGemvRowsMaxLkw = 4, kGemvRowsMaxKw = 1 << kGemvRowsMaxLkw;
+template <bool BF16, int MR>
+__global__ __launch_bounds__(64 * kGemvRowsMaxKw) void k_gemv_rows(const void *__restrict__ W,
+                                                                   const float *__restrict__ a,
+                                                                   const float *__restrict__ bias,
+                                                                   float *__restrict__ c, int M, int N, int K, int lkw,
+                                                                   int lgroups) {
+  constexpr int RW = 4, V = BF16 ? 8 : 4;  // weights per 16-byte load
+  __shared__ float part[kGemvRowsMaxKw][RW * MR];
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int kw = 1 << lkw, kp = wave & (kw - 1), n0 = (((int)blockIdx.x << lgroups) + (wave >> lkw)) * RW;
   const int m0 = (int)blockIdx.y * 8;
-  if (n0 >= N) return;  // whole waves
-  const int K4 = K / 4;
-  const float4 *w4 = reinterpret_cast<const float4 *>(W);
-  const float4 *a4 = reinterpret_cast<const float4 *>(a) + (size_t)m0 * K4;
-  float acc[RW][MR];
-#pragma unroll
-  for (int r = 0; r < RW; ++r)
-#pragma unroll
-    for (int i = 0; i < MR; ++i) acc[r][i] = 0.f;
-#pragma unroll 2
-  for (int k4 = lane; k4 < K4; k4 += 64) {
-    float4 w[RW];
-#pragma unroll
-    for (int r = 0; r < RW; ++r) w[r] = w4[(size_t)min(n0 + r, N - 1) * K4 + k4];
-#pragma unroll
-    for (int i = 0; i < MR; ++i) {
-      const float4 x = a4[(size_t)min(i, M - 1 - m0) * K4 + k4];  // rows past M re-read row M-1, unstored
-#pragma unroll
-      for (int r = 0; r < RW; ++r) {
-        acc[r][i] = fmaf(w[r].x, x.x, acc[r][i]);
-        acc[r][i] = fmaf(w[r].y, x.y, acc[r][i]);
-        acc[r][i] = fmaf(w[r].z, x.z, acc[r][i]);
-        acc[r][i] = fmaf(w[r].w, x.w, acc[r][i]);
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < RW; ++r)
-#pragma unroll
-    for (int i = 0; i < MR; ++i) {
-      const float v = wave_sum(acc[r][i]);
-      if (lane == 0 && n0 + r < N && m0 + i < M) c[(size_t)(m0 + i) * N + n0 + r] = bias ? v + bias[n0 + r] : v;
-    }
-}
-
-// The same for BF16 weights (MatBf16::matmul_by_t, autograd2.rs:757-852, of a
-// few rows): 16-byte loads of eight weights, each widened exactly.
-template <int MR>
-__global__ __launch_bounds__(256) void k_bf16_gemv_rows(const uint16_t *__restrict__ W, const float *__restrict__ a,
-                                                        const float *__restrict__ bias, float *__restrict__ c, int M,
-                                                        int N, int K) {
-  constexpr int RW = 4;
-  const int lane = (int)threadIdx.x & 63;
-  const int n0 = (int)((blockIdx.x * 256u + threadIdx.x) >> 6) * RW;
-  const int m0 = (int)blockIdx.y * 8;
-  if (n0 >= N) return;
-  const int K8 = K / 8;
-  const uint4 *w8 = reinterpret_cast<const uint4 *>(W);
+  const int KV = K / V;
+  const uint4 *w = static_cast<const uint4 *>(W);
   const float4 *a4 = reinterpret_cast<const float4 *>(a) + (size_t)m0 * (K / 4);
   float acc[RW][MR];
 #pragma unroll
   for (int r = 0; r < RW; ++r)
 #pragma unroll
     for (int i = 0; i < MR; ++i) acc[r][i] = 0.f;
-#pragma unroll 2
-  for (int k8 = lane; k8 < K8; k8 += 64) {
-    float wf[RW][8];
+#pragma unroll (MR <= 2 ? 4 : 2)
+  for (int k = lane + 64 * kp; k < KV; k += 64 * kw) {
+    float wf[RW][V];
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
-      const uint4 q = w8[(size_t)min(n0 + r, N - 1) * K8 + k8];
+      const uint4 q = w[(size_t)min(n0 + r, N - 1) * KV + k];  // rows past N re-read row N-1, unstored
       const uint32_t u[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wf[r][2 * j] = bf16_lo(u[j]), wf[r][2 * j + 1] = bf16_hi(u[j]);
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (BF16)
+          wf[r][2 * j] = bf16_lo(u[j]), wf[r][2 * j + 1] = bf16_hi(u[j]);
+        else
+          wf[r][j] = __uint_as_float(u[j]);
+      }
     }
 #pragma unroll
     for (int i = 0; i < MR; ++i) {
-      const float4 *xr = a4 + (size_t)min(i, M - 1 - m0) * (K / 4) + 2 * k8;
-      const float4 x0 = xr[0], x1 = xr[1];
-      const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      const float4 *xr = a4 + (size_t)min(i, M - 1 - m0) * (K / 4) + (V / 4) * k;  // rows past M re-read row M-1
 #pragma unroll
-      for (int r = 0; r < RW; ++r)
+      for (int h = 0; h < V / 4; ++h) {
+        const float4 x = xr[h];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[r][i] = fmaf(wf[r][j], xv[j], acc[r][i]);
+        for (int r = 0; r < RW; ++r) {
+          acc[r][i] = fmaf(wf[r][4 * h], x.x, acc[r][i]);
+          acc[r][i] = fmaf(wf[r][4 * h + 1], x.y, acc[r][i]);
+          acc[r][i] = fmaf(wf[r][4 * h + 2], x.z, acc[r][i]);
+          acc[r][i] = fmaf(wf[r][4 * h + 3], x.w, acc[r][i]);
+        }
+      }
     }
   }
+  float v = 0.f;  // lane r MR + i keeps output (r, i)
 #pragma unroll
   for (int r = 0; r < RW; ++r)
 #pragma unroll
     for (int i = 0; i < MR; ++i) {
-      const float v = wave_sum(acc[r][i]);
-      if (lane == 0 && n0 + r < N && m0 + i < M) c[(size_t)(m0 + i) * N + n0 + r] = bias ? v + bias[n0 + r] : v;
+      const float t = wave_sum(acc[r][i]);
+      if (lane == r * MR + i) v = t;
     }
+  if (lkw) {
+    if (lane < RW * MR) part[wave][lane] = v;
+    __syncthreads();
+    if (kp == 0 && lane < RW * MR)
+      for (int p = 1; p < kw; ++p) v += part[wave + p][lane];
+  }
+  if (kp != 0 || lane >= RW * MR) return;
+  const int n = n0 + lane / MR, m = m0 + lane % MR;
+  if (n < N && m < M) c[(size_t)m * N + n] = bias ? v + bias[n] : v;
 }
 
 // add_bias_rows (qlinear.rs:49-60): c[r][j] += bias[j].
@@ -514,33 +494,42 @@ __global__ __launch_bounds__(256) void k_add_bias_rows(float *__restrict__ c, co
 
 }  // namespace
 
+template <bool BF16>
+static hipError_t gemv_rows(const void *w, const float *a, const float *bias, float *c, int M, int N, int K,
+                            hipStream_t s) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % (BF16 ? 8 : 4) != 0) return hipErrorInvalidValue;
+  const int mgroups = (M + 7) / 8, rows = (N + 3) / 4, chunks = (K / (BF16 ? 8 : 4) + 63) / 64;
+  // Waves per row group: as many as keep the launch within 8192 waves (4096 of
+  // the widest form).  bf16 2560 x 10240 of 5 rows: 1024 waves 44 us, 2048 26,
+  // 4096 18.6, 8192 16.4, 16384 24; of 8 rows 45, 27, 21.0, 24.3, 31; f32 of 8
+  // rows 78, 44, 29, 24.5, 28.
+  const int target = BF16 && M > 6 ? 4096 : 8192;
+  int lkw = 0;
+  while (lkw < kGemvRowsMaxLkw && (2 << lkw) <= chunks && (long)rows * mgroups * (2 << lkw) <= target) ++lkw;
+  const int lgroups = std::max(0, 2 - lkw), groups = 1 << lgroups;  // row groups per workgroup
+  const dim3 grid((unsigned)((rows + groups - 1) / groups), (unsigned)mgroups), block((unsigned)(64 << lkw << lgroups));
+#define RT_ROWS(MR) hipLaunchKernelGGL((k_gemv_rows<BF16, MR>), grid, block, 0, s, w, a, bias, c, M, N, K, lkw, lgroups)
+  switch (std::min(M, 8)) {  // rows of the last group are bounded by M inside
+    case 1: RT_ROWS(1); break;
+    case 2: RT_ROWS(2); break;
+    case 3: RT_ROWS(3); break;
+    case 4: RT_ROWS(4); break;
+    case 5:
+    case 6: RT_ROWS(6); break;
+    default: RT_ROWS(8); break;
+  }
+#undef RT_ROWS
+  return hipGetLastError();
+}
+
 hipError_t launch_f32_gemv_rows(const float *w, const float *a, const float *bias, float *c, int M, int N, int K,
                                 hipStream_t s) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % 4 != 0) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((M + 7) / 8));
-  const int mr = std::min(M, 8);  // rows of the last group are bounded by M inside
-  switch (mr) {
-    case 1: hipLaunchKernelGGL(k_f32_gemv_rows<1>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    case 2: hipLaunchKernelGGL(k_f32_gemv_rows<2>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    case 3: hipLaunchKernelGGL(k_f32_gemv_rows<3>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    case 4: hipLaunchKernelGGL(k_f32_gemv_rows<4>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    default: hipLaunchKernelGGL(k_f32_gemv_rows<8>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-  }
-  return hipGetLastError();
+  return gemv_rows<false>(w, a, bias, c, M, N, K, s);
 }
 
 hipError_t launch_bf16_gemv_rows(const uint16_t *w, const float *a, const float *bias, float *c, int M, int N, int K,
                                  hipStream_t s) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((M + 7) / 8));
-  switch (std::min(M, 8)) {
-    case 1: hipLaunchKernelGGL(k_bf16_gemv_rows<1>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    case 2: hipLaunchKernelGGL(k_bf16_gemv_rows<2>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    case 3: hipLaunchKernelGGL(k_bf16_gemv_rows<3>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    case 4: hipLaunchKernelGGL(k_bf16_gemv_rows<4>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-    default: hipLaunchKernelGGL(k_bf16_gemv_rows<8>, grid, dim3(256), 0, s, w, a, bias, c, M, N, K); break;
-  }
-  return hipGetLastError();
+  return gemv_rows<true>(w, a, bias, c, M, N, K, s);
 }
 
 hipError_t launch_add_bias_rows(float *c, const float *bias, int M, int N, hipStream_t s) {
