@@ -92,8 +92,9 @@ rt_status rt_weight_cache_clear(void);
  * A is bf16 bits (rt_q4k_gemm_bf16) or f32 (rt_q4k_gemm_f32), row-major
  * [m,k]; every row of A must start 16-byte aligned (k % 256 == 0 ensures it).
  * The library keeps a workspace of about m*k*2 bytes per (host thread,
- * device, stream), shared with rt_linear_gemm_f32 and rt_q4k_gemv_batch on
- * that stream.  It grows on demand, but not while the stream is being
+ * device, stream), plus split-K partials of m*n*4 bytes each where K is
+ * split and n*k*2 bytes where a narrow output runs on the weight widened to
+ * f16; shared with rt_linear_gemm_f32 and rt_q4k_gemv_batch on that stream.  It grows on demand, but not while the stream is being
  * captured: a captured call that would need more returns RT_ESTATE, so make
  * the same call once outside capture first.  Outgrown buffers stay
  * allocated (a graph captured earlier may still read them) until
@@ -190,7 +191,8 @@ rt_status rt_q8_0_gemv(const void *w, const float *x, float *y, int64_t n, int64
  * (Q8_0, and BF16 with m > 8), k % 8 == 0 (BF16, m <= 8), k % 4 == 0 (F32);
  * device pointers, a and w 16-byte aligned.  Uses the
  * per-(thread, device, stream) workspace of rt_q4k_gemm_f32, about
- * (m + n) * k * 2 bytes (none for the f32 GEMV). */
+ * (m + n) * k * 2 bytes (m * k * 2 for Q4_K, and for Q6_K and Q8_0 of up to
+ * 384 rows, which stay packed; none for the f32 GEMV), plus split-K partials. */
 rt_status rt_linear_gemm_f32(int32_t fmt, const void *w, const float *a, float *c, int64_t m, int64_t n, int64_t k,
                              void *stream);
 /* QLinear::forward (qlinear.rs:82-111): out[m][n] = x[m][k] . W[n][k], then

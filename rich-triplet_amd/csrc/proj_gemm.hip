@@ -1,15 +1,16 @@
-// proj_gemm.hip -- the GEMM of a projection that is not Q4_K (Q6_K, Q8_0,
-// BF16 kept in their device layouts, or f32), for prefill rows, and the f32
-// weight GEMV of a few rows.
+// proj_gemm.hip -- the GEMM on a weight widened to f16 (Q6_K, Q8_0, BF16 in
+// their device layouts, f32, and Q4_K of narrow outputs), for prefill rows, and
+// the f32 / bf16 weight GEMV of a few rows.
 //
 // The reference runs these weights as BF16 after widening them at load
 // (transformer4.rs:1233-1242) and multiplies on the CPU in f32
 // (MatBf16::matmul_by_t, autograd2.rs:757-852).  Here each row of W is
 // widened to f16 with a power-of-two scale 2^-ew[n] (max |w'| in
 // [2^14, 2^15), exact for BF16, Q8_0 and Q6_K codes times their f16 scales up
-// to f16 rounding), A gets the same treatment per row (k_gemm_prep), and
-// k_gemm_f16_t256 multiplies on v_mfma_f32_32x32x16_f16 with the scales
-// restored in the epilogue, as the Q4_K GEMM does.
+// to f16 rounding), A gets the same treatment per row (in the same launch, or
+// k_gemm_prep for a set), and k_gemm_f16_t128 or k_gemm_f16_t256 multiplies on
+// v_mfma_f32_32x32x16_f16 with the scales restored in the epilogue, as the
+// Q4_K GEMM does.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

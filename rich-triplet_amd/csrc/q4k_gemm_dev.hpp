@@ -1,5 +1,5 @@
 // q4k_gemm_dev.hpp -- device pieces shared by the Q4_K GEMM kernels
-// (q4k_gemm.hip, q4k_gemm_wide.hip): the K chunk, the dequantisation step
+// (q4k_gemm.hip, q4k_gemm_pp.hip): the K chunk, the dequantisation step
 // into an MFMA B operand, and the matrix set of a one-launch projection set.
 #pragma once
 
