@@ -8,20 +8,23 @@
 // consecutive pieces of a row, all ITERS rows' weights are in flight before
 // any arithmetic, and the activations are staged once per workgroup.
 //
-// Arithmetic: each 64-element activation chunk is scaled to integers
-// X = rint(x * s), s = top / 2^e with the chunk's max |x| < 2^e, written as
-// three balanced bytes X = 65536*x2 + 256*x1 + x0; Q6_K and Q8_0 keep
-// x3 = rint(254 (x*s - X)) as a fourth.  The weight codes multiply the digits
-// in exact integer dot products (v_dot4_i32_i8), so the roundings are the
-// last digit and the f32 combine per slot.  Against float64 on N(0,1) rows:
-// Q4_K 2.9e-7 to 3.2e-7 rel-L2, where f32 products and sums give 5.4e-7 to
-// 8.4e-7 (the codes' and the min's parts cancel); Q6_K 0.9e-7 to 1.1e-7
-// (f32 1.4e-7 to 2.8e-7), Q8_0 0.7e-7 to 1.0e-7 (f32 1.0e-7 to 2.3e-7; three
-// digits, 1.9e-7, would not do).  3 or 4 dot operations per 4 weights, where
-// f32 takes 4 conversions and 4 FMAs.
+// Arithmetic, Q6_K and Q8_0: each 64-element activation chunk is scaled to
+// integers X = rint(x * s), s = 2^22 / 2^e with the chunk's max |x| < 2^e,
+// written as three balanced bytes X = 65536*x2 + 256*x1 + x0 and a fourth
+// x3 = rint(254 (x*s - X)).  The weight codes multiply the digits in exact
+// integer dot products (v_dot4_i32_i8), so the roundings are the last digit and
+// the f32 combine per slot.  Against float64 on N(0,1) rows: Q6_K 0.9e-7 to
+// 1.1e-7 (f32 1.4e-7 to 2.8e-7), Q8_0 0.7e-7 to 1.0e-7 (f32 1.0e-7 to 2.3e-7).
 // A chunk that holds an infinity or a NaN has no such digits: its delta is
-// NaN, which makes a Q4_K slot NaN as its f32 form is (scale*inf - min*inf),
-// and sends a Q6_K or Q8_0 slot through f32 products, element by element.
+// NaN, which sends the slot through f32 products, element by element.
+//   Q4_K: f32 activations; per sub-block sum q x in f32 (four chains) and sum x to
+// 48 bits, combined as the reference's scale * sum q x - min * sum x
+// (autograd2.rs:1671-1698).  The two parts cancel, so their roundings make the
+// error: 2.0e-7 to 2.4e-7, where one wave per row gives 2.6e-7 to 6.9e-7.  The
+// same time as 24-bit digits (15360x3840 9.4 us, 3840x15360 11.8), which kept
+// 24 bits of a chunk's largest value only: 2.4e-7 to 3.1e-7, and nothing of a
+// value 2^24 below it.  Finite values whose 16 q x overflows (from 1.4e36 on)
+// are multiplied weight by weight.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,87 +40,86 @@
 namespace rt {
 namespace {
 
-// Stage of one chunk, in dwords: the digit planes of 16 (dword i = elements
-// 4i .. 4i+3), then delta, for Q4_K the sums of X over the chunk's two halves
-// (the min term), padding, and for Q6_K per 16-element sub-block the integer sums of
-// x0 + 256*x1 and, packed in one dword, of x2 (low half) and x3.  The pitches
-// put the 16 lanes that a 16-byte LDS read serves together on distinct banks.
+// Stage of one chunk, in dwords.  Q4_K: the 64 activations, the sums of its two
+// halves and what those sums' f32 rounding left.  Else the four digit planes of 16 (dword i = elements
+// 4i .. 4i+3), then delta, padding, and for Q6_K per 16-element sub-block the
+// integer sums of x0 + 256*x1 and, packed in one dword, of x2 (low half) and x3.
+// The pitches put the 16 lanes that a 16-byte LDS read serves together on
+// distinct banks.
 template <int FMT>
-constexpr int kAnyDigits = FMT == RT_LINEAR_Q4K ? 3 : 4;
-template <int FMT>
-constexpr int kAnyPitch = 16 * kAnyDigits<FMT> + (FMT == RT_LINEAR_Q6K ? 12 : 4);
-constexpr float kAnyTop3 = 8355711.0f;  // 127 * (65536 + 256 + 1)
-constexpr float kAnyTop4 = 4194304.0f;  // 2^22: the scaling is exact
-constexpr float kAnyUnit3 = 1.0f / 8388608.0f, kAnyUnit4 = 1.0f / 4194304.0f;
+constexpr int kAnyPitch = 64 + (FMT == RT_LINEAR_Q6K ? 12 : 4);
+constexpr float kAnyTop = 4194304.0f;  // 2^22: the scaling is exact
+constexpr float kAnyUnit = 1.0f / 4194304.0f;
+
+template <int CTRL>
+RT_DEV double dpp_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)dpp_u32<CTRL>((uint32_t)u) | (uint64_t)dpp_u32<CTRL>((uint32_t)(u >> 32)) << 32);
+}
 
 // Elements 4f .. 4f+3 of the vector (zeros past K); the 16 lanes of a chunk
 // are consecutive lanes of a wave and all call this; `store` masks the lanes
 // past the last chunk.
 template <int FMT>
 RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
-  uint32_t mb = max(max(f32_bits(v.x) & 0x7FFFFFFFu, f32_bits(v.y) & 0x7FFFFFFFu),
-                    max(f32_bits(v.z) & 0x7FFFFFFFu, f32_bits(v.w) & 0x7FFFFFFFu));
-  mb = max(mb, dpp_u32<0xB1>(mb));
-  mb = max(mb, dpp_u32<0x4E>(mb));
-  mb = max(mb, dpp_u32<0x141>(mb));
-  mb = max(mb, dpp_u32<0x140>(mb));
-  constexpr int ND = kAnyDigits<FMT>;
-  constexpr float kTop = ND == 3 ? kAnyTop3 : kAnyTop4;
-  // max < 2^e; below 2^-103 the scale stays at the largest normal one
-  const int e = max((int)(mb >> 23) - 126, -103);
-  const float s = bits_f32(f32_bits(kTop) - ((uint32_t)e << 23));
-  float delta = bits_f32(f32_bits(1.0f / (kTop * (ND == 3 ? kAnyUnit3 : kAnyUnit4))) + ((uint32_t)e << 23));
-  if (mb >= 0x7F800000u) delta = bits_f32(0x7FC00000u);
-  const float xs[4] = {v.x, v.y, v.z, v.w};
-  uint32_t b[4], r[4];  // bytes 0..2: X + 0x808080; the fourth digit + 128
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float t = __builtin_amdgcn_fmed3f(xs[i] * s, -kTop, kTop), X = __builtin_rintf(t);
-    b[i] = (uint32_t)(int)X + 0x808080u;
-    if constexpr (ND == 4) r[i] = (uint32_t)((int)__builtin_rintf((t - X) * 254.0f) + 128);
-  }
-  const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);  // b0.0 b1.0 b0.1 b1.1
-  const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
-  const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0602u);  // b0.2 b1.2 0 0
-  const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0602u);
-  uint32_t d[4];
-  d[0] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
-  d[1] = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
-  d[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u;
-  if constexpr (ND == 4) {
-    const uint32_t r01 = __builtin_amdgcn_perm(r[1], r[0], 0x0C0C0400u), r23 = __builtin_amdgcn_perm(r[3], r[2], 0x0C0C0400u);
-    d[3] = __builtin_amdgcn_perm(r23, r01, 0x05040100u) ^ 0x80808080u;
-  }
-  // Q4_K: sum of X over the 8 lanes of a half, exact (so the codes' and the
-  // min's parts see the same rounded activations)
-  int half = 0;
-  if constexpr (FMT == RT_LINEAR_Q4K) {
-    half = (int)(b[0] + b[1] + b[2] + b[3]) - 4 * 0x808080;
-    half += (int)dpp_u32<0xB1>((uint32_t)half);
-    half += (int)dpp_u32<0x4E>((uint32_t)half);
-    half += (int)dpp_u32<0x141>((uint32_t)half);
-  }
-  int s01 = 0, s23 = 0;
-  if constexpr (FMT == RT_LINEAR_Q6K) {
-    auto sum4 = [](uint32_t q) { return __builtin_amdgcn_sdot4((int)q, 0x01010101, 0, false); };
-    s01 = sum4(d[0]) + 256 * sum4(d[1]);
-    s23 = sum4(d[2]) + 65536 * sum4(d[3]);
-    s01 += (int)dpp_u32<0xB1>((uint32_t)s01);
-    s23 += (int)dpp_u32<0xB1>((uint32_t)s23);
-    s01 += (int)dpp_u32<0x4E>((uint32_t)s01);  // 4 lanes = 16 elements
-    s23 += (int)dpp_u32<0x4E>((uint32_t)s23);
-  }
-  if (!store) return;
   const int sub = f & 15;
-  uint32_t *base = dl + (f >> 4) * kAnyPitch<FMT>, *st = base + 16 * ND;
-#pragma unroll
-  for (int i = 0; i < ND; ++i) base[16 * i + sub] = d[i];
-  if (sub == 0) st[0] = f32_bits(delta);
+  uint32_t *base = dl + (f >> 4) * kAnyPitch<FMT>, *st = base + 64;
   if constexpr (FMT == RT_LINEAR_Q4K) {
-    if ((sub & 7) == 0) st[1 + (sub >> 3)] = f32_bits((float)half * kAnyUnit3);
-  }
-  if constexpr (FMT == RT_LINEAR_Q6K) {
-    if ((sub & 3) == 0) st[4 + 2 * (sub >> 2)] = (uint32_t)s01, st[5 + 2 * (sub >> 2)] = (uint32_t)s23;
+    double half = ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+    half += dpp_f64<0xB1>(half);
+    half += dpp_f64<0x4E>(half);
+    half += dpp_f64<0x141>(half);  // 8 lanes = 32 elements
+    if (!store) return;
+    reinterpret_cast<float4 *>(base)[sub] = v;
+    const float hi = (float)half;
+    if ((sub & 7) == 0) st[sub >> 3] = f32_bits(hi), st[2 + (sub >> 3)] = f32_bits((float)(half - (double)hi));
+  } else {
+    uint32_t mb = max(max(f32_bits(v.x) & 0x7FFFFFFFu, f32_bits(v.y) & 0x7FFFFFFFu),
+                      max(f32_bits(v.z) & 0x7FFFFFFFu, f32_bits(v.w) & 0x7FFFFFFFu));
+    mb = max(mb, dpp_u32<0xB1>(mb));
+    mb = max(mb, dpp_u32<0x4E>(mb));
+    mb = max(mb, dpp_u32<0x141>(mb));
+    mb = max(mb, dpp_u32<0x140>(mb));
+    // max < 2^e; below 2^-103 the scale stays at the largest normal one
+    const int e = max((int)(mb >> 23) - 126, -103);
+    const float s = bits_f32(f32_bits(kAnyTop) - ((uint32_t)e << 23));
+    float delta = bits_f32(f32_bits(1.0f) + ((uint32_t)e << 23));
+    if (mb >= 0x7F800000u) delta = bits_f32(0x7FC00000u);
+    const float xs[4] = {v.x, v.y, v.z, v.w};
+    uint32_t b[4], r[4];  // bytes 0..2: X + 0x808080; the fourth digit + 128
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float t = __builtin_amdgcn_fmed3f(xs[i] * s, -kAnyTop, kAnyTop), X = __builtin_rintf(t);
+      b[i] = (uint32_t)(int)X + 0x808080u;
+      r[i] = (uint32_t)((int)__builtin_rintf((t - X) * 254.0f) + 128);
+    }
+    const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);  // b0.0 b1.0 b0.1 b1.1
+    const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
+    const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0602u);  // b0.2 b1.2 0 0
+    const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0602u);
+    const uint32_t r01 = __builtin_amdgcn_perm(r[1], r[0], 0x0C0C0400u), r23 = __builtin_amdgcn_perm(r[3], r[2], 0x0C0C0400u);
+    uint32_t d[4];
+    d[0] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
+    d[1] = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
+    d[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u;
+    d[3] = __builtin_amdgcn_perm(r23, r01, 0x05040100u) ^ 0x80808080u;
+    int s01 = 0, s23 = 0;
+    if constexpr (FMT == RT_LINEAR_Q6K) {
+      auto sum4 = [](uint32_t q) { return __builtin_amdgcn_sdot4((int)q, 0x01010101, 0, false); };
+      s01 = sum4(d[0]) + 256 * sum4(d[1]);
+      s23 = sum4(d[2]) + 65536 * sum4(d[3]);
+      s01 += (int)dpp_u32<0xB1>((uint32_t)s01);
+      s23 += (int)dpp_u32<0xB1>((uint32_t)s23);
+      s01 += (int)dpp_u32<0x4E>((uint32_t)s01);  // 4 lanes = 16 elements
+      s23 += (int)dpp_u32<0x4E>((uint32_t)s23);
+    }
+    if (!store) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) base[16 * i + sub] = d[i];
+    if (sub == 0) st[0] = f32_bits(delta);
+    if constexpr (FMT == RT_LINEAR_Q6K) {
+      if ((sub & 3) == 0) st[4 + 2 * (sub >> 2)] = (uint32_t)s01, st[5 + 2 * (sub >> 2)] = (uint32_t)s23;
+    }
   }
 }
 
@@ -125,11 +127,8 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
 // exactly (|s0 + 256 s1| < 2^28), then one rounding per step.  The power of
 // two of `top` is taken out here, so delta (about 2^e) neither underflows
 // for small activations nor makes a product overflow before the last one.
-RT_DEV float any_dot(const int (&s)[3]) {
-  return fmaf((float)s[2], 65536.0f * kAnyUnit3, (float)(s[0] + 256 * s[1]) * kAnyUnit3);
-}
 RT_DEV float any_dot(const int (&s)[4]) {
-  return fmaf((float)s[2], 65536.0f * kAnyUnit4, fmaf((float)s[3], 1.0f / 254.0f, (float)(s[0] + 256 * s[1])) * kAnyUnit4);
+  return fmaf((float)s[2], 65536.0f * kAnyUnit, fmaf((float)s[3], 1.0f / 254.0f, (float)(s[0] + 256 * s[1])) * kAnyUnit);
 }
 
 // Weights of a thread's slot in ITERS rows, and their dot products with the
@@ -148,48 +147,80 @@ struct AnyTile<RT_LINEAR_Q4K, ITERS> {
     qb[it] = *reinterpret_cast<const uint4 *>(bp + 32 + 32 * c);
   }
   RT_DEV void compute(const uint32_t *dl, int slot, float (&p)[ITERS]) const {
-    const uint32_t m4 = opaque_u32(0x0F0F0F0Fu);
-    const uint32_t *base = dl + slot * kAnyPitch<RT_LINEAR_Q4K>;
-    int l[ITERS][3], h[ITERS][3];
+    const float *base = reinterpret_cast<const float *>(dl) + slot * kAnyPitch<RT_LINEAR_Q4K>;
+    float l[ITERS][4], h[ITERS][4];  // sums of q x of the low half, 16 q x of the high half
 #pragma unroll
     for (int it = 0; it < ITERS; ++it)
 #pragma unroll
-      for (int d = 0; d < 3; ++d) l[it][d] = h[it][d] = 0;
+      for (int k = 0; k < 4; ++k) l[it][k] = h[it][k] = 0.f;
+    const uint32_t mlo = opaque_u32(0x0F0F0F0Fu), mhi = opaque_u32(0xF0F0F0F0u);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      uint4 a[3], b[3];  // digits of low-half words 4g .. 4g+3 and of the high half's
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        a[d] = *reinterpret_cast<const uint4 *>(base + 16 * d + 4 * g);
-        b[d] = *reinterpret_cast<const uint4 *>(base + 16 * d + 8 + 4 * g);
-      }
+    for (int j = 0; j < 8; ++j) {  // word j: elements 4j .. 4j+3 of the low half and of the high half
+      const float4 a = *reinterpret_cast<const float4 *>(base + 4 * j), b = *reinterpret_cast<const float4 *>(base + 32 + 4 * j);
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
-        const uint4 q = g ? qb[it] : qa[it];
+        const uint4 q = j < 4 ? qa[it] : qb[it];
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        const uint32_t lo = w[j & 3] & mlo, hi = w[j & 3] & mhi;
+        l[it][0] = fmaf(ubyte0(lo), a.x, l[it][0]);
+        l[it][1] = fmaf(ubyte1(lo), a.y, l[it][1]);
+        l[it][2] = fmaf(ubyte2(lo), a.z, l[it][2]);
+        l[it][3] = fmaf(ubyte3(lo), a.w, l[it][3]);
+        h[it][0] = fmaf(ubyte0(hi), b.x, h[it][0]);
+        h[it][1] = fmaf(ubyte1(hi), b.y, h[it][1]);
+        h[it][2] = fmaf(ubyte2(hi), b.z, h[it][2]);
+        h[it][3] = fmaf(ubyte3(hi), b.w, h[it][3]);
+      }
+      if (ITERS == 4 && (j & 1)) {  // sums in step with the reads: all 64 activations at once would spill
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int lo = (int)(w[j] & m4), hi = (int)((w[j] >> 4) & m4);
+        for (int it = 0; it < ITERS; ++it)
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const uint32_t A[4] = {a[d].x, a[d].y, a[d].z, a[d].w}, B[4] = {b[d].x, b[d].y, b[d].z, b[d].w};
-            l[it][d] = __builtin_amdgcn_sdot4(lo, (int)A[j], l[it][d], false);
-            h[it][d] = __builtin_amdgcn_sdot4(hi, (int)B[j], h[it][d], false);
-          }
-        }
+          for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(l[it][k]), "+v"(h[it][k]));
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    const float4 st = *reinterpret_cast<const float4 *>(base + 48);  // delta, sum_lo, sum_hi
+    const float4 sum = *reinterpret_cast<const float4 *>(base + 64);
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const float d = half_bits_to_f32(hd[it].x & 0xFFFFu), dm = half_bits_to_f32(hd[it].x >> 16);
       uint32_t svp, mvp;
       q4k_scale_min_pair(hd[it].y, hd[it].z, hd[it].w, slot & 3, svp, mvp);
-      const float qsum = fmaf((float)(svp >> 8), any_dot(h[it]),
-                              (float)(svp & 0xFFu) * any_dot(l[it]));
-      const float msum = fmaf((float)(mvp >> 8), st.z, (float)(mvp & 0xFFu) * st.y);
-      p[it] = fmaf(d * st.x, qsum, -(dm * st.x * msum));
+      const float s0 = d * (float)(svp & 0xFFu), s1 = 0.0625f * d * (float)(svp >> 8);  // exact
+      const float m0 = dm * (float)(mvp & 0xFFu), m1 = dm * (float)(mvp >> 8);
+      const float lo = fmaf(s0, (l[it][0] + l[it][1]) + (l[it][2] + l[it][3]), -(m0 * sum.x));
+      const float hi = fmaf(s1, (h[it][0] + h[it][1]) + (h[it][2] + h[it][3]), -(m1 * sum.y));
+      p[it] = fmaf(-m0, sum.z, lo) + fmaf(-m1, sum.w, hi);
+      asm volatile("" : "+v"(p[it]));  // summed here: sunk into the branch that stores it, the activations stay live
     }
+  }
+  // Non-finite parts: the codes times the activations overflowed, or an
+  // activation is an infinity or a NaN, which makes the slot NaN as scale * inf
+  // - min * inf is.
+  RT_DEV static bool plain(const uint32_t *, int, const float (&p)[ITERS]) {
+    bool ok = true;
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) ok = ok && __builtin_isfinite(p[it]);
+    return ok;
+  }
+  // The slot's part p of a row weight by weight (unless the block's scales are
+  // what is not finite).
+  RT_DEV static float exact(const uint8_t *W, const float *x, int, int K, int row, int slot, float p) {
+    const uint8_t *bp = W + ((size_t)row * (K / 256) + (slot >> 2)) * kQ4KBlockBytes;
+    const uint4 hd = *reinterpret_cast<const uint4 *>(bp);
+    if ((hd.x & 0x7C00u) == 0x7C00u || (hd.x & 0x7C000000u) == 0x7C000000u) return p;
+    uint32_t svp, mvp;
+    q4k_scale_min_pair(hd.y, hd.z, hd.w, slot & 3, svp, mvp);
+    const float d = half_bits_to_f32(hd.x & 0xFFFFu), dm = half_bits_to_f32(hd.x >> 16);
+    float acc = 0.f;
+    bool finite = true;
+#pragma unroll 1
+    for (int i = 0; i < 64; ++i) {
+      const int h = i >> 5, q = (bp[16 + 32 * (slot & 3) + (i & 31)] >> (4 * h)) & 15;
+      const float v = x[64 * slot + i], w = fmaf(d * (float)((svp >> (8 * h)) & 0xFFu), (float)q, -(dm * (float)((mvp >> (8 * h)) & 0xFFu)));
+      finite = finite && __builtin_isfinite(v);
+      acc = fmaf(w, v, acc);
+    }
+    return finite ? acc : bits_f32(0x7FC00000u);
   }
 };
 
@@ -253,12 +284,12 @@ struct AnyTile<RT_LINEAR_Q6K, ITERS> {  // slot: see Q6KTile (kquant_tile.hpp)
       p[it] = fmaf(acc[it][1], d * d1, acc[it][0] * (d * d0));
     }
   }
-  RT_DEV static bool plain(const uint32_t *dl, int slot) {
+  RT_DEV static bool plain(const uint32_t *dl, int slot, const float (&)[ITERS]) {
     const uint32_t *base = dl + 2 * (slot >> 1) * kAnyPitch<RT_LINEAR_Q6K>;
     return !__builtin_isnan(bits_f32(base[64])) && !__builtin_isnan(bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]));
   }
   // The slot's part of a row in f32: 16 elements of each quarter of its half block.
-  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot) {
+  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot, float) {
     const Q6KPlanes P = q6k_planes(W, (size_t)N * (K / 256));
     float acc = 0.f;
 #pragma unroll 1
@@ -310,10 +341,10 @@ struct AnyTile<RT_LINEAR_Q8_0, ITERS> {
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) p[it] = half_bits_to_f32(dd[it]) * delta * any_dot(s[it]);
   }
-  RT_DEV static bool plain(const uint32_t *dl, int slot) {
+  RT_DEV static bool plain(const uint32_t *dl, int slot, const float (&)[ITERS]) {
     return !__builtin_isnan(bits_f32(dl[(slot >> 1) * kAnyPitch<RT_LINEAR_Q8_0> + 64]));
   }
-  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot) {
+  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot, float) {
     float acc = 0.f;
 #pragma unroll 1
     for (int i = 32 * slot; i < 32 * slot + 32; ++i)
@@ -354,12 +385,10 @@ __global__ __launch_bounds__(1024) void k_gemv_any(const uint8_t *__restrict__ W
   __syncthreads();
   float p[ITERS];
   tile.compute(dl, slot, p);
-  if constexpr (FMT != RT_LINEAR_Q4K) {
-    if (!AnyTile<FMT, ITERS>::plain(dl, slot)) {
+  if (!tile.plain(dl, slot, p)) {
 #pragma unroll
-      for (int it = 0; it < ITERS; ++it)
-        p[it] = AnyTile<FMT, ITERS>::exact(W, x, N, K, min(row0 + it * rpi + rsub, N - 1), slot);
-    }
+    for (int it = 0; it < ITERS; ++it)
+      p[it] = AnyTile<FMT, ITERS>::exact(W, x, N, K, min(row0 + it * rpi + rsub, N - 1), slot, p[it]);
   }
   if (rsub < rpi) {
 #pragma unroll
@@ -546,7 +575,8 @@ __global__ __launch_bounds__(512) void k_any_prologue(DecodeArgs a, const float 
 }  // namespace
 
 // Workgroup shape, from a sweep of 256..1024 threads and 1, 2 or 4 rows per
-// thread over 19 shapes (distinct matrices in a graph, us):
+// thread over 19 shapes (distinct matrices in a graph, us; Q4_K then on digits
+// of the same time):
 //   T: the smallest multiple of 64 from 512 (768 for K >= 8192, whose staging
 //   is longer; 320 or, below K = 2048, 192 where 512
 //   would leave CUs without a workgroup) whose

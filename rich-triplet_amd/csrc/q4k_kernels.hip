@@ -262,7 +262,7 @@ static hipError_t launch_dig(const void *W, const float *x, float *y, int N, hip
 // up to 8k rows, 48 rows (960 threads, two row-iterations) up to 12k, 32 rows
 // beyond; K=2048 with 16 rows; K=10240 with 12 rows (960 threads).  K of 1, 2,
 // 4 or 16 super-blocks use the f32-staged tile (1024x4096 3.2 us against 3.7
-// for gemv_any.hip, and half its error); any other K up to 16384 gemv_any.hip.
+// for gemv_any.hip); any other K up to 16384 gemv_any.hip.
 template <int NB, int T, int ITERS>
 static hipError_t launch_dig_multi(const void *const *w, float *const *y, const int *n, int count, const float *x,
                                    hipStream_t s) {

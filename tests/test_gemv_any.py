@@ -80,3 +80,64 @@ def test_gemv_any_keeps_non_finite_values(rt, orc, dev, fmt, k):
         x[77] = 0.5
         xs = (x * np.float32(big)).astype(np.float32)
         assert rel_l2(gemv(rt, dev, fmt, w, xs, n, k), w64 @ xs.astype(np.float64)) < 2e-6
+
+
+def q4k_parts(w, n, k):
+    """float64 scale * code and min of every weight, [n, k] each: the two sums of
+    the reference's integer trick (autograd2.rs:1671-1698)."""
+    b = w.reshape(n, k // 256, 144)
+    d = b[:, :, 0:2].copy().view(np.float16)[..., 0].astype(np.float64)
+    dm = b[:, :, 2:4].copy().view(np.float16)[..., 0].astype(np.float64)
+    sc, qs = b[:, :, 4:16].astype(np.int64), b[:, :, 16:].reshape(n, -1, 4, 32)
+    sv = np.concatenate([sc[..., 0:4] & 63, (sc[..., 8:12] & 15) | (sc[..., 0:4] >> 6) << 4], -1)
+    mv = np.concatenate([sc[..., 4:8] & 63, (sc[..., 8:12] >> 4) | (sc[..., 4:8] >> 6) << 4], -1)
+    q = np.stack([qs & 15, qs >> 4], 3).reshape(n, -1, 8, 32).astype(np.float64)
+    s, m = (d[..., None] * sv)[..., None], (dm[..., None] * mv)[..., None]
+    return (q * s).reshape(n, k), np.broadcast_to(m, q.shape).reshape(n, k)
+
+
+def q4k_bound(w, x, n, k):
+    """What f32 products and sums may differ by: the longest chain of roundings
+    from a product to the result (8 of a quarter sub-block, 2 + 2 + 1 to the
+    slot, k / 1024 + 4 over the slots, sum x and the last store), 2^-24 each, of
+    the sum of the magnitudes that meet in it."""
+    sq, m = q4k_parts(w, n, k)
+    return (8 + 5 + -(-k // 1024) + 4 + 2) * 2.0 ** -24 * ((np.abs(sq) + np.abs(m)) @ np.abs(x.astype(np.float64)))
+
+
+@pytest.mark.parametrize("n,k", [(70, 768), (600, 3840), (4000, 1280)])
+def test_gemv_any_q4k_keeps_small_activations(rt, orc, dev, n, k):
+    """A channel 2^20 times the others, its weights and its sub-blocks' mins zero:
+    the rest of its 64 activations keep all their bits."""
+    big = 200  # super-block 0, chunk 3, sub-block 6
+    w = orc.synth_q4k(9, n, k).reshape(n, k // 256, 144).copy()
+    w[:, 0, 16 + 32 * 3 + big - 192] &= 0xF0  # code of the channel
+    w[:, 0, 12 + 2] &= 0x0F  # the min of sub-block 6: low bits ...
+    w[:, 0, 8 + 2] &= 0x3F   # ... and high bits
+    w = w.reshape(-1)
+    w64 = orc.q4k_dequant(w, n, k).reshape(n, k).astype(np.float64)
+    assert np.all(w64[:, big] == 0.0)
+    x = np.random.default_rng(k).normal(size=k).astype(np.float32)
+    x[big] = 2.0 ** 20
+    got = gemv(rt, dev, Q4K, w, x, n, k)
+    rest = x.copy()
+    rest[big] = 0.0
+    assert np.all(np.abs(got - w64 @ x.astype(np.float64)) <= q4k_bound(w, rest, n, k))
+
+
+def test_gemv_any_q4k_top_of_the_range(rt, orc, dev):
+    """Activations whose products with the codes overflow, and the weight's own
+    products do not: finite, and as exact."""
+    n, k = 333, 1280
+    w = orc.synth_q4k(11, n, k).reshape(-1, 144).copy()
+    w[:, 0:4] = (w[:, 0:4].copy().view(np.float16) / np.float16(256)).view(np.uint8)
+    w = w.reshape(-1)
+    w64 = orc.q4k_dequant(w, n, k).reshape(n, k).astype(np.float64)
+    assert np.abs(w64).max() < 0.9
+    x = np.random.default_rng(2).normal(size=k).astype(np.float32)
+    for at in ([77], [500, 501, 1270]):
+        for big in (2e36, 3.3e38):
+            y = x.copy()
+            y[at] = np.float32(big) / len(at)
+            got = gemv(rt, dev, Q4K, w, y, n, k)
+            assert np.all(np.abs(got - w64 @ y.astype(np.float64)) <= q4k_bound(w, y, n, k))
