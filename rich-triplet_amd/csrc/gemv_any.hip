@@ -49,7 +49,7 @@ namespace {
 template <int FMT>
 constexpr int kAnyPitch = 64 + (FMT == RT_LINEAR_Q6K ? 12 : 4);
 constexpr float kAnyTop = 4194304.0f;  // 2^22: the scaling is exact
-constexpr float kAnyUnit = 1.0f / 4194304.0f;
+constexpr float kAnyUnit = 65536.0f / 4194304.0f;  // delta is 2^(e - 16): finite up to the largest x
 
 template <int CTRL>
 RT_DEV double dpp_f64(double v) {
@@ -83,7 +83,7 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
     // max < 2^e; below 2^-103 the scale stays at the largest normal one
     const int e = max((int)(mb >> 23) - 126, -103);
     const float s = bits_f32(f32_bits(kAnyTop) - ((uint32_t)e << 23));
-    float delta = bits_f32(f32_bits(1.0f) + ((uint32_t)e << 23));
+    float delta = bits_f32(f32_bits(1.0f / 65536.0f) + ((uint32_t)e << 23));
     if (mb >= 0x7F800000u) delta = bits_f32(0x7FC00000u);
     const float xs[4] = {v.x, v.y, v.z, v.w};
     uint32_t b[4], r[4];  // bytes 0..2: X + 0x808080; the fourth digit + 128
@@ -124,9 +124,9 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
 }
 
 // sum_k c_k x_k / delta from a group's digit sums: the middle digits combine
-// exactly (|s0 + 256 s1| < 2^28), then one rounding per step.  The power of
-// two of `top` is taken out here, so delta (about 2^e) neither underflows
-// for small activations nor makes a product overflow before the last one.
+// exactly (|s0 + 256 s1| < 2^28), then one rounding per step.  Below 2^34 with
+// Q6_K's scales, so the block's f16 scale multiplies it safely; the product with
+// delta, the last one, is the slot's value.
 RT_DEV float any_dot(const int (&s)[4]) {
   return fmaf((float)s[2], 65536.0f * kAnyUnit, fmaf((float)s[3], 1.0f / 254.0f, (float)(s[0] + 256 * s[1])) * kAnyUnit);
 }
@@ -281,7 +281,7 @@ struct AnyTile<RT_LINEAR_Q6K, ITERS> {  // slot: see Q6KTile (kquant_tile.hpp)
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const float d = half_bits_to_f32(dd[it]);
-      p[it] = fmaf(acc[it][1], d * d1, acc[it][0] * (d * d0));
+      p[it] = fmaf(acc[it][1] * d, d1, acc[it][0] * d * d0);
     }
   }
   RT_DEV static bool plain(const uint32_t *dl, int slot, const float (&)[ITERS]) {
@@ -339,7 +339,7 @@ struct AnyTile<RT_LINEAR_Q8_0, ITERS> {
     }
     const float delta = bits_f32(base[64]);
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) p[it] = half_bits_to_f32(dd[it]) * delta * any_dot(s[it]);
+    for (int it = 0; it < ITERS; ++it) p[it] = half_bits_to_f32(dd[it]) * any_dot(s[it]) * delta;
   }
   RT_DEV static bool plain(const uint32_t *dl, int slot, const float (&)[ITERS]) {
     return !__builtin_isnan(bits_f32(dl[(slot >> 1) * kAnyPitch<RT_LINEAR_Q8_0> + 64]));

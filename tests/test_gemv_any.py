@@ -141,3 +141,28 @@ def test_gemv_any_q4k_top_of_the_range(rt, orc, dev):
             y[at] = np.float32(big) / len(at)
             got = gemv(rt, dev, Q4K, w, y, n, k)
             assert np.all(np.abs(got - w64 @ y.astype(np.float64)) <= q4k_bound(w, y, n, k))
+
+
+@pytest.mark.parametrize("fmt,n,k", [(Q6K, 333, 1280), (Q8_0, 333, 1120)])
+def test_gemv_any_top_of_the_range(rt, orc, dev, fmt, n, k):
+    """Finite activations up to the largest float, products within range: the
+    digits' scale stays finite."""
+    if fmt == Q6K:
+        b, at, scale = synth_q6k(np.random.default_rng(12), n * k // 256).reshape(-1, 210), 208, 2.0 ** -9
+    else:
+        b, at, scale = synth_q8_0(np.random.default_rng(12), n * k // 32).reshape(-1, 34), 0, 2.0 ** -5
+    b[:, at:at + 2] = (b[:, at:at + 2].copy().view(np.float16) * np.float16(scale)).view(np.uint8)
+    w = (rt.q6k_repack if fmt == Q6K else rt.q8_0_repack)(b.reshape(-1))
+    w64 = (orc.q6k_dequant if fmt == Q6K else orc.q8_0_dequant)(b.reshape(-1), n * k).reshape(n, k).astype(np.float64)
+    assert 0 < np.abs(w64).max() < 0.9
+    x = np.random.default_rng(2).normal(size=k).astype(np.float32)
+    for at in ([77], [500, 501, 1000]):
+        for big in (1.75e38, 3.3e38):
+            y = x.copy()
+            y[at] = np.float32(big) / len(at)
+            ref = w64 @ y.astype(np.float64)
+            got = gemv(rt, dev, fmt, w, y, n, k)
+            assert np.all(np.isfinite(got))
+            # 2^-30 of a chunk's largest x per product, and a few f32 roundings
+            assert np.all(np.abs(got - ref) <= 16 * 2.0 ** -24 * (np.abs(w64) @ np.abs(y.astype(np.float64))) +
+                          len(at) * 64 * 2.0 ** -30 * big)
