@@ -15,8 +15,10 @@
 // integer dot products (v_dot4_i32_i8), so the roundings are the last digit and
 // the f32 combine per slot.  Against float64 on N(0,1) rows: Q6_K 0.9e-7 to
 // 1.1e-7 (f32 1.4e-7 to 2.8e-7), Q8_0 0.7e-7 to 1.0e-7 (f32 1.0e-7 to 2.3e-7).
-// A chunk that holds an infinity or a NaN has no such digits: its delta is
-// NaN, which sends the slot through f32 products, element by element.
+// The last digit is 2^-31 of the chunk's bound.  Where that is not enough -- a
+// group of 16 that lies 2^6 below the chunk's largest value (one channel far
+// above the others), values below 2^-102, infinities and NaNs -- the chunk's
+// slots are multiplied in f32, weight by weight (direct()).
 //   Q4_K: f32 activations; per sub-block sum q x in f32 (four chains) and sum x to
 // 48 bits, combined as the reference's scale * sum q x - min * sum x
 // (autograd2.rs:1671-1698).  The two parts cancel, so their roundings make the
@@ -41,13 +43,15 @@ namespace rt {
 namespace {
 
 // Stage of one chunk, in dwords.  Q4_K: the 64 activations, the sums of its two
-// halves and what those sums' f32 rounding left.  Else the four digit planes of 16 (dword i = elements
-// 4i .. 4i+3), then delta, padding, and for Q6_K per 16-element sub-block the
-// integer sums of x0 + 256*x1 and, packed in one dword, of x2 (low half) and x3.
-// The pitches put the 16 lanes that a 16-byte LDS read serves together on
+// halves and what those sums' f32 rounding left.  Else the four digit planes of
+// 16 (dword i = elements 4i .. 4i+3), then delta (negative or NaN where the
+// digits do not serve the chunk), padding, and for Q6_K per 16-element sub-block
+// the integer sums of x0 + 256*x1 and, packed in one dword, of x2 (low half) and
+// x3.  The pitches put the 16 lanes that a 16-byte LDS read serves together on
 // distinct banks.
 template <int FMT>
 constexpr int kAnyPitch = 64 + (FMT == RT_LINEAR_Q6K ? 12 : 4);
+constexpr uint32_t kAnySpread = 6;  // powers of two from a chunk's largest value down to each group's of 16
 constexpr float kAnyTop = 4194304.0f;  // 2^22: the scaling is exact
 constexpr float kAnyUnit = 65536.0f / 4194304.0f;  // delta is 2^(e - 16): finite up to the largest x
 
@@ -57,11 +61,11 @@ RT_DEV double dpp_f64(double v) {
   return __builtin_bit_cast(double, (uint64_t)dpp_u32<CTRL>((uint32_t)u) | (uint64_t)dpp_u32<CTRL>((uint32_t)(u >> 32)) << 32);
 }
 
-// Elements 4f .. 4f+3 of the vector (zeros past K); the 16 lanes of a chunk
-// are consecutive lanes of a wave and all call this; `store` masks the lanes
-// past the last chunk.
+// Elements 4f .. 4f+3 of the vector (zeros and not `in` past K); the 16 lanes of
+// a chunk are consecutive lanes of a wave and all call this; `store` masks the
+// lanes past the last chunk.
 template <int FMT>
-RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
+RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool in, bool store) {
   const int sub = f & 15;
   uint32_t *base = dl + (f >> 4) * kAnyPitch<FMT>, *st = base + 64;
   if constexpr (FMT == RT_LINEAR_Q4K) {
@@ -78,6 +82,9 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
                       max(f32_bits(v.z) & 0x7FFFFFFFu, f32_bits(v.w) & 0x7FFFFFFFu));
     mb = max(mb, dpp_u32<0xB1>(mb));
     mb = max(mb, dpp_u32<0x4E>(mb));
+    uint32_t gb = in ? mb : 0x7F7FFFFFu;  // least largest |x| of a group of 16; none past K
+    gb = min(gb, dpp_u32<0x141>(gb));
+    gb = min(gb, dpp_u32<0x140>(gb));
     mb = max(mb, dpp_u32<0x141>(mb));
     mb = max(mb, dpp_u32<0x140>(mb));
     // max < 2^e; below 2^-103 the scale stays at the largest normal one
@@ -85,13 +92,19 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
     const float s = bits_f32(f32_bits(kAnyTop) - ((uint32_t)e << 23));
     float delta = bits_f32(f32_bits(1.0f / 65536.0f) + ((uint32_t)e << 23));
     if (mb >= 0x7F800000u) delta = bits_f32(0x7FC00000u);
+    // negative: the digits do not serve the chunk
+    if ((mb >> 23) - (gb >> 23) > kAnySpread || ((mb >> 23) < 24 && mb != 0)) delta = -delta;
     const float xs[4] = {v.x, v.y, v.z, v.w};
-    uint32_t b[4], r[4];  // bytes 0..2: X + 0x808080; the fourth digit + 128
+    // 1.5 * 2^23 + v holds rint(v) in its low mantissa bits: 5 operations per
+    // element, where rounding and converting took 10 (0.3 us at K = 9024)
+    constexpr float magic = 12582912.0f;
+    uint32_t b[4], r[4];  // bytes 0..2: X + 0x808080; byte 0: the fourth digit
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float t = __builtin_amdgcn_fmed3f(xs[i] * s, -kAnyTop, kAnyTop), X = __builtin_rintf(t);
-      b[i] = (uint32_t)(int)X + 0x808080u;
-      r[i] = (uint32_t)((int)__builtin_rintf((t - X) * 254.0f) + 128);
+      const float t = fmaf(xs[i], s, magic);
+      b[i] = f32_bits(t) + 0x408080u;
+      r[i] = f32_bits(fmaf(fmaf(xs[i], s, magic - t), 254.0f, magic));
+      asm volatile("" : "+v"(b[i]), "+v"(r[i]));  // one after the other: registers
     }
     const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);  // b0.0 b1.0 b0.1 b1.1
     const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
@@ -102,7 +115,7 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
     d[0] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
     d[1] = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
     d[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u;
-    d[3] = __builtin_amdgcn_perm(r23, r01, 0x05040100u) ^ 0x80808080u;
+    d[3] = __builtin_amdgcn_perm(r23, r01, 0x05040100u);
     int s01 = 0, s23 = 0;
     if constexpr (FMT == RT_LINEAR_Q6K) {
       auto sum4 = [](uint32_t q) { return __builtin_amdgcn_sdot4((int)q, 0x01010101, 0, false); };
@@ -124,9 +137,9 @@ RT_DEV void any_stage(uint32_t *dl, int f, float4 v, bool store) {
 }
 
 // sum_k c_k x_k / delta from a group's digit sums: the middle digits combine
-// exactly (|s0 + 256 s1| < 2^28), then one rounding per step.  Below 2^34 with
-// Q6_K's scales, so the block's f16 scale multiplies it safely; the product with
-// delta, the last one, is the slot's value.
+// exactly (|s0 + 256 s1| < 2^28), then one rounding per step.  The product of
+// delta and a block's f16 scale is exact and finite, and its product with the
+// dot is the slot's value.
 RT_DEV float any_dot(const int (&s)[4]) {
   return fmaf((float)s[2], 65536.0f * kAnyUnit, fmaf((float)s[3], 1.0f / 254.0f, (float)(s[0] + 256 * s[1])) * kAnyUnit);
 }
@@ -202,25 +215,29 @@ struct AnyTile<RT_LINEAR_Q4K, ITERS> {
     for (int it = 0; it < ITERS; ++it) ok = ok && __builtin_isfinite(p[it]);
     return ok;
   }
-  // The slot's part p of a row weight by weight (unless the block's scales are
-  // what is not finite).
-  RT_DEV static float exact(const uint8_t *W, const float *x, int, int K, int row, int slot, float p) {
-    const uint8_t *bp = W + ((size_t)row * (K / 256) + (slot >> 2)) * kQ4KBlockBytes;
-    const uint4 hd = *reinterpret_cast<const uint4 *>(bp);
-    if ((hd.x & 0x7C00u) == 0x7C00u || (hd.x & 0x7C000000u) == 0x7C000000u) return p;
+  // The slot's part p of the (first) row weight by weight, unless the block's
+  // scales are what is not finite.
+  RT_DEV float direct(const float *x, int slot, float p) const {
+    const float4 *xp = reinterpret_cast<const float4 *>(x + 64 * slot);
     uint32_t svp, mvp;
-    q4k_scale_min_pair(hd.y, hd.z, hd.w, slot & 3, svp, mvp);
-    const float d = half_bits_to_f32(hd.x & 0xFFFFu), dm = half_bits_to_f32(hd.x >> 16);
-    float acc = 0.f;
-    bool finite = true;
-#pragma unroll 1
-    for (int i = 0; i < 64; ++i) {
-      const int h = i >> 5, q = (bp[16 + 32 * (slot & 3) + (i & 31)] >> (4 * h)) & 15;
-      const float v = x[64 * slot + i], w = fmaf(d * (float)((svp >> (8 * h)) & 0xFFu), (float)q, -(dm * (float)((mvp >> (8 * h)) & 0xFFu)));
-      finite = finite && __builtin_isfinite(v);
-      acc = fmaf(w, v, acc);
+    q4k_scale_min_pair(hd[0].y, hd[0].z, hd[0].w, slot & 3, svp, mvp);
+    const float d = half_bits_to_f32(hd[0].x & 0xFFFFu), dm = half_bits_to_f32(hd[0].x >> 16);
+    const float s[2] = {d * (float)(svp & 0xFFu), d * (float)(svp >> 8)};
+    const float m[2] = {dm * (float)(mvp & 0xFFu), dm * (float)(mvp >> 8)};
+    float acc[4] = {0.f, 0.f, 0.f, 0.f}, nan = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {  // elements 4j .. 4j+3
+      const float4 v = xp[j];
+      const uint4 q = (j & 4) ? qb[0] : qa[0];
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w}, c = (w[j & 3] >> (4 * (j >> 3))) & 0x0F0F0F0Fu;
+      acc[0] = fmaf(fmaf(s[j >> 3], ubyte0(c), -m[j >> 3]), v.x, acc[0]);
+      acc[1] = fmaf(fmaf(s[j >> 3], ubyte1(c), -m[j >> 3]), v.y, acc[1]);
+      acc[2] = fmaf(fmaf(s[j >> 3], ubyte2(c), -m[j >> 3]), v.z, acc[2]);
+      acc[3] = fmaf(fmaf(s[j >> 3], ubyte3(c), -m[j >> 3]), v.w, acc[3]);
+      nan = fmaf(0.f, v.x, fmaf(0.f, v.y, fmaf(0.f, v.z, fmaf(0.f, v.w, nan))));
     }
-    return finite ? acc : bits_f32(0x7FC00000u);
+    const bool scales = (hd[0].x & 0x7C00u) != 0x7C00u && (hd[0].x & 0x7C000000u) != 0x7C000000u;
+    return scales ? (acc[0] + acc[1]) + (acc[2] + acc[3]) + nan : p;
   }
 };
 
@@ -277,27 +294,41 @@ struct AnyTile<RT_LINEAR_Q6K, ITERS> {  // slot: see Q6KTile (kquant_tile.hpp)
         acc[it][m >> 1] = fmaf((float)(int)__builtin_amdgcn_sbfe(scw, 16 * (m & 1) + 8 * a, 8), t, acc[it][m >> 1]);
       }
     }
-    const float d0 = bits_f32(base[64]), d1 = bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]);
+    const float d0 = fabsf(bits_f32(base[64])), d1 = fabsf(bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]));
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const float d = half_bits_to_f32(dd[it]);
-      p[it] = fmaf(acc[it][1] * d, d1, acc[it][0] * d * d0);
+      p[it] = fmaf(acc[it][1], d * d1, acc[it][0] * (d * d0));
     }
   }
   RT_DEV static bool plain(const uint32_t *dl, int slot, const float (&)[ITERS]) {
     const uint32_t *base = dl + 2 * (slot >> 1) * kAnyPitch<RT_LINEAR_Q6K>;
-    return !__builtin_isnan(bits_f32(base[64])) && !__builtin_isnan(bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]));
+    return bits_f32(base[64]) > 0.f && bits_f32(base[kAnyPitch<RT_LINEAR_Q6K> + 64]) > 0.f;
   }
-  // The slot's part of a row in f32: 16 elements of each quarter of its half block.
-  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot, float) {
-    const Q6KPlanes P = q6k_planes(W, (size_t)N * (K / 256));
-    float acc = 0.f;
-#pragma unroll 1
-    for (int i = 0; i < 64; ++i) {
-      const int e = 128 * ((slot >> 1) & 1) + 32 * (i >> 4) + 16 * (slot & 1) + (i & 15);
-      acc = fmaf(q6k_value(P, (size_t)row * (K / 256) + (slot >> 2), e), x[256 * (slot >> 2) + e], acc);
+  // The slot's part of the (first) row in f32, q6k_value by q6k_value: 16
+  // elements of each quarter of its half block.
+  RT_DEV float direct(const float *x, int slot, float) const {
+    const int a = slot & 1;
+    const float4 *xp = reinterpret_cast<const float4 *>(x + 128 * (slot >> 1) + 16 * a);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      asm volatile("" : "+v"(xp), "+v"(acc[0]));  // one quarter after the other: registers
+      const uint4 ql = (m & 1) ? qb[0] : qa[0];
+      const uint32_t lw[4] = {ql.x, ql.y, ql.z, ql.w}, hb[4] = {qh[0].x, qh[0].y, qh[0].z, qh[0].w};
+      const float s = half_bits_to_f32(dd[0]) *
+                      (float)(int)__builtin_amdgcn_sbfe(m < 2 ? sc[0].x : sc[0].y, 16 * (m & 1) + 8 * a, 8);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float4 v = xp[8 * m + k];
+        const uint32_t q = ((m < 2 ? lw[k] : lw[k] >> 4) & 0x0F0F0F0Fu) | (((hb[k] >> (2 * m)) & 0x03030303u) << 4);
+        acc[0] = fmaf(mul_nc(s, (float)((int)(q & 0xFFu) - 32)), v.x, acc[0]);
+        acc[1] = fmaf(mul_nc(s, (float)((int)((q >> 8) & 0xFFu) - 32)), v.y, acc[1]);
+        acc[2] = fmaf(mul_nc(s, (float)((int)((q >> 16) & 0xFFu) - 32)), v.z, acc[2]);
+        acc[3] = fmaf(mul_nc(s, (float)((int)(q >> 24) - 32)), v.w, acc[3]);
+      }
     }
-    return acc;
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
   }
 };
 
@@ -321,6 +352,7 @@ struct AnyTile<RT_LINEAR_Q8_0, ITERS> {
       for (int d = 0; d < 4; ++d) s[it][d] = 0;
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
+      if (ITERS == 4 && g) __builtin_amdgcn_sched_barrier(0);
       uint4 x[4];
 #pragma unroll
       for (int d = 0; d < 4; ++d) x[d] = *reinterpret_cast<const uint4 *>(base + 16 * d + 8 * (slot & 1) + 4 * g);
@@ -337,28 +369,41 @@ struct AnyTile<RT_LINEAR_Q8_0, ITERS> {
           }
       }
     }
-    const float delta = bits_f32(base[64]);
+    const float delta = fabsf(bits_f32(base[64]));
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) p[it] = half_bits_to_f32(dd[it]) * any_dot(s[it]) * delta;
+    for (int it = 0; it < ITERS; ++it) p[it] = half_bits_to_f32(dd[it]) * delta * any_dot(s[it]);
   }
   RT_DEV static bool plain(const uint32_t *dl, int slot, const float (&)[ITERS]) {
-    return !__builtin_isnan(bits_f32(dl[(slot >> 1) * kAnyPitch<RT_LINEAR_Q8_0> + 64]));
+    return bits_f32(dl[(slot >> 1) * kAnyPitch<RT_LINEAR_Q8_0> + 64]) > 0.f;
   }
-  RT_DEV static float exact(const uint8_t *W, const float *x, int N, int K, int row, int slot, float) {
-    float acc = 0.f;
-#pragma unroll 1
-    for (int i = 32 * slot; i < 32 * slot + 32; ++i)
-      acc = fmaf(q8_0_value(W, (size_t)N * K, (size_t)row * K + i), x[i], acc);
-    return acc;
+  RT_DEV float direct(const float *x, int slot, float) const {
+    const float4 *xp = reinterpret_cast<const float4 *>(x + 32 * slot);
+    const float d = half_bits_to_f32(dd[0]);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      if (g == 4) asm volatile("" : "+v"(xp), "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+      const float4 v = xp[g];
+      const uint4 q = g < 4 ? qa[0] : qb[0];
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+      acc[0] = fmaf(d * (float)(int8_t)(w[g & 3] & 0xFFu), v.x, acc[0]);
+      acc[1] = fmaf(d * (float)(int8_t)((w[g & 3] >> 8) & 0xFFu), v.y, acc[1]);
+      acc[2] = fmaf(d * (float)(int8_t)((w[g & 3] >> 16) & 0xFFu), v.z, acc[2]);
+      acc[3] = fmaf(d * (float)(int8_t)(w[g & 3] >> 24), v.w, acc[3]);
+    }
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
   }
 };
 
 // Dynamic LDS: the staged chunks, then ITERS * T slot sums.  T = blockDim.x as
 // an argument: reading blockDim makes the runtime fill the launch's hidden
 // arguments, 0.6 us of host time.
+// Q8_0 in 80 registers: three workgroups of 512 threads per CU, so that the 615 of
+// 12288x3072 run at once (89 registers: 10.0 us against 9.8).
 template <int FMT, int ITERS>
-__global__ __launch_bounds__(1024) void k_gemv_any(const uint8_t *__restrict__ W, const float *__restrict__ x,
-                                                   float *__restrict__ y, int N, int K, int S, int rpi, int T) {
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FMT == RT_LINEAR_Q8_0 ? 6 : 4))) void
+k_gemv_any(const uint8_t *__restrict__ W, const float *__restrict__ x, float *__restrict__ y, int N, int K, int S, int rpi,
+           int T) {
   extern __shared__ __attribute__((aligned(16))) uint32_t any_lds[];
   const int tid = (int)threadIdx.x;
   const int nchunk = (K + 63) / 64, nf = K / 4;
@@ -380,15 +425,21 @@ __global__ __launch_bounds__(1024) void k_gemv_any(const uint8_t *__restrict__ W
     const int f = tid + i * T;
     if (i > 0 && i * T >= 16 * nchunk) break;  // uniform
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    any_stage<FMT>(dl, f, f < nf ? xv[i] : z, f < 16 * nchunk);
+    any_stage<FMT>(dl, f, f < nf ? xv[i] : z, f < nf, f < 16 * nchunk);
   }
   __syncthreads();
   float p[ITERS];
   tile.compute(dl, slot, p);
-  if (!tile.plain(dl, slot, p)) {
+  if (__builtin_expect(!tile.plain(dl, slot, p), 0)) {
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it)
-      p[it] = AnyTile<FMT, ITERS>::exact(W, x, N, K, min(row0 + it * rpi + rsub, N - 1), slot, p[it]);
+    for (int it = 0; it < ITERS; ++it) {
+      // the row's weights again, one row at a time: kept across compute() they spill
+      int row = min(row0 + it * rpi + rsub, N - 1);
+      asm volatile("" : "+v"(row), "+v"(p[it > 0 ? it - 1 : 0]));
+      AnyTile<FMT, 1> again;
+      again.load(0, W, N, K, row, slot);
+      p[it] = again.direct(x, slot, p[it]);
+    }
   }
   if (rsub < rpi) {
 #pragma unroll
@@ -478,7 +529,7 @@ RT_DEV void any_stage_pro(uint32_t *dl, const float4 (&xn)[2], int K, int T) {
   for (int i = 0; i < 2; ++i) {
     const int f = (int)threadIdx.x + i * T;
     if (i > 0 && T >= nst) break;  // uniform
-    any_stage<FMT>(dl, f, f < nf ? xn[i] : make_float4(0.f, 0.f, 0.f, 0.f), f < nst);
+    any_stage<FMT>(dl, f, f < nf ? xn[i] : make_float4(0.f, 0.f, 0.f, 0.f), f < nf, f < nst);
   }
 }
 

@@ -166,3 +166,43 @@ def test_gemv_any_top_of_the_range(rt, orc, dev, fmt, n, k):
             # 2^-30 of a chunk's largest x per product, and a few f32 roundings
             assert np.all(np.abs(got - ref) <= 16 * 2.0 ** -24 * (np.abs(w64) @ np.abs(y.astype(np.float64))) +
                           len(at) * 64 * 2.0 ** -30 * big)
+
+
+@pytest.mark.parametrize("fmt,n,k", [(Q6K, 70, 1280), (Q6K, 9001, 768), (Q8_0, 70, 1120), (Q8_0, 7000, 1152)])
+def test_gemv_any_wide_chunks(rt, orc, dev, fmt, n, k):
+    """Chunks that four digits of one scale do not cover, in every workgroup
+    shape: a channel 2^20 (and 2^8) times the others whose weights are zero, a
+    chunk of small values beside it, and a vector below 2^-110.  The others keep
+    f32 accuracy: 2^-24 of the sum of the magnitudes for each of 8 products of a
+    chain, 2 and 1 to the slot, k / 1024 + 4 over the slots, and the store."""
+    rng = np.random.default_rng(13)
+    big = k - 40  # in Q8_0's half chunk at the end of 1120
+    if fmt == Q6K:
+        b = synth_q6k(rng, n * k // 256).reshape(n, k // 256, 210).copy()
+        i = big % 256
+        j, m, l = i // 128, i % 128 // 32, i % 32
+        ql, qh = 64 * j + 32 * (m & 1) + l, 128 + 32 * j + l
+        b[:, big // 256, ql] &= 0xF0 if m < 2 else 0x0F
+        b[:, big // 256, qh] = b[:, big // 256, qh] & ~np.uint8(3 << 2 * m) | np.uint8(2 << 2 * m)  # code 32: zero
+        w, w64 = rt.q6k_repack(b.reshape(-1)), orc.q6k_dequant(b.reshape(-1), n * k)
+    else:
+        b = synth_q8_0(rng, n * k // 32).reshape(n, k // 32, 34).copy()
+        b[:, big // 32, 2 + big % 32] = 0
+        w, w64 = rt.q8_0_repack(b.reshape(-1)), orc.q8_0_dequant(b.reshape(-1), n * k)
+    w64 = w64.reshape(n, k).astype(np.float64)
+    assert np.all(w64[:, big] == 0.0)
+    x0 = rng.normal(size=k).astype(np.float32)
+    steps = 8 + 2 + 1 + -(-k // 512) + 4 + 1
+    for what in ("channel 2^20", "channel 2^8", "small chunk", "small vector"):
+        x = x0.copy()
+        if what.startswith("channel"):
+            x[big] = 2.0 ** 20 if what.endswith("20") else 2.0 ** 8
+        elif what == "small chunk":
+            x[64:112] *= np.float32(2.0 ** -30)
+        else:
+            x *= np.float32(2.0 ** -112)
+        rest = x.astype(np.float64)
+        rest[big] = 0.0
+        got = gemv(rt, dev, fmt, w, x, n, k)
+        bound = steps * 2.0 ** -24 * (np.abs(w64) @ np.abs(rest)) + k * 2.0 ** -149
+        assert np.all(np.abs(got - w64 @ x.astype(np.float64)) <= bound), what
