@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 
 #include "../../include/rt_hip.h"
 #include "decode.hpp"
@@ -644,13 +645,29 @@ __global__ __launch_bounds__(512) void k_any_prologue(DecodeArgs a, const float 
 // 12288x3072 47.0 -> 9.7, 6912x1152 8.1 -> 3.7.
 constexpr int kAnyMaxK = 16384;  // four float4 of x per thread at T = 1024
 
+// Allows k_gemv_any the LDS of its longest rows (86 KB of the CU's 160), once per
+// device: the allowance is the kernel's, so one set per call and to that call's
+// size could take it from a launch of another host thread.
+template <int FMT, int ITERS>
+static hipError_t any_allow_lds() {
+  static std::atomic<uint64_t> done{0};  // a bit per device
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+  if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
+  e = hipFuncSetAttribute((const void *)k_gemv_any<FMT, ITERS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          kAnyMaxK / 64 * kAnyPitch<FMT> * 4 + ITERS * 1024 * 4);
+  if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
+  return e;
+}
+
 template <int FMT, int ITERS>
 static hipError_t launch_any(const void *W, const float *x, float *y, int N, int K, int S, int T, hipStream_t s) {
   const int rpi = T / S, rows = rpi * ITERS;
   const size_t lds = (size_t)((K + 63) / 64) * kAnyPitch<FMT> * 4 + (size_t)rows * S * 4;
-  if (lds > 65536) {  // up to 92 KB of the CU's 160 KB
-    const hipError_t e = hipFuncSetAttribute((const void *)k_gemv_any<FMT, ITERS>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (lds > 65536) {
+    const hipError_t e = any_allow_lds<FMT, ITERS>();
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL((k_gemv_any<FMT, ITERS>), dim3((unsigned)((N + rows - 1) / rows)), dim3(T), lds, s,

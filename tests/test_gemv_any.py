@@ -206,3 +206,58 @@ def test_gemv_any_wide_chunks(rt, orc, dev, fmt, n, k):
         got = gemv(rt, dev, fmt, w, x, n, k)
         bound = steps * 2.0 ** -24 * (np.abs(w64) @ np.abs(rest)) + k * 2.0 ** -149
         assert np.all(np.abs(got - w64 @ x.astype(np.float64)) <= bound), what
+
+
+def test_gemv_any_large_lds_from_two_threads(rt, orc, dev):
+    """Rows whose staging needs more than 64 KB of LDS, of two lengths, launched by
+    two host threads at once: neither takes the other's allowance away."""
+    import threading
+    import torch
+    work = []
+    for n, k in ((40, 16384), (64, 14336)):
+        w, w64 = weight(rt, orc, Q6K, n, k, seed=k)
+        x = np.random.default_rng(n).normal(size=k).astype(np.float32)
+        work.append((to_dev(w, dev), to_dev(x, dev), torch.zeros(200, n, device=dev), n, k, w64 @ x.astype(np.float64)))
+    errors = []
+
+    def run(w, x, y, n, k, ref):
+        try:
+            stream = torch.cuda.Stream()
+            for i in range(y.shape[0]):
+                rt.q6k_gemv(w, x, y[i], n, k, stream=stream)
+            stream.synchronize()
+        except Exception as e:  # reported by the test's own thread
+            errors.append(e)
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=run, args=a) for a in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for _, _, y, _, _, ref in work:
+        got = y.cpu().numpy()
+        assert rel_l2(got[0], ref) < 2e-6 and np.array_equal(got, np.broadcast_to(got[0], got.shape))
+
+
+def test_gemv_any_large_lds_captured(rt, orc, dev):
+    """The first call of that length inside a capture; calls of a shorter length
+    between the replays."""
+    import torch
+    n, k = 40, 16384
+    w, w64 = weight(rt, orc, Q8_0, n, k, seed=1)
+    ws, ws64 = weight(rt, orc, Q8_0, n, 16000, seed=2)
+    x = np.random.default_rng(3).normal(size=k).astype(np.float32)
+    wd, xd, y = to_dev(w, dev), to_dev(x, dev), torch.zeros(n, device=dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        rt.q8_0_gemv(wd, xd, y, n, k, stream=torch.cuda.current_stream())
+    for _ in range(4):
+        y.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(y.cpu().numpy(), w64 @ x.astype(np.float64)) < 2e-6
+        assert rel_l2(gemv(rt, dev, Q8_0, ws, x[:16000], n, 16000), ws64 @ x[:16000].astype(np.float64)) < 2e-6

@@ -16,7 +16,8 @@ BF16, Q6K, Q8_0 = 2, 4, 5
 
 
 # hidden 768: 24 Q8_0 slots per row (workgroups that hold rows of two
-# matrices); hidden 3840 (Gemma-3-12B's): 1024-thread workgroups of q|k|v
+# matrices); hidden 3840 (Gemma-3-12B's): 1024-thread workgroups of q|k|v; ffn
+# 15360: a down projection that stages more than 64 KB, captured
 @pytest.mark.parametrize("hidden,ffn,heads,kv,plan", [
     (768, 1536, (4, 128), 2, {}),
     (768, 1536, (4, 128), 2, {p: Q6K for p in ("q", "k", "v", "o", "gate", "up", "down")}),
@@ -24,6 +25,7 @@ BF16, Q6K, Q8_0 = 2, 4, 5
     (768, 1536, (4, 128), 1, dict(v=Q6K, o=BF16, gate=Q8_0, down=Q8_0)),
     (768, 1536, (2, 256), 2, dict(q=BF16, k=BF16, v=BF16, gate=BF16, up=BF16, down=BF16)),
     (3840, 4096, (16, 256), 8, dict(v=Q6K, down=Q6K)),
+    (768, 15360, (4, 128), 2, dict(down=Q6K)),
 ])
 def test_step_any_matches_oracle(rt, orc, hidden, ffn, heads, kv, plan):
     from test_oracle import make_model
