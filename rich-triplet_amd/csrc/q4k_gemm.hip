@@ -669,6 +669,11 @@ static GemmPlan gemm_plan(int M, int N, int K, double *est = nullptr) {
   return best;
 }
 
+int q4k_gemm_kernel(int M, int tiles_n, int K, bool set) {
+  const GemmPlan p = set ? GemmPlan{gemm_set_kind(M, tiles_n, K), 1} : gemm_plan(M, 256 * tiles_n, K);
+  return 16 * p.ks + (int)p.kind;
+}
+
 // Narrow outputs of many rows have few tiles for these kernels: where the
 // weight widened to f16 once (N K words written and read, 4 TB/s) and the
 // smaller tiles of proj_gemm.hip come out a tenth ahead, they take the

@@ -121,6 +121,11 @@ size_t proj_gemm_prepped_ws_bytes(int M, int N, int K);
 // Q4_K GEMM C[M,N] = A[M,K] . W[N,K]^T; A bf16 bits (a_bf16) or f32; ws holds
 // q4k_gemm_workspace_bytes(M, N, K) bytes of device scratch.
 size_t q4k_gemm_workspace_bytes(int M, int N, int K);
+// The kernel that takes a product of tiles_n 256-column tiles, or a set of
+// matrices sharing A (gate|up: tiles_n of 128 columns of both): 0 eight-wave,
+// 1 half-block, 2 ping-pong, plus 16 times the K splits.  The tests hold their
+// shapes to it.
+int q4k_gemm_kernel(int M, int tiles_n, int K, bool set);
 // Whether a Q4_K product runs faster on launch_proj_gemm (RT_LINEAR_Q4K) than
 // on launch_q4k_gemm, from the two time models.
 bool q4k_gemm_widen(int M, int N, int K);

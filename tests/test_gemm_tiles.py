@@ -1,6 +1,7 @@
 """The tiled GEMMs at the edges of their tiles, against float64 products: the
 256x256 ping-pong kernel on Q4_K (q4k_gemm_pp.hip: partial row and column
-tiles, unaligned widths, one super-block, K splits), and the 128x128 and
+tiles, unaligned widths, K splits; its sets and one super-block per row in
+test_prefill.py), the half-block and eight-wave kernels, and the 128x128 and
 256x256 kernels on widened weights (proj_gemm.hip: one stage, ring remainders,
 K splits, bias, narrow outputs of Q4_K)."""
 from __future__ import annotations

@@ -43,16 +43,16 @@ def _run_bf16(rt, dev, a_bits, blocks, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k,seed", [
-    (2, 256, 256, 1),        # smaller than one tile
+    (2, 256, 256, 1),        # few-row kernel: smaller than one tile
     (17, 300, 512, 2),       # ragged M and N (N not a multiple of 16)
     (130, 260, 768, 3),      # ragged, more than one tile each way
     (64, 2048, 2560, 4),     # Gemma q-projection shape, short prompt
-    (512, 10240, 2560, 5),   # prefill, gate/up shape
-    (512, 2560, 10240, 6),   # prefill, down-projection shape
-    (1100, 1024, 2560, 7),   # above 1024 rows: half-block kernel, K split 4 ways, ragged M
-    (2100, 2560, 10240, 8),  # half-block kernel, K split 3 ways (long-prompt down shape)
-    (1024, 2560, 2048, 9),   # the kernel switch: eight-wave kernel up to 1024 rows (K split 2 ways) ...
-    (1025, 2560, 2048, 10),  # ... half-block kernel from 1025 (K split 2 ways), one ragged row
+    (512, 10240, 2560, 5),   # prefill, gate/up shape: eight-wave kernel
+    (512, 2560, 10240, 6),   # prefill, down-projection shape: eight-wave kernel, K split 6 ways
+    (1100, 1024, 2560, 7),   # a narrow output: the weight widened to f16, ragged M
+    (2100, 2560, 10240, 8),  # ping-pong kernel, K split 2 ways (long-prompt down shape)
+    (1024, 2560, 2048, 9),   # widened to f16, whole row tiles ...
+    (1025, 2560, 2048, 10),  # ... and one ragged row
     (1000, 16384, 512, 11),  # under 1024 rows with 512 tiles: half-block kernel, ragged M
 ])
 def test_gemm_bf16_vs_oracle(rt, orc, dev, m, n, k, seed):
@@ -67,17 +67,17 @@ def test_gemm_bf16_vs_oracle(rt, orc, dev, m, n, k, seed):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (4608, 9216, 3072),    # FLUX-12B QKV: half-block kernel (648 tiles of 256 x 256)
-    (4608, 12288, 3072),   # FLUX-12B MLP up: half-block kernel
-    (4608, 3072, 12288),   # FLUX-12B MLP down: 256 x 256 kernel (216 tiles), one round
-    (4096, 2560, 10240),   # 4096-row prefill down: 256 x 256 kernel, K split 3 ways
-    (4096, 2560, 2048),    # 4096-row prefill o: 256 x 256 kernel (160 tiles)
-    (1500, 5632, 8192),    # 256 x 256 kernel, K split 3 ways, ragged M
-    (1300, 9000, 2560),    # 256 x 256 kernel, ragged M and N
+    (4608, 9216, 3072),    # FLUX-12B QKV: 648 tiles
+    (4608, 12288, 3072),   # FLUX-12B MLP up
+    (4608, 3072, 12288),   # FLUX-12B MLP down: 216 tiles, one round
+    (4096, 2560, 10240),   # 4096-row prefill down
+    (4096, 2560, 2048),    # 4096-row prefill o: 160 tiles
+    (1500, 5632, 8192),    # ragged M
+    (1300, 9000, 2560),    # ragged M and N
 ])
 def test_gemm_flux_shapes(rt, orc, dev, m, n, k):
-    """FLUX-12B shapes (QKV, MLP-up, MLP-down) and the shapes that take the
-    256 x 256-tile kernel; reference on the GPU in f32 from the oracle's
+    """FLUX-12B shapes (QKV, MLP-up, MLP-down) and others that take the
+    ping-pong kernel of 256 x 256 tiles; reference on the GPU in f32 from the oracle's
     dequantised weights (a library GEMM, not this library's kernels)."""
     import torch
     blocks = orc.synth_q4k(7 + n, n, k)

@@ -4,6 +4,8 @@ over the whole prompt, transformer4.rs:1900-1964 and 2103-2139; attention
 (rt_decode_prefill) against it."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -522,7 +524,7 @@ def test_gpu_generic_shape_prefill_matches_oracle(rt, orc, mode, T):
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", [0, 1])
 def test_gpu_long_prompt_prefill_matches_oracle(rt, orc, mode):
-    """1100 rows: the projections run on the half-block GEMM with K split
+    """1100 rows: the projections run on the half-block GEMM, down with K split
     (the consumers add the partial tiles while reading them), attention on
     eight-wave workgroups of 128 columns; logits and KV rows vs the oracle."""
     cfg = tiny(2, sliding_window=300)
@@ -643,15 +645,60 @@ def test_gemma3_4b_shape_prefill_equals_decode_steps(rt, orc):
     d2.close()
 
 
+PING_PONG = 16 + 2  # q4k_gemm_kernel's number of the 256 x 256 kernel, K whole
+
+
+def set_kernel(rt, rows, tiles, k):
+    """The GEMM kernel the library picks for a set of matrices sharing their rows."""
+    fn = rt.lib()["_ZN2rt15q4k_gemm_kernelEiiib"]
+    fn.argtypes, fn.restype = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_bool], ctypes.c_int
+    return fn(rows, tiles, k, True)
+
+
+# Shapes whose q|k|v and gate|up sets run on the 256 x 256 ping-pong kernel, the
+# row count past a whole tile, with the q/k norm and RoPE in its epilogue
+# (head_dim 256) and without (128), and with one super-block per row
+PING_PONG_SETS = [
+    (dict(hidden=512, ffn=3072, n_q_heads=16, n_kv_heads=4, head_dim=256), 1300, 1),
+    (dict(hidden=512, ffn=3072, n_q_heads=32, n_kv_heads=8, head_dim=128, attn_scale=1.0 / np.sqrt(128.0)), 1301, 0),
+    (dict(hidden=256, ffn=3840, n_q_heads=20, n_kv_heads=5, head_dim=256), 1030, 1),
+]
+
+
+@pytest.mark.parametrize("shape,T,mode", PING_PONG_SETS)
+def test_ping_pong_sets_take_the_ping_pong_kernel(rt, shape, T, mode):
+    heads = shape["n_q_heads"] + 2 * shape["n_kv_heads"]
+    assert set_kernel(rt, T, heads * shape["head_dim"] // 256, shape["hidden"]) == PING_PONG
+    assert set_kernel(rt, T, shape["ffn"] // 128, shape["hidden"]) == PING_PONG
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,T,mode", PING_PONG_SETS)
+def test_gpu_ping_pong_sets_match_oracle(rt, orc, shape, T, mode):
+    """q|k|v and gate|up of a long prompt on the ping-pong kernel: logits and every
+    KV row of two layers (one local, one global)."""
+    cfg = tiny(2, n_layers=2, global_every=2, sliding_window=300, **shape)
+    layers, embed, fnorm = make_model(orc, cfg, max_seq=T + 4, ctx=0, seed=6900 + T)
+    toks = [(29 * i + 7) % cfg["vocab"] for i in range(T)]
+    d = gpu_ctx(rt, cfg, layers, embed, fnorm, T + 4)
+    got = d.prefill(toks, 0, mode)
+    ref_layers = fresh_caches(layers)
+    ref = orc.gemma3_prefill(cfg, ref_layers, embed, fnorm, toks, 0, mode)
+    assert np.all(np.isfinite(got))
+    assert rel_l2(got, ref) < LOGITS_TOL, rel_l2(got, ref)
+    assert_kv_rows(d, cfg, layers, embed, fnorm, toks, mode, True, ref_layers)
+    d.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,mode", [(1100, 0), (1100, 1), (960, 1)])
 def test_gemma3_4b_width_long_prefill_matches_oracle(rt, orc, T, mode):
     """The benchmarked prefill path at Gemma-3-4B widths: 2 layers (one local
     with window 1024, one global) and 1100 rows, so each projection set
-    (q|k|v, gate|up) runs as one launch of the half-block GEMM, K is split
-    where tiles are few and the consumers add the partial tiles; both window
-    rules.  At 960 rows the gate|up set (640 tiles) still runs as one
-    half-block launch while q|k|v, o and down take the eight-wave kernel.
+    (q|k|v, gate|up) runs as one launch of the half-block GEMM, o on it and down
+    on the ping-pong kernel with K split (the consumers add the partial tiles);
+    both window rules.  At 960 rows the gate|up set (640 tiles) still runs as
+    one half-block launch while q, k, v and o take the few-row kernel.
     Logits against the oracle at the north-star bar.  KV rows: the oracle
     on every row against a float64 restatement (np_prefill), and the GPU on
     every row within KV_TOL of the same restatement with the GPU's operand
