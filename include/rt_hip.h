@@ -330,7 +330,10 @@ rt_status rt_decode_step_async(rt_decode *d, int32_t token, int32_t position);
  * start_position .. start_position+m-1, as used by speculative verify.  Each
  * token attends to the K/V of the tokens before it in the batch; logits_host
  * (may be NULL) receives m x vocab floats, row i for token i.  The lm_head
- * reads the embedding once for all m tokens. */
+ * reads the embedding once for all m tokens.  The logits are those of m steps
+ * up to rounding, not bit for bit: the verify rounds activations to 16 bits of
+ * their 64-element chunk's maximum, the step sums in another order and, at
+ * widths without fused kernels, keeps 24 to 32 bits. */
 rt_status rt_decode_step_batch(rt_decode *d, const int32_t *tokens, int32_t m, int32_t start_position,
                                float *logits_host);
 rt_status rt_decode_step_batch_async(rt_decode *d, const int32_t *tokens, int32_t m, int32_t start_position);

@@ -10,7 +10,7 @@ import copy
 import numpy as np
 import pytest
 
-from test_gpu_decode import tiny
+from test_gpu_decode import generic_cfg, tiny
 from test_oracle import make_model
 
 
@@ -150,6 +150,19 @@ def test_speculative_equals_plain_on_oracle_model(rt, orc):
     assert st["spec_attempts"] > 0 and st["spec_accepted"] < st["spec_drafted"]
 
 
+def gpu_runs(rt, cfg, layers, embed, fnorm, max_seq):
+    """(tokens, stats) on the GPU without and with drafts of up to 4 tokens."""
+    runs = []
+    for draft_len in (0, 4):
+        d = rt.HipDecodeContext(cfg, max_seq)
+        for i, L in enumerate(layers):
+            d.set_layer(i, L)
+        d.set_embed(embed, fnorm)
+        runs.append(rt.generate_greedy(d, SPEC_PROMPT, 40, draft_len=draft_len))
+        d.close()
+    return runs
+
+
 @pytest.mark.gpu
 def test_gpu_speculative_generation_matches_plain_and_oracle(rt, orc):
     """The batched verify in the loop: rejected drafts leave cache rows that
@@ -159,16 +172,22 @@ def test_gpu_speculative_generation_matches_plain_and_oracle(rt, orc):
     max_seq = 64
     layers, embed, fnorm = make_model(orc, cfg, max_seq=max_seq, ctx=0, seed=0)
     ref, _ = rt.generate_greedy(OracleCtx(orc, cfg, layers, embed, fnorm), SPEC_PROMPT, 40, draft_len=0)
-    runs = {}
-    for draft_len in (0, 4):
-        d = rt.HipDecodeContext(cfg, max_seq)
-        for i, L in enumerate(layers):
-            d.set_layer(i, L)
-        d.set_embed(embed, fnorm)
-        runs[draft_len] = rt.generate_greedy(d, SPEC_PROMPT, 40, draft_len=draft_len)
-        d.close()
-    (plain, s0), (spec, s1) = runs[0], runs[4]
+    (plain, s0), (spec, s1) = gpu_runs(rt, cfg, layers, embed, fnorm, max_seq)
     assert plain == ref
     assert spec == plain
     assert s0["decode_steps"] == 39
     assert s1["spec_attempts"] > 0 and s1["spec_accepted"] < s1["spec_drafted"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seed", [0, 4])
+def test_gpu_speculative_generation_at_a_generic_width(rt, orc, seed):
+    """A width without fused kernels, where the step keeps f32 activations and the
+    verify rounds them to 16 bits: the margins of these models are far above
+    that difference, so the tokens are the same."""
+    cfg = generic_cfg()
+    layers, embed, fnorm = make_model(orc, cfg, max_seq=64, ctx=0, seed=seed)
+    ref, _ = rt.generate_greedy(OracleCtx(orc, cfg, layers, embed, fnorm), SPEC_PROMPT, 40, draft_len=0)
+    (plain, _), (spec, st) = gpu_runs(rt, cfg, layers, embed, fnorm, 64)
+    assert plain == ref and spec == plain
+    assert st["spec_attempts"] > 0
