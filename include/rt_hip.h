@@ -191,8 +191,10 @@ rt_status rt_q8_0_gemv(const void *w, const float *x, float *y, int64_t n, int64
  * (Q8_0, and BF16 with m > 8), k % 8 == 0 (BF16, m <= 8), k % 4 == 0 (F32);
  * device pointers, a and w 16-byte aligned.  Uses the
  * per-(thread, device, stream) workspace of rt_q4k_gemm_f32, about
- * (m + n) * k * 2 bytes (m * k * 2 for Q4_K, and for Q6_K and Q8_0 of up to
- * 384 rows, which stay packed; none for the f32 GEMV), plus split-K partials. */
+ * (m + n) * k * 2 bytes (m * k * 2, in whole groups of 32 rows, for Q4_K, and
+ * for Q6_K and Q8_0 of up to 384 rows, or up to 1024 where k <= 4096 and
+ * m * n <= 2,600,000, which stay packed; none for the f32 GEMV), plus split-K
+ * partials. */
 rt_status rt_linear_gemm_f32(int32_t fmt, const void *w, const float *a, float *c, int64_t m, int64_t n, int64_t k,
                              void *stream);
 /* QLinear::forward (qlinear.rs:82-111): out[m][n] = x[m][k] . W[n][k], then

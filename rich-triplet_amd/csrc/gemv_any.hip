@@ -640,9 +640,9 @@ __global__ __launch_bounds__(512) void k_any_prologue(DecodeArgs a, const float 
 //   3072x12288 in 192 workgroups 9.4, 384 10.0, 768 10.3; 12288x3072 in 512
 //   to 768 workgroups 7.4-7.7).  Q6_K stops at two: four spill registers.
 // Before, one wave per row in f32 (kept for longer K): Q4_K 15360x3840 30.3 us
-// (1.1 TB/s; now 10.0, 3.3 TB/s, of a 6.7 us streaming floor), 3072x12288
-// 24.4 -> 9.4; Q6_K 12288x3072 57.5 -> 9.7, 1152x6912 39.2 -> 5.6; Q8_0
-// 12288x3072 47.0 -> 9.7, 6912x1152 8.1 -> 3.7.
+// (1.1 TB/s; now 9.4, 3.5 TB/s, of a 6.7 us streaming floor), 3072x12288
+// 24.4 -> 8.9; Q6_K 12288x3072 57.5 -> 9.8, 1152x6912 39.2 -> 5.2; Q8_0
+// 12288x3072 47.0 -> 9.8, 6912x1152 8.1 -> 3.7.
 constexpr int kAnyMaxK = 16384;  // four float4 of x per thread at T = 1024
 
 // Allows k_gemv_any the LDS of its longest rows (86 KB of the CU's 160), once per

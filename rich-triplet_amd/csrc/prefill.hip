@@ -873,8 +873,8 @@ hipError_t enqueue_rows(const DecodeShape &s, const DecodeArgs &a, const LayerAr
     char *rest = static_cast<char *>(b.ws) + r256((size_t)n * kmax * 2) + r256((size_t)n * 4);
     hipError_t r = A ? launch_gemm_prep_a(A, n, K, a16, ea, st) : hipSuccess;
     if (r != hipSuccess) return r;
-    // A set of Q4_K matrices with enough rows or tiles for the half-block
-    // kernel (long prompts, or a gate|up set from about 900 rows at 4B
+    // A set of Q4_K matrices with enough rows or tiles for the half-block or
+    // ping-pong kernel (long prompts, or a gate|up set from about 900 rows at 4B
     // widths): one matrix-core launch for the set (its tiles fill the CUs in
     // whole rounds), row exponents of each matrix at the start of its region
     bool all_q4k = true;

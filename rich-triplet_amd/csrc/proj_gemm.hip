@@ -301,8 +301,9 @@ __global__ __launch_bounds__(512) void k_gemm_f16_t128(const _Float16 *__restric
 //   distinct bank groups.
 //   4608 x 12288 x 3072 333 us (1.04 PFLOP/s; the four-wave form with 64-wide
 //   stages and 128 x 128 wave tiles 400), 4096 x 4096 x 2560 82 us, 2000 x 12000
-//   x 3072 159 us.  With zero operands 250 us: the rest is the card's power
-//   limit.  Storing C takes 45 us of the 333.
+//   x 3072 159 us.  With zero operands 250 us: the clock is 1.77 GHz under real
+//   ones; and the matrix cores are busy 53% of the cycles, where a library f16
+//   product keeps them 66% busy (265 us).  Storing C takes 45 us of the 333.
 // ---------------------------------------------------------------------------
 constexpr int kT256Slot = 256 * 64;  // one operand, one stage
 

@@ -15,7 +15,7 @@ namespace rt {
 constexpr int kBK = 64;  // K per pipeline stage = one Q4_K chunk (32 qs bytes, 2 sub-blocks)
 
 // ---------------------------------------------------------------------------
-// Matrix-core kernels.  Both use v_mfma_f32_32x32x16_f16 (lane l: A row / B
+// Matrix-core kernels.  All use v_mfma_f32_32x32x16_f16 (lane l: A row / B
 // column l%32, k group g = l/32, 8 halves each) and the same K order inside a
 // 64-wide chunk (A and B agree on it, so the sum is unchanged):
 //   lane group g holds qs bytes [16g, 16g+16) of the chunk's 32; k-step t
@@ -24,9 +24,10 @@ constexpr int kBK = 64;  // K per pipeline stage = one Q4_K chunk (32 qs bytes, 
 //   bytes (sub-block 2c+1).
 // A (and in the eight-wave kernel the packed W bytes) reaches LDS by
 // global_load_lds_dwordx4 (no VGPRs, no ds_write); each ring slot is its own
-// __shared__ variable.  Every lane dequantises the qs bytes of its own column
-// straight into the MFMA B operand, so no dequantised weight is written back
-// to LDS.
+// __shared__ variable.  In the eight-wave and half-block kernels every lane
+// dequantises the qs bytes of its own column straight into the MFMA B operand,
+// so no dequantised weight is written back to LDS; the ping-pong kernel
+// (q4k_gemm_pp.hip) writes it there once for all the waves of a workgroup.
 // ---------------------------------------------------------------------------
 // Eight f16 weights of one k-step from two qs words (low or high nibbles).
 // v_perm builds halves 1024+q (low nibbles) or 1024+16q (high nibbles), and
@@ -156,80 +157,80 @@ RT_DEV void store_qkv_tile(const floatx16 (&acc)[4][2], float *stage, float (*ws
                            int row0, int n0, int mi, const int *ea, const int (&ecol)[2], const QkRope &qr) {
   const int lane = (int)(threadIdx.x & 63), g = lane >> 5, l32 = lane & 31;
   const int colp[2] = {n0 + 32 * w, n0 + 128 + 32 * w};
-      const int cl = 32 * w + l32;  // the pair's column within the head
-      const float *gam = mi == 0 ? qr.g_q : qr.g_k;
-      const float g0 = mi < 2 ? 1.0f + gam[cl] : 0.f, g1 = mi < 2 ? 1.0f + gam[cl + 128] : 0.f;
-  #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        __builtin_amdgcn_sched_barrier(0);
-        floatx16 v0, v1;
-  #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int er = ea[min(row0 + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), M - 1)];
-          v0[r] = __builtin_amdgcn_ldexpf(acc[i][0][r], er + ecol[0]);
-          v1[r] = __builtin_amdgcn_ldexpf(acc[i][1][r], er + ecol[1]);
-        }
-        if (mi < 2) {  // workgroup-uniform
-          // sums of squares of the 32 rows: this wave's 64 columns through its
-          // LDS slot ([row][l32], 16-byte groups swizzled by the row), two
-          // lanes per row, then the four waves' sums through wsum
-  #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int R = 8 * (r >> 2) + 4 * g + (r & 3);
-            stage[R * 32 + ((((l32 >> 2) ^ R) & 7) << 2) + (l32 & 3)] = v0[r] * v0[r] + v1[r] * v1[r];
-          }
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          {
-            const int R = lane >> 1;
-            float t = 0.f;
-  #pragma unroll
-            for (int m4 = 4 * (lane & 1); m4 < 4 * (lane & 1) + 4; ++m4) {
-              const float4 x = *reinterpret_cast<const float4 *>(stage + R * 32 + (((m4 ^ R) & 7) << 2));
-              t += (x.x + x.y) + (x.z + x.w);
-            }
-            t += __shfl_xor(t, 1);
-            if ((lane & 1) == 0) wsum[w][32 * i + R] = t;
-          }
-          wg_barrier();
-  #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-  #pragma clang fp contract(off)
-            const int R = 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
-            const float ss = (wsum[0][R] + wsum[1][R]) + (wsum[2][R] + wsum[3][R]);
-            const float rinv = rms_inv_from_sumsq(ss, 1.0f / 256.0f, qr.eps);
-            const int co = min(row0 + R, M - 1) * qr.cs_stride + cl;  // 32-bit offset from the uniform base
-            const float cv = qr.cs[co], sv = qr.cs[co + 128];
-            const float a0 = (v0[r] * rinv) * g0, a1 = (v1[r] * rinv) * g1;
-            v0[r] = a0 * cv - a1 * sv;
-            v1[r] = a0 * sv + a1 * cv;
-          }
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-        // stage and store the tile's 32 rows x (32 + 32) columns
-        constexpr int P = 72;
-  #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + l32] = v0[r];
-          stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + 32 + l32] = v1[r];
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int rl = q * 4 + lane / 16, f = lane % 16;
-          const int row = row0 + 32 * i + rl, cc = colp[f >> 3] + 4 * (f & 7);
-          const float4 x = *reinterpret_cast<const float4 *>(stage + rl * P + 4 * f);
-          if (row < M) *reinterpret_cast<float4 *>(c + (size_t)row * N + cc) = x;
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int cl = 32 * w + l32;  // the pair's column within the head
+  const float *gam = mi == 0 ? qr.g_q : qr.g_k;
+  const float g0 = mi < 2 ? 1.0f + gam[cl] : 0.f, g1 = mi < 2 ? 1.0f + gam[cl + 128] : 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    __builtin_amdgcn_sched_barrier(0);
+    floatx16 v0, v1;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int er = ea[min(row0 + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), M - 1)];
+      v0[r] = __builtin_amdgcn_ldexpf(acc[i][0][r], er + ecol[0]);
+      v1[r] = __builtin_amdgcn_ldexpf(acc[i][1][r], er + ecol[1]);
+    }
+    if (mi < 2) {  // workgroup-uniform
+      // sums of squares of the 32 rows: this wave's 64 columns through its
+      // LDS slot ([row][l32], 16-byte groups swizzled by the row), two
+      // lanes per row, then the four waves' sums through wsum
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int R = 8 * (r >> 2) + 4 * g + (r & 3);
+        stage[R * 32 + ((((l32 >> 2) ^ R) & 7) << 2) + (l32 & 3)] = v0[r] * v0[r] + v1[r] * v1[r];
       }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      {
+        const int R = lane >> 1;
+        float t = 0.f;
+#pragma unroll
+        for (int m4 = 4 * (lane & 1); m4 < 4 * (lane & 1) + 4; ++m4) {
+          const float4 x = *reinterpret_cast<const float4 *>(stage + R * 32 + (((m4 ^ R) & 7) << 2));
+          t += (x.x + x.y) + (x.z + x.w);
+        }
+        t += __shfl_xor(t, 1);
+        if ((lane & 1) == 0) wsum[w][32 * i + R] = t;
+      }
+      wg_barrier();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+#pragma clang fp contract(off)
+        const int R = 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
+        const float ss = (wsum[0][R] + wsum[1][R]) + (wsum[2][R] + wsum[3][R]);
+        const float rinv = rms_inv_from_sumsq(ss, 1.0f / 256.0f, qr.eps);
+        const int co = min(row0 + R, M - 1) * qr.cs_stride + cl;  // 32-bit offset from the uniform base
+        const float cv = qr.cs[co], sv = qr.cs[co + 128];
+        const float a0 = (v0[r] * rinv) * g0, a1 = (v1[r] * rinv) * g1;
+        v0[r] = a0 * cv - a1 * sv;
+        v1[r] = a0 * sv + a1 * cv;
+      }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // stage and store the tile's 32 rows x (32 + 32) columns
+    constexpr int P = 72;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + l32] = v0[r];
+      stage[(8 * (r >> 2) + 4 * g + (r & 3)) * P + 32 + l32] = v1[r];
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int rl = q * 4 + lane / 16, f = lane % 16;
+      const int row = row0 + 32 * i + rl, cc = colp[f >> 3] + 4 * (f & 7);
+      const float4 x = *reinterpret_cast<const float4 *>(stage + rl * P + 4 * f);
+      if (row < M) *reinterpret_cast<float4 *>(c + (size_t)row * N + cc) = x;
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
 }
 
 // The 256 x 256-tile ping-pong kernel (q4k_gemm_pp.hip) on prepared operands:

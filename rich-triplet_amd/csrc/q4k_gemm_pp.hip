@@ -20,8 +20,10 @@
 //   Measured (us, the product alone; C stores nontemporal, which gives 4-7%):
 //   4608 x 12288 x 3072 351 (0.99 PFLOP/s; k_q4k_gemm_h 385), 4096 x 20480 x 2560
 //   396 (1.08; 465), 4096 x 2560 x 10240 214 (1.00; 256 split three ways), 1000
-//   x 10240 x 2560 61 (0.86; 100).  On zeros it runs a quarter faster: the
-//   card's power limit, then the stores of C (45 us of the first), set it.
+//   x 10240 x 2560 61 (0.86; 100).  Bound by the schedule, then by power: at the
+//   first shape the matrix cores are busy 53% of 624,000 cycles (a library f16
+//   product: 66% of 509,000), and the clock is 1.72 GHz, where zero operands
+//   take as many cycles at 2.13 (285 us).  Storing C takes 45 us.
 //   A slot row is 64 B (4 segments of 8 halves), logical segment s at
 //   s ^ ((row >> 2) & 3): the 16 lanes of a ds_read_b128 hit 16 distinct bank
 //   groups.
