@@ -525,6 +525,8 @@ struct AnyPrologue {
   }
 };
 
+// The fused launches keep the digits in every chunk (32 bits of its largest
+// normalised value, where the one-row pass before them kept 16).
 template <int FMT>
 RT_DEV void any_stage_pro(uint32_t *dl, const float4 (&xn)[2], int K, int T) {
   const int nf = K / 4, nst = 16 * ((K + 63) / 64);
