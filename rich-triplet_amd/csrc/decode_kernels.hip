@@ -1210,7 +1210,9 @@ hipError_t prepare_lm_head_batch(int hidden) {
   if (hidden == 2560) return hipFuncSetAttribute((const void *)k_lmhead_batch<2560>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (hidden == 512) return hipSuccess;
-  return hipFuncSetAttribute((const void *)k_lmhead_batch<0>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  // the widest hidden's: a context of a smaller one takes nothing from another
+  return hipFuncSetAttribute((const void *)k_lmhead_batch<0>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             kLmHeadMaxHidden * 32);
 }
 
 hipError_t enqueue_lm_head_batch(const DecodeShape &s, const DecodeArgs &a, const float *xn, float *logits_b, int m,

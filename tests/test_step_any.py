@@ -45,3 +45,22 @@ def test_step_any_matches_oracle(rt, orc, hidden, ffn, heads, kv, plan):
     d.set_graph(False)
     assert np.array_equal(d.decode_step(19, pos), got)
     d.close()
+
+
+def test_verify_of_two_widths_at_once(rt, orc):
+    """A context of hidden 3840, whose batched head stages 120 KB, verifies after
+    one of hidden 768 was created: each gives its own steps' logits."""
+    from test_oracle import make_model
+    made = []
+    for hidden, heads in ((3840, (16, 256)), (768, (4, 128))):
+        cfg = dict(hidden=hidden, ffn=1536, n_q_heads=heads[0], n_kv_heads=4, head_dim=heads[1], n_layers=1, vocab=777,
+                   sliding_window=9, global_every=2, rope_theta_local=10000.0, rope_theta_global=1000000.0,
+                   rope_fs_local=1.0, rope_fs_global=0.125, eps=1e-6, attn_scale=1.0 / np.sqrt(heads[1]))
+        layers, embed, fnorm = make_model(orc, cfg, max_seq=24, ctx=5, seed=hidden)
+        made.append((cfg, layers, embed, fnorm, mixed_ctx(rt, cfg, layers, [[1] * 7], embed, fnorm, 5, 24, layers)))
+    for cfg, layers, embed, fnorm, d in made:
+        got = d.decode_step_batch([3, 4, 5], 5)
+        for i, t in enumerate((3, 4, 5)):
+            ref = orc.gemma3_decode_step(cfg, layers, embed, fnorm, token=t, pos=5 + i)
+            assert rel_l2(got[i], ref) < 1e-3
+        d.close()
